@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -53,6 +54,26 @@ const JumpTable& host_jump_table() {
 namespace {
 std::mutex g_dev_mu;
 std::vector<std::unique_ptr<DeviceContext>> g_devices;
+
+// The jump matrices of byte positions [first, end), kPositionInts each:
+// A^(d 2^(kJumpBits k)), d = 0..kJumpValues; A^(2^j) past the last
+// jump_matrix.txt entry by squaring.  False when an entry is out of bounds.
+bool build_digits(int first, int end, int32_t* out) {
+  const JumpTable& jt = host_jump_table();
+  for (int k = first; k < end; ++k) {
+    const int j = kJumpBits * k;
+    std::vector<uint32_t> m(jt.at(std::min(j, kNumJump - 1)), jt.at(std::min(j, kNumJump - 1)) + 64);
+    for (int q = kNumJump - 1; q < j; ++q) m = mat_mul(m.data(), m.data());
+    std::vector<uint32_t> p(64, 0);
+    for (int r = 0; r < 8; ++r) p[(size_t)r * 9] = 1;  // the identity: a digit 0 leaves the state as it is
+    for (int d = 0; d <= kJumpValues; ++d) {
+      if (d > 0) p = d > 1 ? mat_mul(p.data(), m.data()) : m;
+      if (!jump_matrix_entries(p.data(), out + (size_t)(k - first) * kPositionInts + (size_t)d * kJumpMatrixInts))
+        return false;
+    }
+  }
+  return true;
+}
 }  // namespace
 
 int device_context(int device, DeviceContext** out) {
@@ -104,6 +125,13 @@ int device_context(int device, DeviceContext** out) {
     jump[(size_t)kIdentityRec + r] = make_record(row);
   }
 
+  // the same matrices as the bulk advance reads them
+  std::vector<int32_t> digits((size_t)kJumpPositions * kPositionInts);
+  if (!build_digits(0, kJumpPositions, digits.data())) {
+    (void)hipSetDevice(prev);
+    return fail(MRG8_ERR_STATE, "a jump matrix exceeds the device arithmetic's bound");
+  }
+
   // Matrix-core fill tables (operand digits, combine constants, column
   // start records); a fan-out row with a zero entry would need the exact-zero
   // test, so such a table turns the matrix-core fill off.
@@ -132,20 +160,25 @@ int device_context(int device, DeviceContext** out) {
   for (int i = 0; i < 2; ++i)
     mfma_bytes += sizeof(CoefRecord) * mt[i].fan.size() + sizeof(uint32_t) * (mn[i].a.size() + mn[i].k.size());
   if (!mfma_ok) mfma_bytes = 0;
-  const size_t bytes = rec_bytes + mfma_bytes;
+  const size_t digit_bytes = sizeof(int32_t) * digits.size();
+  const size_t bytes = digit_bytes + rec_bytes + mfma_bytes;
   if ((e = hipMalloc(&p, bytes)) != hipSuccess) {
     (void)hipSetDevice(prev);
     return hip_fail(e, "hipMalloc(tables)");
   }
-  ctx->tables.lane = static_cast<CoefRecord*>(p);
+  // the jump matrices first: their 256-byte blocks stay on line boundaries
+  ctx->tables.digits = static_cast<const int32_t*>(p);
+  ctx->tables.lane = reinterpret_cast<CoefRecord*>(static_cast<uint8_t*>(p) + digit_bytes);
   ctx->tables.jump = ctx->tables.lane + lane.size();
-  e = hipMemcpy(ctx->tables.lane, lane.data(), sizeof(CoefRecord) * lane.size(), hipMemcpyHostToDevice);
+  e = hipMemcpy(p, digits.data(), digit_bytes, hipMemcpyHostToDevice);
+  if (e == hipSuccess)
+    e = hipMemcpy(ctx->tables.lane, lane.data(), sizeof(CoefRecord) * lane.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(ctx->tables.jump, jump.data(), sizeof(CoefRecord) * jump.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess && mfma_ok) {
     // records first (16-byte aligned after the 48-byte records), then the
     // operand digits, the accumulator start values and the step tables
-    uint8_t* m = static_cast<uint8_t*>(p) + rec_bytes;
+    uint8_t* m = static_cast<uint8_t*>(p) + digit_bytes + rec_bytes;
     auto put = [&](const void* src, size_t n) {
       uint8_t* at = m;
       if (e == hipSuccess) e = hipMemcpy(at, src, n, hipMemcpyHostToDevice);
@@ -189,26 +222,13 @@ DeviceContext* existing_device_context(int device) {
 
 int ensure_wide_table(DeviceContext& ctx) {
   std::lock_guard<std::mutex> lk(ctx.wide_mu);
-  if (ctx.tables.wide) return MRG8_OK;
-  // A^(d 2^(kJumpBits k)) for k = kJumpPositions..kWidePositions-1 and
-  // d = 1..kJumpValues; A^(2^j) past the last jump_matrix.txt entry by squaring.
-  const JumpTable& jt = host_jump_table();
-  const int npos = kWidePositions - kJumpPositions;
-  std::vector<CoefRecord> wide((size_t)npos * kJumpValues * 8);
-  for (int k = kJumpPositions; k < kWidePositions; ++k) {
-    const int j = kJumpBits * k;
-    std::vector<uint32_t> m(jt.at(std::min(j, kNumJump - 1)), jt.at(std::min(j, kNumJump - 1)) + 64);
-    for (int q = kNumJump - 1; q < j; ++q) m = mat_mul(m.data(), m.data());
-    std::vector<uint32_t> p = m;
-    for (int d = 1; d <= kJumpValues; ++d) {
-      if (d > 1) p = mat_mul(p.data(), m.data());
-      for (int r = 0; r < 8; ++r)
-        wide[((size_t)(k - kJumpPositions) * kJumpValues + (d - 1)) * 8 + r] = make_record(&p[(size_t)r * 8]);
-    }
-  }
+  if (ctx.tables.digits_wide) return MRG8_OK;
+  std::vector<int32_t> wide((size_t)(kWidePositions - kJumpPositions) * kPositionInts);
+  if (!build_digits(kJumpPositions, kWidePositions, wide.data()))
+    return fail(MRG8_ERR_STATE, "a jump matrix exceeds the device arithmetic's bound");
   DeviceGuard dg(ctx.device);
   void* dev = nullptr;
-  const size_t bytes = sizeof(CoefRecord) * wide.size();
+  const size_t bytes = sizeof(int32_t) * wide.size();
   hipError_t e = hipMalloc(&dev, bytes);
   if (e != hipSuccess) return hip_fail(e, "hipMalloc(wide jump table)");
   e = hipMemcpy(dev, wide.data(), bytes, hipMemcpyHostToDevice);
@@ -216,7 +236,7 @@ int ensure_wide_table(DeviceContext& ctx) {
     (void)hipFree(dev);
     return hip_fail(e, "hipMemcpy(wide jump table)");
   }
-  ctx.tables.wide = static_cast<CoefRecord*>(dev);
+  ctx.tables.digits_wide = static_cast<const int32_t*>(dev);
   return MRG8_OK;
 }
 
@@ -792,6 +812,30 @@ extern "C" int mrg8_rand1(mrg8_gen_t g, double* value) {
 
 // ---- bulk advance of device-resident states ----------------------------------------
 
+// States per group of four lanes of a bulk advance of n states (0: matrices
+// from memory).  Per byte position, measured on MI355X (256 CUs): from memory
+// 1.32 us per 2^17 states once the card is full (k_advance, in proportion to
+// n); through LDS one round of blocks, 256 G states a CU, takes 0.94 us with
+// G = 2, 1.59 us with 4 and 2.84 us with 8, however full it is.  The least of
+// the four times rounds is taken.  2^20 states with 256-bit offsets: 286 us
+// from memory, 245, 211 and 197 us through LDS; 2^16: 23.5 us from memory,
+// 31 us with G = 2.  (2^20 states with 200-bit offsets: 164 us, 427 us with
+// 48-byte coefficient records read from memory.)
+static int advance_states_per_group(const DeviceContext& ctx, uint64_t n) {
+  const double cu = ctx.num_cu;
+  double best = 1.32 * (double)n / (512.0 * cu);
+  int group = 0;
+  const struct { int g; double us; } lds[] = {{2, 0.94}, {4, 1.59}, {8, 2.84}};
+  for (const auto& l : lds) {
+    const double t = l.us * std::ceil((double)n / (256.0 * l.g * cu));
+    if (t < best) {
+      best = t;
+      group = l.g;
+    }
+  }
+  return group;
+}
+
 extern "C" int mrg8_advance_states(int device, const uint32_t* d_in, const uint64_t* d_offsets, uint32_t words,
                                    uint32_t* d_out, uint64_t n, void* stream) {
   clear_error();
@@ -816,9 +860,9 @@ extern "C" int mrg8_advance_states(int device, const uint32_t* d_in, const uint6
     a.out = d_out + 8 * first;
     a.n = std::min(chunk, n - first);
     a.words = words;
-    a.jump = ctx->tables.jump;
-    a.wide = ctx->tables.wide;
-    hipError_t e = launch_advance(a, static_cast<hipStream_t>(stream));
+    a.digits = ctx->tables.digits;
+    a.digits_wide = ctx->tables.digits_wide;
+    hipError_t e = launch_advance(a, advance_states_per_group(*ctx, a.n), static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "advance launch");
   }
   return MRG8_OK;

@@ -697,91 +697,300 @@ __global__ __launch_bounds__(1024) void k_batch_queue(BatchArgs a) {
 
 // ---- bulk advance: many states, offsets of up to kAdvanceWords words --------
 
-__device__ __forceinline__ const CoefRecord* wide_rec(const AdvanceArgs& a, int k, uint32_t d, int row) {
-  if (d == 0u) return a.jump + (kIdentityRec + row);
-  return k < kJumpPositions ? a.jump + ((k * kJumpValues + (int)d - 1) * 8 + row)
-                            : a.wide + (((k - kJumpPositions) * kJumpValues + (int)d - 1) * 8 + row);
+// The value of v in the lanes l ^ 0 .. l ^ 7 of this lane's group of eight.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
 }
 
-// Eight lanes per state (lane r of a group computes row r, as in the jumps
-// above); byte positions of the offset in order, each digit extracted once,
-// positions where no state of the wave has a digit skipped, the next
-// position's records fetched while the current step computes.  Waves whose
-// states have no zero word skip the zero-product test and keep the words
-// centred between steps (2^20 states, 200-bit offsets: 400 us against 446 us
-// for the plain loop).  A state is read before it is written, so `in` and
-// `out` may be the same buffer.
-// jump_step for states with no zero word, on centred words e = s - 2^30:
-// each lane centres its one new word before the gather instead of every lane
-// centring eight after it.
-__device__ __forceinline__ void jump_step_centred(int32_t e[8], const Coef& c) {
-  const uint32_t ey = dot_residue(c, e) + 1u - kCenter;
+__device__ __forceinline__ void gather_xor(uint32_t v, uint32_t w[8]) {
+  constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kXor3 = 0x1B;  // quad_perm [1,0,3,2], [2,3,0,1], [3,2,1,0]
+  const uint32_t m = dpp<0x141>(v);                        // row_half_mirror: lane ^ 7
+  w[0] = v;
+  w[1] = dpp<kXor1>(v);
+  w[2] = dpp<kXor2>(v);
+  w[3] = dpp<kXor3>(v);
+  w[4] = dpp<kXor3>(m);
+  w[5] = dpp<kXor2>(m);
+  w[6] = dpp<kXor1>(m);
+  w[7] = m;
+}
+
+// This lane's row of a jump matrix (entries in the order of gather_xor).
+struct JumpRow {
+  int32_t c[8];
+};
+
+__device__ __forceinline__ JumpRow load_row(const int32_t* p) {  // p: the matrix + 4 * row
+  const u4_t a = *reinterpret_cast<const u4_t*>(p), b = *reinterpret_cast<const u4_t*>(p + 32);
+  return JumpRow{{(int32_t)a.x, (int32_t)a.y, (int32_t)a.z, (int32_t)a.w, (int32_t)b.x, (int32_t)b.y, (int32_t)b.z,
+                  (int32_t)b.w}};
+}
+
+// The next centred word from a row's sum (see jump_matrix_entries).
+__device__ __forceinline__ int32_t reduce_centred(uint64_t v) {
+  const uint64_t f = fold_hi((uint32_t)(v >> 32), (uint32_t)v);
+  return (int32_t)(((uint32_t)f & kP) + (uint32_t)(f >> 31) - kCenter);
+}
+
+// One product: this lane's centred word of (matrix) x (state), the state's
+// words being the centred e of the group's lanes.
+__device__ __forceinline__ int32_t jump_row(const JumpRow& m, int32_t e) {
   uint32_t w[8];
-  gather_group(ey, w);
+  gather_xor((uint32_t)e, w);
+  uint64_t v = kJumpBase;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) e[j] = (int32_t)w[j];
+  for (int k = 0; k < 8; ++k) v += (uint64_t)((int64_t)m.c[k] * (int64_t)(int32_t)w[k]);
+  return reduce_centred(v);
 }
 
-template <bool ZERO_WORDS>
-__device__ __forceinline__ void advance_digits(uint32_t s[8], const uint64_t (&off)[kAdvanceWords],
-                                               const AdvanceArgs& a, int row) {
-  const int npos = 8 * (int)a.words;
-  int32_t e[8];
-  if (!ZERO_WORDS) centre(s, e);
-  uint32_t d = (uint32_t)off[0] & (uint32_t)kJumpValues;
-  Coef c = load_coef11(wide_rec(a, 0, d, row));
+__device__ __forceinline__ int32_t centre_word(uint32_t s) { return (int32_t)(s >= kCenter ? s - kP : s); }
+__device__ __forceinline__ uint32_t word_of(int32_t e) { return (uint32_t)(e > 0 ? e : e + (int32_t)kP); }  // in [1, p]
+
+__device__ __forceinline__ const int32_t* position_table(const AdvanceArgs& a, int k) {
+  return k < kJumpPositions ? a.digits + k * kPositionInts : a.digits_wide + (k - kJumpPositions) * kPositionInts;
+}
+
+__device__ __forceinline__ uint32_t digit_of(uint32_t half, int k) { return (half >> (8 * (k & 3))) & 0xffu; }
+
+// The jump of a state that has a zero word (this lane's word s): bigDotProd
+// is 0 exactly where every product of a row is.  A state without one never
+// gets one (no row of a power of A is zero), so only waves that start with
+// such a state come here.
+__device__ __forceinline__ uint32_t advance_zero_words(uint32_t s, const uint32_t* off, const AdvanceArgs& a) {
+  const int row = threadIdx.x & 7;
+  for (int k = 0; k < 8 * (int)a.words; ++k) {
+    const uint32_t d = digit_of(off[k / 4], k);
+    if (!__ballot(d != 0u)) continue;
+    const JumpRow m = load_row(position_table(a, k) + d * kJumpMatrixInts + 4 * row);
+    uint32_t w[8];
+    gather_xor(s, w);
+    bool any = false;
 #pragma unroll
-  for (int w = 0; w < kAdvanceWords; ++w) {
-    if (w >= (int)a.words) break;
-    for (int b = 0; b < 8; ++b) {
-      const int k = 8 * w + b;
-      uint32_t dn;
-      if (b < 7)
-        dn = (uint32_t)(off[w] >> (8 * (b + 1))) & (uint32_t)kJumpValues;
-      else
-        dn = w + 1 < kAdvanceWords ? (uint32_t)off[w + 1 < kAdvanceWords ? w + 1 : w] & (uint32_t)kJumpValues : 0u;
-      const bool last = k + 1 == npos;
-      if (last) dn = 0u;
-      const Coef next = load_coef11(wide_rec(a, last ? 0 : k + 1, dn, row));
-      if (__ballot(d != 0u)) {
-        if (ZERO_WORDS)
-          jump_step<true>(s, c);
-        else
-          jump_step_centred(e, c);
-      }
-      c = next;
-      d = dn;
-    }
+    for (int q = 0; q < 8; ++q) any = any || (m.c[q] != 0 && w[q] != 0u);
+    const uint32_t y = word_of(jump_row(m, centre_word(s)));
+    s = any ? y : 0u;
   }
-  if (!ZERO_WORDS) {
+  return s;
+}
+
+// Eight lanes per state, lane r holding word r and computing row r of each
+// product; the byte positions of the offset in order, the rows of four
+// positions fetched while the four before them are computed (20011 states,
+// 64-bit offsets: 3.8 us a launch, one position ahead 4.3 us; 1000 states,
+// 256 bits: 5.5 and 8.1 us).  Positions where
+// no state of the wave has a digit are skipped.  A state is read before it is
+// written, so `in` and `out` may be the same buffer.
+__device__ __forceinline__ void load_rows4(JumpRow m[4], const AdvanceArgs& a, int half, uint32_t d, int row) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s[j] = (uint32_t)e[j] + kCenter;
-  }
+  for (int b = 0; b < 4; ++b)
+    m[b] = load_row(position_table(a, 4 * half + b) + digit_of(d, b) * kJumpMatrixInts + 4 * row);
+}
+
+__device__ __forceinline__ int32_t apply_rows4(const JumpRow m[4], uint32_t d, int32_t e) {
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+    if (__ballot(digit_of(d, b) != 0u)) e = jump_row(m[b], e);
+  return e;
 }
 
 __global__ __launch_bounds__(256) void k_advance(AdvanceArgs a) {
   const int row = threadIdx.x & 7;
   const uint64_t item = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3;
   const bool live = item < a.n;
-  uint32_t s[8];
-  uint64_t off[kAdvanceWords];
-#pragma unroll
-  for (int w = 0; w < kAdvanceWords; ++w) off[w] = live && w < (int)a.words ? a.offsets[item * a.words + w] : 0;
-  uint32_t smin = 1u;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    s[j] = live ? a.in[8 * item + j] : 1u;
-    smin = min(smin, s[j]);
+  const uint32_t* off = reinterpret_cast<const uint32_t*>(a.offsets) + (live ? item : 0) * 2 * a.words;
+  const uint32_t s = live ? a.in[8 * item + row] : 1u;
+  uint32_t out;
+  if (__ballot(s == 0u)) {
+    out = advance_zero_words(s, off, a);
+  } else {
+    int32_t e = centre_word(s);
+    JumpRow m0[4], m1[4];
+    uint32_t d0 = off[0], d1 = off[1];
+    load_rows4(m0, a, 0, d0, row);
+    for (uint32_t w = 0; w < a.words; ++w) {
+      load_rows4(m1, a, 2 * w + 1, d1, row);
+      e = apply_rows4(m0, d0, e);
+      const uint32_t da = d1;
+      if (w + 1 < a.words) {
+        d0 = off[2 * w + 2];
+        d1 = off[2 * w + 3];
+        load_rows4(m0, a, 2 * w + 2, d0, row);
+      }
+      e = apply_rows4(m1, da, e);
+    }
+    out = word_of(e);
   }
-  // a state with no zero word never gets one (no row of a power of A is
-  // zero), so the zero-product test is needed only by waves that start with one
-  if (__ballot(smin == 0u))
-    advance_digits<true>(s, off, a, row);
-  else
-    advance_digits<false>(s, off, a, row);
-  if (live && row == 0) {
+  if (live) a.out[8 * item + row] = out;
+}
+
+// The same jumps with each position's 256 matrices (64 KB) staged in LDS by
+// the block: 256 x G states, G per group of four lanes, take one position
+// together while the next one's matrices are copied to the other buffer
+// (global-to-LDS loads, no registers; two arrays, so that reads of one wait
+// for no copy into the other).  From memory, each state and digit costs 256
+// bytes of L2 and L1 traffic, which bounds k_advance at large n; here that is
+// 64 KB per block and position, and the step is bound by its 18 64-bit
+// multiply-adds and 16 other VALU operations per two rows.
+// Lane r of a group holds words r and r + 4 and computes both rows, so it
+// reaches the other six words with six quad permutations for two rows (seven
+// for one with eight lanes per state).  Odd groups keep the two words in the
+// other order, so that neighbouring groups read different halves of a matrix
+// (all four 64-byte quarters in turn would remove the LDS bank conflicts
+// left, at four more operations a step: measured the same).
+// 2^20 states, 200-bit offsets: see advance_states_per_group.
+constexpr int kAdvanceGroups = 256;  // groups of four lanes in a block
+
+struct JumpPair {  // rows of a lane's first and second word: entries for the words held alike, and for the other ones
+  u4_t near0, far0, near1, far1;
+};
+
+__device__ __forceinline__ void mad4(uint64_t& v, const u4_t& c, const uint32_t w[4]) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) a.out[8 * item + j] = s[j];
+  for (int k = 0; k < 4; ++k) v += (uint64_t)((int64_t)(int32_t)c[k] * (int64_t)(int32_t)w[k]);
+}
+
+__device__ __forceinline__ void gather_quad(uint32_t v, uint32_t w[4]) {
+  w[0] = v;
+  w[1] = dpp<0xB1>(v);
+  w[2] = dpp<0x4E>(v);
+  w[3] = dpp<0x1B>(v);
+}
+
+template <int G>
+__global__ __launch_bounds__(4 * kAdvanceGroups) void k_advance_lds(AdvanceArgs a) {
+  constexpr int kThreads = 4 * kAdvanceGroups, kStates = kAdvanceGroups * G;
+  constexpr int kNoLoads = 0x0f70;  // s_waitcnt vmcnt(0)
+  __shared__ __attribute__((aligned(1024))) int32_t table0[kPositionInts], table1[kPositionInts];
+  __shared__ uint32_t used;
+  const uint32_t tid = threadIdx.x, grp = tid >> 2, r = tid & 3, odd = grp & 1;
+  const uint32_t word0 = r + 4 * odd, word1 = r + 4 * (odd ^ 1);
+  const uint64_t first = (uint64_t)blockIdx.x * kStates;
+  const uint32_t count = (uint32_t)min((uint64_t)kStates, a.n - first);
+  const uint32_t halves = 2 * a.words;  // an offset as 32-bit halves
+  const uint32_t* const in = a.in + 8 * first;
+  uint32_t* const out = a.out + 8 * first;
+  const uint32_t* const offs = reinterpret_cast<const uint32_t*>(a.offsets) + first * halves;
+  auto state = [&](int g) { return min(grp + kAdvanceGroups * g, count - 1); };  // past the end: the last one again
+  // copies position k's matrices to LDS, 8 KiB per wave
+  auto stage = [&](int k, int32_t* table) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int kInts = kPositionInts / (kThreads / 64);
+    const int32_t* src = position_table(a, k) + wave * kInts + 4 * (tid & 63);
+#pragma unroll
+    for (int i = 0; i < kInts / 256; ++i)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + 256 * i),
+                                       (__attribute__((address_space(3))) void*)&table[wave * kInts + 256 * i], 16, 0, 0);
+  };
+  if (tid == 0) used = 0u;
+  uint32_t zero = 0;  // bit g: this group's state g has a zero word
+  int32_t e0[G], e1[G];
+  {
+    uint32_t s0[G], s1[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      s0[g] = in[8 * state(g) + word0];
+      s1[g] = in[8 * state(g) + word1];
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      zero |= s0[g] == 0u || s1[g] == 0u ? 1u << g : 0u;
+      e0[g] = centre_word(s0[g]);
+      e1[g] = centre_word(s1[g]);
+    }
+    zero |= dpp<0xB1>(zero);
+    zero |= dpp<0x4E>(zero);
+  }
+  // byte positions at which some offset of the block has a digit
+  uint32_t mine = 0;
+  for (uint32_t i = tid; i < count * halves; i += kThreads) {
+    const uint32_t h = offs[i], q = i % halves;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) mine |= digit_of(h, b) ? 1u << (4 * q + b) : 0u;
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) mine |= __shfl_xor(mine, d);
+  __syncthreads();
+  if ((tid & 63) == 0) atomicOr(&used, mine);
+  __syncthreads();
+  uint32_t todo = __builtin_amdgcn_readfirstlane(used);
+  uint64_t base = kJumpBase;
+  asm("" : "+v"(base));  // in vector registers: the first multiply-add's addend
+  uint32_t half[G];
+  auto fetch_half = [&](int q) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) half[g] = offs[state(g) * halves + (uint32_t)q];
+  };
+  // takes position k from `table` while position `next` is copied to `other`
+  auto position = [&](int k, int next, const int32_t* table, int32_t* other) {
+    if (next >= 0) stage(next, other);
+    const uint32_t m0 = 16 * word0, m1 = 16 * word1;
+    const uint32_t sel = 0x03020000u + ((4u + (uint32_t)(k & 3)) << 8);  // the digit goes into bits 8..15
+    auto rows = [&](uint32_t digits) {
+      const uint8_t* t = reinterpret_cast<const uint8_t*>(table);
+      const uint8_t* p0 = t + __builtin_amdgcn_perm(digits, m0, sel);
+      const uint8_t* p1 = t + __builtin_amdgcn_perm(digits, m1, sel);
+      return JumpPair{*reinterpret_cast<const u4_t*>(p0), *reinterpret_cast<const u4_t*>(p0 + 128),
+                      *reinterpret_cast<const u4_t*>(p1), *reinterpret_cast<const u4_t*>(p1 + 128)};
+    };
+    JumpPair cur = rows(half[0]);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      JumpPair ahead{};
+      if (g + 1 < G) ahead = rows(half[g + 1]);
+      uint32_t w0[4], w1[4];
+      gather_quad((uint32_t)e0[g], w0);
+      gather_quad((uint32_t)e1[g], w1);
+      uint64_t v0 = base, v1 = base;
+      mad4(v0, cur.near0, w0);
+      mad4(v1, cur.near1, w1);
+      mad4(v0, cur.far0, w1);
+      mad4(v1, cur.far1, w0);
+      e0[g] = reduce_centred(v0);
+      e1[g] = reduce_centred(v1);
+      cur = ahead;
+    }
+    if (next >= 0 && next / 4 != k / 4) fetch_half(next / 4);
+    __builtin_amdgcn_s_waitcnt(kNoLoads);  // this wave's part of the next matrices is in LDS
+    __syncthreads();
+  };
+  if (todo) {
+    int k = __builtin_ctz(todo);
+    todo &= todo - 1;
+    stage(k, table0);
+    fetch_half(k / 4);
+    __builtin_amdgcn_s_waitcnt(kNoLoads);
+    __syncthreads();
+    for (;;) {
+      int next = todo ? __builtin_ctz(todo) : -1;
+      todo &= todo - 1;
+      position(k, next, table0, table1);
+      if (next < 0) break;
+      k = next;
+      next = todo ? __builtin_ctz(todo) : -1;
+      todo &= todo - 1;
+      position(k, next, table1, table0);
+      if (next < 0) break;
+      k = next;
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+    if (grp + kAdvanceGroups * g < count && !((zero >> g) & 1u)) {
+      out[8 * state(g) + word0] = word_of(e0[g]);
+      out[8 * state(g) + word1] = word_of(e1[g]);
+    }
+  // states with a zero word, eight lanes each: the two groups of four in turn
+#pragma unroll 1
+  for (int g = 0; g < 2 * G; ++g) {
+    const int src = (int)((tid & 0x38u) | (g & 1 ? 4u : 0u)) * 4;  // a lane of the group that owns the state
+    const bool theirs = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)(zero >> (g / 2))) & 1u;
+    const uint32_t at = (grp & ~1u) + (g & 1) + kAdvanceGroups * (g / 2);
+    const bool mine_zero = theirs && at < count;
+    if (!__ballot(mine_zero)) continue;
+    const uint32_t i = mine_zero ? at : 0;
+    const uint32_t z = advance_zero_words(mine_zero ? in[8 * i + (tid & 7)] : 1u, offs + i * halves, a);
+    if (mine_zero) out[8 * i + (tid & 7)] = z;
   }
 }
 
@@ -1099,12 +1308,28 @@ hipError_t launch_batch_queue(const BatchArgs& a, int grid, int block_threads, h
   return hipGetLastError();
 }
 
-hipError_t launch_advance(const AdvanceArgs& a, hipStream_t stream) {
+namespace {
+
+template <int G>
+hipError_t advance_lds(const AdvanceArgs& a, hipStream_t stream) {
+  const uint64_t per = (uint64_t)kAdvanceGroups * G;
+  hipLaunchKernelGGL((k_advance_lds<G>), dim3((uint32_t)((a.n + per - 1) / per)), dim3(4 * kAdvanceGroups), 0, stream, a);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_advance(const AdvanceArgs& a, int states, hipStream_t stream) {
   if (a.n == 0) return hipSuccess;
-  const uint64_t threads = a.n * 8;
   if (a.n > (0xffffffffull >> 3) || a.words < 1 || a.words > (uint32_t)kAdvanceWords) return hipErrorInvalidValue;
-  const uint64_t blocks = (threads + 255) / 256;
-  hipLaunchKernelGGL(k_advance, dim3((uint32_t)blocks), dim3(256), 0, stream, a);
+  switch (states) {
+    case 0: break;
+    case 2: return advance_lds<2>(a, stream);
+    case 4: return advance_lds<4>(a, stream);
+    case 8: return advance_lds<8>(a, stream);
+    default: return hipErrorInvalidValue;
+  }
+  hipLaunchKernelGGL(k_advance, dim3((uint32_t)((a.n * 8 + 255) / 256)), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 

@@ -23,6 +23,9 @@ constexpr int kIdentityRec = kJumpPositions * kJumpValues * 8;
 // on first use.
 constexpr int kAdvanceWords = 4;
 constexpr int kWidePositions = 8 * kAdvanceWords;
+// Jump matrices (jump_matrix_entries) of one byte position: digits 0 (the
+// identity) to 255.
+constexpr int kPositionInts = (kJumpValues + 1) * kJumpMatrixInts;
 
 // Largest batch tile (outputs): keeps head + (k + 1) * tile of the tile
 // bounds within 64 bits.
@@ -35,11 +38,12 @@ struct DeviceTables {
   // at ((k * kJumpValues) + (d - 1)) * 8 + r; then the 8 rows of the
   // identity at kIdentityRec + r
   CoefRecord* jump = nullptr;
-  // (kWidePositions - kJumpPositions) * kJumpValues * 8 records: row r of
-  // A^(d 2^(kJumpBits k)) for k >= kJumpPositions at
-  // (((k - kJumpPositions) * kJumpValues) + (d - 1)) * 8 + r; null until the
+  // Jump matrices of the bulk advance: A^(d 2^(kJumpBits k)) at
+  // k kPositionInts + d kJumpMatrixInts, positions 0..kJumpPositions-1
+  const int32_t* digits = nullptr;
+  // the same for positions kJumpPositions..kWidePositions-1; null until the
   // first bulk advance with offsets wider than 64 bits
-  CoefRecord* wide = nullptr;
+  const int32_t* digits_wide = nullptr;
   // Matrix-core fill (k_fill_mfma): kMfmaClasses x 64 lanes x 8 bytes of
   // operand digits and kMfmaClasses x 4 x 4 accumulator start values; per
   // column length kMfmaColumnLen[i], the (kMfmaColumns - 1) x 8 records that
@@ -218,8 +222,8 @@ struct AdvanceArgs {
   uint32_t* out;
   uint64_t n;
   uint32_t words;  // 1..kAdvanceWords
-  const CoefRecord* jump;
-  const CoefRecord* wide;  // needed when words > 1
+  const int32_t* digits;
+  const int32_t* digits_wide;  // needed when words > 1
 };
 
 // Launchers (mrg8_device.hip).  All are asynchronous on `stream`.
@@ -233,8 +237,10 @@ hipError_t launch_batch(const BatchArgs& a, int grid, int block_threads, hipStre
 hipError_t launch_batch_queue(const BatchArgs& a, int grid, int block_threads, hipStream_t stream);
 // One tile per wave: ceil(ntiles / waves per block) blocks.
 hipError_t launch_batch_tiles(const BatchArgs& a, uint64_t ntiles, int block_threads, hipStream_t stream);
-// Eight lanes per state; a.n * 8 must stay below 2^32.
-hipError_t launch_advance(const AdvanceArgs& a, hipStream_t stream);
+// a.n * 8 must stay below 2^32.  `states` states per
+// group of four lanes: 0 reads the jump matrices from memory (k_advance), 2, 4
+// or 8 through LDS (k_advance_lds, blocks of 256 such groups).
+hipError_t launch_advance(const AdvanceArgs& a, int states, hipStream_t stream);
 // Copies `bytes` (a multiple of 4) from coherent pinned host memory `src` to
 // device memory `dst`, both 16-byte aligned, with a kernel on `stream`.
 hipError_t launch_stage(const void* src, void* dst, size_t bytes, hipStream_t stream);

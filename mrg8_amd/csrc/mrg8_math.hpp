@@ -187,6 +187,40 @@ inline bool all_nonzero(const uint32_t row[8]) {
   return true;
 }
 
+// ---- device jump matrices ----------------------------------------------------
+//
+// A jump matrix as eight lanes apply it, lane r computing row r of M s with
+// every word held by the lane that computed it, as a centred e == s (mod p).
+// Lane r reaches the words of its group in the order r ^ 0 .. r ^ 7 (what the
+// cross-lane moves of one instruction give), so entry k of row r is
+// M[r][r ^ k], centred: 64 int32, entries 0..3 of the eight rows and then
+// entries 4..7, so that a group's two 16-byte loads per lane each cover one
+// 128-byte line.  With e centred about 0 instead of about 2^30 a row needs no
+// additive constant of its own, and 32 bytes instead of a record's 48:
+//   V = kJumpBase + sum_k c_k e_k,  kJumpBase == 2^30 (mod p),
+// and the partly reduced x of V (x < 2^31 + 6) gives the next e = x - 2^30,
+// |e| <= 2^30 + 5.  V stays in (0, 2^64) while sum_k |c_k| (2^30 + 5) is
+// below 2^63 - 2^31, which holds unless all eight entries of a row are within
+// a few parts of 2^30; the tables are checked for it when they are built.
+constexpr int kJumpMatrixInts = 64;
+constexpr uint64_t kJumpBase = (1ull << 63) - 2 + kCenter;  // 2^63 == 2 (mod p)
+
+inline int32_t centred(uint32_t x) { return x <= (kP - 1) / 2 ? (int32_t)x : (int32_t)((int64_t)x - kP); }
+
+// `m` row-major; false when a row's coefficients are too large (see above).
+inline bool jump_matrix_entries(const uint32_t* m, int32_t* out) {
+  for (int r = 0; r < 8; ++r) {
+    uint64_t sum = 0;
+    for (int k = 0; k < 8; ++k) {
+      const int32_t c = centred(m[r * 8 + (r ^ k)] % kP);
+      out[(k / 4) * 32 + r * 4 + k % 4] = c;
+      sum += (uint64_t)(c < 0 ? -(int64_t)c : (int64_t)c);
+    }
+    if (sum > ((1ull << 63) - (1ull << 31)) / ((1ull << 30) + 5)) return false;
+  }
+  return true;
+}
+
 // ---- matrix-core fill tables ------------------------------------------------
 //
 // The int8 MFMA form of a step (16 outputs of each of 16 columns, output j

@@ -191,3 +191,54 @@ def test_advance_p_words_on_the_centred_path(gpu, oracle_mod):
         for i in range(n):
             want = oracle_mod.jump_bits(states[i], set_bits(offs[i]))
             assert got[i].tolist() == want.tolist(), (words, i, states[i].tolist(), hex(offs[i]))
+
+
+# Sizes at which the matrices come through LDS with 2, 4 or 8 states per lane
+# group on 256 CUs, an odd one with a partial last block for each, and the
+# last ones that read them from memory; sparse offsets skip byte positions.
+@pytest.mark.parametrize("n,words,sparse", [(80_000, 2, False), (120_001, 4, False), (131_072, 1, False),
+                                            (200_003, 3, False), (262_144, 4, True), (400_009, 4, False),
+                                            (1_048_577, 1, False), (1_100_000, 2, True)])
+def test_advance_large_n_against_small_calls(gpu, oracle_mod, n, words, sparse):
+    rng = np.random.default_rng(n + words)
+    states = rng.integers(1, P + 1, size=(n, 8), dtype=np.int64).astype(np.uint32)
+    zeros = rng.choice(n, size=40, replace=False)
+    states[zeros[:20], rng.integers(0, 8, size=20)] = 0
+    states[zeros[20:30], :7] = 0
+    states[zeros[30:]] = 0
+    offs = rng.integers(0, 2**64, size=(n, words), dtype=np.uint64)
+    if sparse:
+        offs &= np.uint64(0x00ff00000000ff00)
+    offs[5] = 0
+    say("advance large", n, words)
+    whole = run_advance_words(gpu, states, offs, words)
+    inplace = run_advance_words(gpu, states, offs, words, in_place=True)
+    assert np.array_equal(whole, inplace)
+    # the same states in calls small enough to read the matrices from memory
+    parts = np.concatenate([run_advance_words(gpu, states[i:i + 50_000], offs[i:i + 50_000], words)
+                            for i in range(0, n, 50_000)])
+    assert np.array_equal(whole, parts)
+    check = np.concatenate([zeros, [0, 5, 255, 256, n - 257, n - 256, n - 1], rng.integers(0, n, size=10)])
+    for i in check:
+        x = sum(int(v) << (64 * j) for j, v in enumerate(offs[i]))
+        if x < 1 << 200:
+            want = oracle_mod.jump_bits(states[i], set_bits(x)).tolist()
+        else:
+            want = closed_form_jump(oracle_mod.coeffs(), states[i], x)
+        assert whole[i].tolist() == want, (i, hex(x))
+
+
+def run_advance_words(gpu, states, offs, words, in_place=False):
+    from mrg8_amd.hip import DeviceBuffer
+
+    n = len(states)
+    d_in, d_off = DeviceBuffer(n * 32), DeviceBuffer(n * words * 8)
+    d_in.copy_from_host(np.ascontiguousarray(states))
+    d_off.copy_from_host(np.ascontiguousarray(offs))
+    d_out = d_in if in_place else DeviceBuffer(n * 32)
+    gpu.advance_states(d_in, d_off, words, d_out, n)
+    gpu.hip.synchronize()
+    got = d_out.copy_to_host(np.uint32, n * 8).reshape(n, 8)
+    for b in {id(x): x for x in (d_in, d_off, d_out)}.values():
+        b.free()
+    return got
