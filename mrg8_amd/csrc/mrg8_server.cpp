@@ -283,14 +283,19 @@ extern "C" int mrg8_server_create(int device, const mrg8_server_config* cfg, uin
   // accept requests whose rounded size can never fit
   s->cfg.max_output_bytes = s->cfg.max_output_bytes / kAlign * kAlign;
   if (!s->cfg.max_inflight) s->cfg.max_inflight = 4096;
-  // Defaults measured on MI355X with the log-uniform request mix at 490-680
-  // G samples/s offered: 4096-output tiles, one 256-thread block per CU (the
-  // batched kernel's best shape), 2^26-output steps (16 tiles per wave),
-  // three steps in flight, 1 ms age limit.  2^25-output steps stop keeping up
-  // above ~600 G samples/s; 2^27-output steps add ~0.2-0.4 ms to p99.
+  // Defaults measured on MI355X with the log-uniform request mix at 300-680
+  // G samples/s offered: 4096-output tiles, one 512-thread block per CU,
+  // 2^26-output steps (8 tiles per wave), three steps in flight, 1 ms age
+  // limit.  Two waves per SIMD and step: with one (256 threads) a step alone
+  // on the card leaves its SIMDs waiting for the recurrence, p99 0.44, 0.66,
+  // 0.95 and 1.61 ms at 300, 490, 600 and 680 G samples/s against 0.36, 0.54,
+  // 0.77 and 1.57 ms, a burst of 48 requests 0.79 against 0.72 ms; with three
+  // or more the steps in flight get in each other's way (p99 3 ms and more at
+  // 680).  2^25-output steps stop keeping up above ~600 G samples/s;
+  // 2^27-output steps add ~0.2-0.4 ms to p99.
   if (!s->cfg.tile_outputs) s->cfg.tile_outputs = 4096;
   if (!s->cfg.step_outputs) s->cfg.step_outputs = 1ull << 26;
-  if (!s->cfg.block_threads) s->cfg.block_threads = 256;
+  if (!s->cfg.block_threads) s->cfg.block_threads = s->cfg.blocks_per_cu ? 256 : 512;
   if (!s->cfg.blocks_per_cu) s->cfg.blocks_per_cu = 1;
   if (!s->cfg.steps_in_flight) s->cfg.steps_in_flight = 3;
   if (!s->cfg.age_limit_us) s->cfg.age_limit_us = 1000;
