@@ -96,8 +96,8 @@ int device_context(int device, DeviceContext** out) {
   (void)hipGetDevice(&prev);
   if ((e = hipSetDevice(device)) != hipSuccess) return hip_fail(e, "hipSetDevice");
 
-  // Coefficient records: block rows (row 0 of A^(k+1)) and jump rows.
-  std::vector<CoefRecord> lane(kLaneRows), jump((size_t)kIdentityRec + 8);
+  // Coefficient records: block rows (row 0 of A^(k+1)).
+  std::vector<CoefRecord> lane(kLaneRows);
   const std::vector<uint32_t> rows = block_rows(kLaneRows);
   for (int k = 0; k < kLaneRows; ++k) {
     if (!all_nonzero(&rows[(size_t)k * 8])) {
@@ -106,26 +106,8 @@ int device_context(int device, DeviceContext** out) {
     }
     lane[k] = make_record(&rows[(size_t)k * 8]);
   }
-  // Jump table: A^(d 2^(kJumpBits k)) for digit d = 1..kJumpValues at
-  // position k, built from A^(2^(kJumpBits k)) (a table entry) by repeated
-  // products.  Rows of the small powers (A^1..A^7) have structural zeros;
-  // the support mask keeps their exact-zero results exact.
-  const JumpTable& jt = host_jump_table();
-  for (int k = 0; k < kJumpPositions; ++k) {
-    std::vector<uint32_t> m(jt.at(kJumpBits * k), jt.at(kJumpBits * k) + 64), p = m;
-    for (int d = 1; d <= kJumpValues; ++d) {
-      if (d > 1) p = mat_mul(p.data(), m.data());
-      for (int r = 0; r < 8; ++r)
-        jump[((size_t)k * kJumpValues + (d - 1)) * 8 + r] = make_record(&p[(size_t)r * 8]);
-    }
-  }
-  for (int r = 0; r < 8; ++r) {  // the identity: a digit 0 leaves the state as it is
-    uint32_t row[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    row[r] = 1;
-    jump[(size_t)kIdentityRec + r] = make_record(row);
-  }
-
-  // the same matrices as the bulk advance reads them
+  // Jump matrices.  Rows of the small powers (A^1..A^7) have structural
+  // zeros, which keep exact-zero results exact (jump_zero_words).
   std::vector<int32_t> digits((size_t)kJumpPositions * kPositionInts);
   if (!build_digits(0, kJumpPositions, digits.data())) {
     (void)hipSetDevice(prev);
@@ -154,7 +136,7 @@ int device_context(int device, DeviceContext** out) {
   if (xcc < 1) xcc = 1;
   ctx->num_xcc = xcc;
   void* p = nullptr;
-  const size_t rec_bytes = sizeof(CoefRecord) * (lane.size() + jump.size());
+  const size_t rec_bytes = sizeof(CoefRecord) * lane.size();
   // operand digits and accumulator start values do not depend on the column length
   size_t mfma_bytes = sizeof(uint32_t) * (mt[0].a.size() + mt[0].c.size());
   for (int i = 0; i < 2; ++i)
@@ -169,12 +151,9 @@ int device_context(int device, DeviceContext** out) {
   // the jump matrices first: their 256-byte blocks stay on line boundaries
   ctx->tables.digits = static_cast<const int32_t*>(p);
   ctx->tables.lane = reinterpret_cast<CoefRecord*>(static_cast<uint8_t*>(p) + digit_bytes);
-  ctx->tables.jump = ctx->tables.lane + lane.size();
   e = hipMemcpy(p, digits.data(), digit_bytes, hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(ctx->tables.lane, lane.data(), sizeof(CoefRecord) * lane.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(ctx->tables.jump, jump.data(), sizeof(CoefRecord) * jump.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess && mfma_ok) {
     // records first (16-byte aligned after the 48-byte records), then the
     // operand digits, the accumulator start values and the step tables
@@ -255,41 +234,43 @@ int format_size(int format) {
   }
 }
 
-// Default launch shape for a single-stream fill of n outputs.  Measured on
-// MI355X (2^28 outputs): doubles are fastest with 512-thread blocks in XCD
-// runs (fill_xcd_group), 4 outputs per lane and 2048 outputs per wave, words
-// with 256-thread blocks and 8192 per wave; small fills shrink the per-wave
-// run (down to four iterations) so that every SIMD still gets waves.
+// Default launch shape for a single-stream fill of n outputs with the vector
+// kernel.  Doubles: one-wave blocks of 1024 outputs.  Short-lived waves keep
+// the grid's stores close to address order, and a block of one wave makes
+// room for the next as soon as it ends.  Measured on MI355X against 512-thread
+// blocks of 2048 per wave: 2^28 doubles 320-330 us against 332-339 us, 2^26
+// 81 against 90 us, 2^24 23.8 against 26.2 us, 2^22 8.4 against 8.9 us; 512
+// per wave takes 425 us at 2^28 (the wave's start costs as much as its
+// outputs).  At four or fewer waves per CU the wave's own time counts, and
+// 512 outputs are faster (2^20: 4.65 against 4.8 us).  Words below the
+// matrix-core fill's sizes: 256-thread blocks, down to 1024 outputs per wave
+// while that leaves fewer than four waves per SIMD (2^20: 4.4 us, 512 per
+// wave 4.6 us).
 void default_shape(const DeviceContext& ctx, uint64_t n, int format, int per_lane, int* block, uint64_t* tile) {
   const uint64_t quantum = 64ull * per_lane;
-  uint64_t t = format == MRG8_U32 ? 8192 : 2048;
   const uint64_t cu = (uint64_t)ctx.num_cu;
-  const uint64_t min_waves = cu * 4 * 4;  // four waves per SIMD
-  while (t > 4 * quantum && (n + t - 1) / t < min_waves) t /= 2;
+  uint64_t t = 1024;
+  if (format == MRG8_U32) {
+    t = 8192;
+    while (t > 4 * quantum && (n + t - 1) / t < cu * 16) t /= 2;  // four waves per SIMD
+  } else if ((n + t - 1) / t <= cu * 4) {
+    t = 512;
+  }
   *tile = std::max<uint64_t>(quantum, t / quantum * quantum);
-  // Double fills take 512-thread blocks, and 256-thread blocks when every CU
-  // gets at most 4 waves (on MI355X, against 1024-thread blocks: 2^20 and
-  // 2^21 doubles 15-44 % faster, 2^22..2^25 0-4 % faster; from 2^25 on in
-  // XCD runs, 2^26 the same, 2^27 1 % and 2^28 1-2 % faster at full clock
-  // and 3.5-5 % faster in the first launches after an idle spell, while the
-  // power manager holds the clock down).
-  int b = format == MRG8_U32 ? 256 : 512;
-  const uint64_t waves = (n + *tile - 1) / *tile;
-  if (format != MRG8_U32 && waves <= cu * 4) b = 256;
-  *block = b;
+  *block = format == MRG8_U32 ? 256 : 64;
 }
 
 // Blocks per XCD run of a vector-kernel fill (1: blocks in dispatch order).
-// The dispatcher deals blocks to the XCDs in turn; a double fill of 64 or
-// more waves per CU instead gives each XCD runs of 32768 threads' worth of
-// consecutive output (64 blocks of 512 threads).  Measured on MI355X, 2^28
-// doubles at 2048 per wave: 512-thread blocks 366 us in dispatch order and
-// 337-341 us in runs of 64; 256-thread blocks 391 and 340 us (runs of 128);
-// 1024-thread blocks 338-349 us either way.  Word fills (8192 per wave) were
-// 1-17 % slower in runs, and are left in dispatch order.
+// The dispatcher deals blocks to the XCDs in turn; a double fill of 16 or
+// more waves per CU instead gives each XCD runs of 64 blocks' consecutive
+// output, or of 32768 threads' with blocks of more than 512.  Measured on
+// MI355X with the default shape, runs of 1, 16, 64 and 256 blocks: 2^28
+// doubles 382, 335, 318 and 326 us, 2^24 24.5, 25.6, 24.0 and 25.3 us, 2^22
+// 8.5, 8.8, 8.4 and 9.1 us; 2^21 (8 waves per CU) 5.5, 5.8, 5.7 and 5.9 us.
+// Word fills were slower in runs and are left in dispatch order.
 uint32_t fill_xcd_group(const DeviceContext& ctx, int format, uint64_t waves, int block_threads) {
-  if (format == MRG8_U32 || ctx.num_xcc <= 1 || waves < (uint64_t)ctx.num_cu * 64) return 1;
-  return xcd_run_blocks(ctx, block_threads);
+  if (format == MRG8_U32 || ctx.num_xcc <= 1 || waves < (uint64_t)ctx.num_cu * 16) return 1;
+  return std::min(64u, xcd_run_blocks(ctx, block_threads));
 }
 
 namespace {
@@ -319,14 +300,20 @@ int fill_mfma(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, void
   a.head = head;
   a.tiles = tiles;
   a.column = (uint32_t)column;
-  a.waves_per_block = (uint32_t)(block_threads ? block_threads / 64 : format == MRG8_U32 ? 8 : 16);
-  // default: 32 KiB of output per wave, fewer tiles when that would leave
-  // fewer than 8 waves per CU
+  a.waves_per_block = (uint32_t)(block_threads ? block_threads / 64 : format == MRG8_U32 ? 4 : 16);
+  // default: 32 KiB of output per wave for doubles and 16 KiB for words, fewer
+  // tiles when that would leave fewer than 8 waves per CU
+  const uint64_t bytes_per_wave = format == MRG8_U32 ? 16384 : 32768;
   const uint64_t per = outputs_per_wave
                            ? outputs_per_wave / tile
-                           : std::min<uint64_t>(32768 / (uint64_t)esz / tile, tiles / ((uint64_t)ctx.num_cu * 8));
+                           : std::min<uint64_t>(bytes_per_wave / (uint64_t)esz / tile, tiles / ((uint64_t)ctx.num_cu * 8));
   a.tiles_per_wave = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(per, 1), 1u << 20);
   a.waves = (tiles + a.tiles_per_wave - 1) / a.tiles_per_wave;
+  // blocks of four waves in XCD runs of 16 (1 MiB of words at the default
+  // run): 2^28 words 174-177 us; in dispatch order 190 us, 512-thread blocks
+  // of 8192 words per wave 179-181 us either way
+  a.xcds = (uint32_t)ctx.num_xcc;
+  a.xcd_group = a.waves_per_block == 4 && a.waves >= (uint64_t)ctx.num_cu * 16 ? 16 : 1;
   const uint64_t tail_first = head + tiles * tile;
   if (head) {
     a.extra_first[a.extra] = 0;
@@ -339,7 +326,7 @@ int fill_mfma(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, void
   std::memcpy(a.start.state, state, sizeof a.start.state);
   a.start.offset = offset;
   a.lane = ctx.tables.lane;
-  a.jump = ctx.tables.jump;
+  a.digits = ctx.tables.digits;
   a.mfma_a = ctx.tables.mfma_a;
   a.mfma_c = ctx.tables.mfma_c;
   a.mfma_fan = ctx.tables.mfma_fan[ci];
@@ -423,7 +410,7 @@ int fill_device(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, vo
   std::memcpy(a.start.state, state, sizeof a.start.state);
   a.start.offset = offset;
   a.lane = ctx.tables.lane;
-  a.jump = ctx.tables.jump;
+  a.digits = ctx.tables.digits;
   a.xcds = (uint32_t)ctx.num_xcc;
   a.xcd_group = fill_xcd_group(ctx, format, fill_waves(n, head, tile), block_threads);
   int prev = 0;

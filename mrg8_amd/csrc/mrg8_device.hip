@@ -16,10 +16,10 @@
 //   * A wave reaches its first position with a jump: each non-zero byte d
 //     at position k of the 64-bit offset is one product with A^(d 256^k)
 //     (at most 8 steps).  Eight lane groups of eight lanes jump eight states
-//     at once, lane r of a group computing row r, and the next digit's
-//     record is fetched one step ahead.
-//   * k_fill: one stream, one tile per wave; the block's start states are
-//     jumped by its first waves and shared through LDS.
+//     at once, lane r of a group holding word r and computing row r, with
+//     the rows of the next digits already on their way.
+//   * k_fill: one stream, one tile per wave, each wave on its own (no LDS, no
+//     barrier).
 //   * k_batch: many streams (segments), a persistent grid striding over
 //     tiles, tables and counts read from one device block.
 //   * Blocks reach their part of the output through xcd_block: the
@@ -39,34 +39,19 @@ typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
 struct Coef {
   int32_t c[8];
   uint64_t b0;
-  uint32_t support;
 };
 
 __device__ __forceinline__ Coef load_coef(const CoefRecord* __restrict__ p) {
   const u4_t* q = reinterpret_cast<const u4_t*>(p);
-  u4_t a = q[0], b = q[1], c = q[2];
-  Coef k;
-  k.c[0] = (int32_t)a.x; k.c[1] = (int32_t)a.y; k.c[2] = (int32_t)a.z; k.c[3] = (int32_t)a.w;
-  k.c[4] = (int32_t)b.x; k.c[5] = (int32_t)b.y; k.c[6] = (int32_t)b.z; k.c[7] = (int32_t)b.w;
-  k.b0 = (uint64_t)c.x | ((uint64_t)c.y << 32);
-  k.support = c.z;
-  return k;
-}
-
-// The 11 used words of a record, without its pad word: a load into a register
-// nothing reads lets the compiler reuse that register while the load is in
-// flight, which forces a wait for the load where the register is reused --
-// in a prefetching loop, before the step the prefetch should overlap.
-__device__ __forceinline__ Coef load_coef11(const CoefRecord* __restrict__ p) {
-  const u4_t* q = reinterpret_cast<const u4_t*>(p);
   const u4_t a = q[0], b = q[1];
+  // the two words of b0 alone: a load into a register nothing reads lets the
+  // compiler reuse that register while the load is in flight, which forces a
+  // wait for it there, before loads that could be in flight with it
   const u2_t c = *reinterpret_cast<const u2_t*>(q + 2);
-  const uint32_t support = reinterpret_cast<const uint32_t*>(q + 2)[2];
   Coef k;
   k.c[0] = (int32_t)a.x; k.c[1] = (int32_t)a.y; k.c[2] = (int32_t)a.z; k.c[3] = (int32_t)a.w;
   k.c[4] = (int32_t)b.x; k.c[5] = (int32_t)b.y; k.c[6] = (int32_t)b.z; k.c[7] = (int32_t)b.w;
   k.b0 = (uint64_t)c.x | ((uint64_t)c.y << 32);
-  k.support = support;
   return k;
 }
 
@@ -108,131 +93,142 @@ __device__ __forceinline__ void dot_residues(const Coef (&k)[PL], const int32_t 
   }
 }
 
-// The value of v in each of the eight lanes of this lane's 8-lane group,
-// w[j] from lane (lane & ~7) | j: ds_swizzle in bit mode (and-mask 0x18 keeps
-// the group bits within the 32-lane half, or-mask j picks the lane), so no
-// lane-address registers are needed.
-template <int J>
-__device__ __forceinline__ uint32_t group_lane(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x18 | (J << 5));
-}
-
-__device__ __forceinline__ void gather_group(uint32_t v, uint32_t w[8]) {
-  w[0] = group_lane<0>(v);
-  w[1] = group_lane<1>(v);
-  w[2] = group_lane<2>(v);
-  w[3] = group_lane<3>(v);
-  w[4] = group_lane<4>(v);
-  w[5] = group_lane<5>(v);
-  w[6] = group_lane<6>(v);
-  w[7] = group_lane<7>(v);
-}
-
 __device__ __forceinline__ void centre(const uint32_t s[8], int32_t e[8]) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) e[j] = (int32_t)(s[j] - kCenter);
 }
 
-// Advances eight states at once: lane group g = lane / 8 holds its own state
-// (replicated in the group's lanes, s[] per lane) and its own 64-bit offset;
-// for the group's lowest non-zero digit d (kJumpBits bits) at position k,
-// lane r of the group computes row r of A^(d 2^(kJumpBits k)), and the
-// group's eight new words are gathered back with ds_swizzle.  Groups with no
-// digits left idle until every group is done; a 64-bit jump takes at most
-// kJumpPositions steps.
-__device__ __forceinline__ const CoefRecord* digit_row(const CoefRecord* __restrict__ jrec, uint64_t off, int row) {
-  const int k = __builtin_ctzll(off) / kJumpBits;
-  const int d = (int)((off >> (kJumpBits * k)) & (uint64_t)kJumpValues);
-  return jrec + ((k * kJumpValues + (d - 1)) * 8 + row);
+// ---- jumps: eight lanes per state, lane r holding word r and computing row r
+
+// The value of v in the lanes l ^ 0 .. l ^ 7 of this lane's group of eight.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
 }
 
-__device__ __forceinline__ uint64_t drop_digit(uint64_t off) {
-  return off & ~((uint64_t)kJumpValues << (__builtin_ctzll(off) / kJumpBits * kJumpBits));
+__device__ __forceinline__ void gather_xor(uint32_t v, uint32_t w[8]) {
+  constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kXor3 = 0x1B;  // quad_perm [1,0,3,2], [2,3,0,1], [3,2,1,0]
+  const uint32_t m = dpp<0x141>(v);                        // row_half_mirror: lane ^ 7
+  w[0] = v;
+  w[1] = dpp<kXor1>(v);
+  w[2] = dpp<kXor2>(v);
+  w[3] = dpp<kXor3>(v);
+  w[4] = dpp<kXor3>(m);
+  w[5] = dpp<kXor2>(m);
+  w[6] = dpp<kXor1>(m);
+  w[7] = m;
 }
 
-__device__ __forceinline__ void jump_groups(uint32_t s[8], uint64_t off, const CoefRecord* __restrict__ jrec) {
-  const int row = threadIdx.x & 7;
-  Coef k = {};
-  if (off) k = load_coef(digit_row(jrec, off, row));
-  while (__ballot(off != 0)) {
-    const bool active = off != 0;
-    const uint64_t rest = active ? drop_digit(off) : 0;
-    Coef next = {};
-    if (rest) next = load_coef(digit_row(jrec, rest, row));  // one step ahead
-    int32_t e[8];
-    uint32_t nz = 0;
-    centre(s, e);
+// This lane's row of a jump matrix (entries in the order of gather_xor).
+struct JumpRow {
+  int32_t c[8];
+};
+
+__device__ __forceinline__ JumpRow load_row(const int32_t* p) {  // p: the matrix + 4 * row
+  const u4_t a = *reinterpret_cast<const u4_t*>(p), b = *reinterpret_cast<const u4_t*>(p + 32);
+  return JumpRow{{(int32_t)a.x, (int32_t)a.y, (int32_t)a.z, (int32_t)a.w, (int32_t)b.x, (int32_t)b.y, (int32_t)b.z,
+                  (int32_t)b.w}};
+}
+
+// The next centred word from a row's sum (see jump_matrix_entries).
+__device__ __forceinline__ int32_t reduce_centred(uint64_t v) {
+  const uint64_t f = fold_hi((uint32_t)(v >> 32), (uint32_t)v);
+  return (int32_t)(((uint32_t)f & kP) + (uint32_t)(f >> 31) - kCenter);
+}
+
+// One product: this lane's centred word of (matrix) x (state), the state's
+// words being the centred e of the group's lanes.
+__device__ __forceinline__ int32_t jump_row(const JumpRow& m, int32_t e) {
+  uint32_t w[8];
+  gather_xor((uint32_t)e, w);
+  uint64_t v = kJumpBase;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) nz |= (s[j] != 0u ? 1u : 0u) << j;
-    const uint32_t y = (k.support & nz) ? dot_residue(k, e) + 1u : 0u;
-    uint32_t w[8];
-    gather_group(y, w);
+  for (int k = 0; k < 8; ++k) v += (uint64_t)((int64_t)m.c[k] * (int64_t)(int32_t)w[k]);
+  return reduce_centred(v);
+}
+
+__device__ __forceinline__ int32_t centre_word(uint32_t s) { return (int32_t)(s >= kCenter ? s - kP : s); }
+__device__ __forceinline__ uint32_t word_of(int32_t e) { return (uint32_t)(e > 0 ? e : e + (int32_t)kP); }  // in [1, p]
+
+__device__ __forceinline__ uint32_t digit_of(uint32_t half, int k) { return (half >> (8 * (k & 3))) & 0xffu; }
+
+// The product for a state that has a zero word (this lane's word s, its
+// group's digit d): bigDotProd is 0 exactly where every product of a row is.
+// A state without a zero word never gets one (no row of a power of A is
+// zero), so only waves that start with such a state need this.
+__device__ __forceinline__ uint32_t jump_zero_words(uint32_t s, uint32_t d, const int32_t* position) {
+  const JumpRow m = load_row(position + d * kJumpMatrixInts + 4 * (threadIdx.x & 7));
+  uint32_t w[8];
+  gather_xor(s, w);
+  bool any = false;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s[j] = active ? w[j] : s[j];
-    off = rest;
-    k = next;
+  for (int q = 0; q < 8; ++q) any = any || (m.c[q] != 0 && w[q] != 0u);
+  const uint32_t y = word_of(jump_row(m, centre_word(s)));
+  return any ? y : 0u;
+}
+
+// Rows of four byte positions of an offset (32 bits of it), and their
+// products; positions where no group of the wave has a digit are skipped.
+__device__ __forceinline__ void load_rows4(JumpRow m[4], const int32_t* positions, uint32_t half) {
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+    m[b] = load_row(positions + b * kPositionInts + digit_of(half, b) * kJumpMatrixInts + 4 * (threadIdx.x & 7));
+}
+
+__device__ __forceinline__ int32_t apply_rows4(const JumpRow m[4], uint32_t half, int32_t e) {
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+    if (__ballot(digit_of(half, b) != 0u)) e = jump_row(m[b], e);
+  return e;
+}
+
+// Jumps eight states at once: this lane's group of eight holds one state (word
+// s of it here) and its own 64-bit offset.  The rows of all of an offset's
+// digits are independent loads: AHEAD of them are in flight, so a jump does not
+// wait for memory once per digit.  65536 random 63-bit jumps and 256 words
+// each: 25.5 us, 27.4 us with 48-byte records fetched one digit ahead and
+// words gathered through LDS swizzles; one tile per wave 73 against 104 us.
+template <int AHEAD = 4>
+__device__ __forceinline__ uint32_t jump_group(uint32_t s, uint64_t off, const int32_t* __restrict__ digits) {
+  if (!__ballot(off != 0)) return s;
+  const uint32_t lo = (uint32_t)off, hi = (uint32_t)(off >> 32);
+  const bool more = __ballot(hi != 0u);
+  auto row = [&](int k) {
+    return load_row(digits + k * kPositionInts + digit_of(k < 4 ? lo : hi, k) * kJumpMatrixInts + 4 * (threadIdx.x & 7));
+  };
+  // issued before the state is looked at, which may still be on its way
+  JumpRow m[AHEAD];
+#pragma unroll
+  for (int k = 0; k < AHEAD; ++k) m[k] = row(k);
+  if (__ballot(s == 0u)) {
+#pragma unroll 1
+    for (int k = 0; k < kJumpPositions; ++k) {
+      const uint32_t d = digit_of(k < 4 ? lo : hi, k);
+      if (__ballot(d != 0u)) s = jump_zero_words(s, d, digits + k * kPositionInts);
+    }
+    return s;
   }
-}
-
-// The same jump, pipelined, for the persistent batched kernel, whose jumps
-// are on the critical path when segments are short and offsets long.  The
-// offset's digits are taken position by position, up to the highest position
-// where some group has a digit, skipping positions where every group's digit
-// is 0: at position k, lane r of each group computes row r of
-// A^(d 2^(kJumpBits k)) for its group's digit d (row r of the identity when d
-// is 0).  The next position's record is fetched while the current step
-// computes (an unconditional load, so that the compiler's wait for it is not
-// hoisted above the step), and the zero-product test runs only when the
-// state has a zero word.  65536 random 63-bit jumps + 256 words each: 30 us
-// against 34 us with jump_groups.  The one-tile-per-wave kernels keep
-// jump_groups: with this version their long fills ran 2 % slower (and 3 %
-// slower still with no jump at all, so a block's jump phase, which delays its
-// first stores, does not cost those kernels time).
-__device__ __forceinline__ uint32_t digit_at(uint64_t off, int k) {
-  return (uint32_t)(off >> (kJumpBits * k)) & (uint32_t)kJumpValues;
-}
-
-__device__ __forceinline__ const CoefRecord* digit_rec(const CoefRecord* __restrict__ jrec, uint64_t off, int k,
-                                                       int row) {
-  const int d = (int)digit_at(off, k);
-  return jrec + (d ? (k * kJumpValues + d - 1) * 8 + row : kIdentityRec + row);
-}
-
-// One step of the pipelined jumps below: lane r of group g computes row r of
-// the group's matrix (record c) times the group's state, and the group's
-// eight new words are gathered back.
-template <bool ZERO_WORDS = true>
-__device__ __forceinline__ void jump_step(uint32_t s[8], const Coef& c) {
-  int32_t e[8];
-  centre(s, e);
-  uint32_t y = dot_residue(c, e) + 1u;
-  // bigDotProd is 0 when every product is 0; with all eight words non-zero
-  // that cannot happen (no row of a power of A is zero)
-  uint32_t smin = s[0];
+  int32_t e = centre_word(s);
 #pragma unroll
-  for (int j = 1; j < 8; ++j) smin = min(smin, s[j]);
-  if (ZERO_WORDS && smin == 0u) {
-    uint32_t nz = 0;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) nz |= (s[j] != 0u ? 1u : 0u) << j;
-    if (!(c.support & nz)) y = 0u;
+  for (int k = 0; k < kJumpPositions; ++k) {
+    if (k == 4 && !more) break;
+    if (__ballot(digit_of(k < 4 ? lo : hi, k) != 0u)) e = jump_row(m[k % AHEAD], e);
+    if (k + AHEAD < 4 || (k + AHEAD < kJumpPositions && more)) m[k % AHEAD] = row(k + AHEAD);
   }
-  gather_group(y, s);
+  return word_of(e);
 }
 
-__device__ __forceinline__ void jump_groups_pipelined(uint32_t s[8], uint64_t off,
-                                                      const CoefRecord* __restrict__ jrec) {
-  const int row = threadIdx.x & 7;
-  if (!__ballot(off != 0)) return;
-  Coef c = load_coef11(digit_rec(jrec, off, 0, row));
-  for (int k = 0;; ++k) {
-    // wave-uniform: no group has a digit above position k
-    const bool last = k + 1 == kJumpPositions || !__ballot((off >> (kJumpBits * (k + 1))) != 0);
-    const Coef next = load_coef11(digit_rec(jrec, last ? 0 : off, last ? 0 : k + 1, row));
-    if (__ballot(digit_at(off, k) != 0)) jump_step(s, c);
-    if (last) break;
-    c = next;
+// This lane's word (lane & 7) of a state in uniform registers.
+__device__ __forceinline__ uint32_t own_word(const uint32_t st[8]) {
+  const uint32_t row = threadIdx.x & 7;
+  uint32_t w = st[0];
+#pragma unroll
+  for (int j = 1; j < 8; ++j) {
+    uint32_t x = st[j];
+    asm("" : "+s"(x));  // a select between registers, not a load at a computed address
+    w = row == (uint32_t)j ? x : w;
   }
+  return w;
 }
 
 template <int FMT>
@@ -435,35 +431,27 @@ __device__ __forceinline__ uint64_t xcd_block(uint32_t b, uint32_t nb, uint32_t 
   return (uint64_t)(q / g * span + (b - q * x) * g + q % g);
 }
 
+// Bound by the store stream for long fills and by the latency of a wave's
+// start (rows of its jump, then its lane records) for short ones.  A wave jumps
+// its own state, all eight lane groups alike: with the block's states jumped
+// by one wave and handed over in LDS behind a barrier, 2^28 doubles took 327
+// us against 320 us, 2^26 86 against 82 us (64-thread blocks, 1024 outputs
+// per wave).  The lane records are loaded after the jump: loaded before it, or
+// between its loads and its products, 2^24 doubles took 25.1 and 24.9 us
+// against 24.1 us (2^28: 314 and 316 against 320 us).  Limited to 80
+// registers for a sixth wave per SIMD it spills (2^28: 401 us).
 template <int FMT, int PL>
 __global__ __launch_bounds__(1024) void k_fill(FillArgs a) {
-  // Start states of the block's waves: wave j (j < ceil(nw / 8)) jumps the
-  // states of waves 8j..8j+7 together (one 8-lane group each) and leaves
-  // them in LDS; every wave then reads its own.
-  __shared__ uint32_t start_state[16][8];
-  const int lane = threadIdx.x & 63;
   const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform wave index
   const uint32_t nw = blockDim.x >> 6;
-  const uint64_t wave0 = xcd_block(blockIdx.x, gridDim.x, a.xcds, a.xcd_group) * nw;
-  if (wib * 8 < nw) {
-    const uint32_t target = wib * 8 + (lane >> 3);
-    uint32_t s[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s[j] = a.start.state[j];
-    jump_groups(s, target < nw ? a.start.offset + fill_first(a, wave0 + target) : 0, a.jump);
-    if (target < nw && (lane & 7) == 0) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) start_state[target][j] = s[j];
-    }
-  }
-  __syncthreads();
-  const uint64_t w = wave0 + wib;
+  const uint64_t w = xcd_block(blockIdx.x, gridDim.x, a.xcds, a.xcd_group) * nw + wib;
   const uint64_t first = fill_first(a, w);
   if (first >= a.n) return;
   const uint64_t cnt = min(a.head + (w + 1) * a.tile, a.n) - first;
+  const uint32_t word = jump_group(own_word(a.start.state), a.start.offset + first, a.digits);
   uint32_t s[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) s[j] = __builtin_amdgcn_readfirstlane(start_state[wib][j]);
+  for (int j = 0; j < 8; ++j) s[j] = __builtin_amdgcn_readlane(word, j);
   Coef k[PL];
   load_lane_coefs<FMT, PL>(k, a.lane);
   generate_run<FMT, PL>(static_cast<typename Out<FMT>::T*>(a.out) + first, cnt, s, k, a.lane);
@@ -483,6 +471,13 @@ __device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int lane) {
   const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, lane);
   const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(v >> 32), lane);
   return (uint64_t)lo | ((uint64_t)hi << 32);
+}
+
+// A device address read from memory as a pointer: known to be global memory,
+// so that stores through it are global and not flat, which also count as LDS
+// accesses (4096 streams on the address-order grid: 2.601 to 2.591 ms).
+__device__ __forceinline__ void* global_pointer(uint64_t address) {
+  return (void*)(__attribute__((address_space(1))) void*)address;
 }
 
 // The tables of a batch block (see BatchHeader).
@@ -551,18 +546,15 @@ __global__ __launch_bounds__(1024) void k_batch(BatchArgs a) {
     const uint32_t ngrp = (uint32_t)min<uint64_t>(kGroup, mine_total - j0);
     const bool mine = (uint32_t)grp < ngrp;
     const TileInfo ti = lookup_tile(tab, a, (j0 + (mine ? grp : 0)) * nwaves + wave);
-    uint32_t s[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s[j] = ti.state[j];
-    jump_groups_pipelined(s, mine ? ti.offset : 0, a.jump);
+    const uint32_t s = jump_group(ti.state[lane & 7], mine ? ti.offset : 0, a.digits);
     // loaded after the jumps so that they hold no registers during them
     Coef k[2];
     load_lane_coefs<0, 2>(k, a.lane);  // the PL = 2 layout is the same for every format
     for (uint32_t g = 0; g < ngrp; ++g) {
       uint32_t u[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) u[j] = __builtin_amdgcn_readlane(s[j], 8 * g);
-      void* out = reinterpret_cast<void*>(readlane_u64(ti.dst, 8 * g));
+      for (int j = 0; j < 8; ++j) u[j] = __builtin_amdgcn_readlane(s, 8 * g + j);
+      void* out = global_pointer(readlane_u64(ti.dst, 8 * g));
       const uint64_t ucnt = readlane_u64(ti.cnt, 8 * g);
       switch (__builtin_amdgcn_readlane(ti.fmt, 8 * g)) {
         case 0: batch_tile<0, 2, 16>(out, ucnt, u, k, a.lane); break;
@@ -582,10 +574,10 @@ __device__ __forceinline__ void batch_tile_alone(void* out, uint64_t cnt, uint32
   batch_tile<FMT, 4>(out, cnt, s, k, lane_rec);
 }
 
-// Batched kernel with one tile per wave (grid = tiles / waves per block), the
-// structure of k_fill: waves 0-1 of a block look up and jump the start states
-// of the block's tiles (8-lane groups) and leave them in LDS; every wave then
-// generates its own tile and exits.
+// Batched kernel with one tile per wave (grid = tiles / waves per block):
+// wave 0 of a block looks up and jumps the start states of the block's tiles
+// (8-lane groups; wave 1 too in blocks of more than eight waves) and leaves
+// them in LDS; every wave then generates its own tile and exits.
 __global__ __launch_bounds__(1024) void k_batch_tiles(BatchArgs a) {
   __shared__ uint32_t start_state[16][8];
   __shared__ uint64_t start_dst[16], start_cnt[16];
@@ -600,13 +592,9 @@ __global__ __launch_bounds__(1024) void k_batch_tiles(BatchArgs a) {
     const uint32_t target = wib * 8 + (lane >> 3);
     const bool mine = target < nw && tile0 + target < tab.ntiles;
     const TileInfo ti = lookup_tile(tab, a, mine ? tile0 + target : tile0);
-    uint32_t s[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s[j] = ti.state[j];
-    jump_groups(s, mine ? ti.offset : 0, a.jump);
+    const uint32_t s = jump_group(ti.state[lane & 7], mine ? ti.offset : 0, a.digits);
+    if (mine) start_state[target][lane & 7] = s;
     if (mine && (lane & 7) == 0) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) start_state[target][j] = s[j];
       start_dst[target] = ti.dst;
       start_cnt[target] = ti.cnt;
       start_fmt[target] = ti.fmt;
@@ -618,7 +606,7 @@ __global__ __launch_bounds__(1024) void k_batch_tiles(BatchArgs a) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) u[j] = __builtin_amdgcn_readfirstlane(start_state[wib][j]);
   const uint64_t d = start_dst[wib], c = start_cnt[wib];
-  void* out = reinterpret_cast<void*>(readlane_u64(d, 0));
+  void* out = global_pointer(readlane_u64(d, 0));
   const uint64_t cnt = readlane_u64(c, 0);
   switch (__builtin_amdgcn_readfirstlane(start_fmt[wib])) {
     case 0: batch_tile_alone<0>(out, cnt, u, a.lane); break;
@@ -657,13 +645,9 @@ __global__ __launch_bounds__(1024) void k_batch_queue(BatchArgs a) {
       const uint32_t target = wib * 8 + (lane >> 3);
       const bool mine = target < nw && tile0 + target < tab.ntiles;
       const TileInfo ti = lookup_tile(tab, a, mine ? tile0 + target : tile0);
-      uint32_t s[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) s[j] = ti.state[j];
-      jump_groups(s, mine ? ti.offset : 0, a.jump);
+      const uint32_t s = jump_group<2>(ti.state[lane & 7], mine ? ti.offset : 0, a.digits);
+      if (mine) start_state[target][lane & 7] = s;
       if (mine && (lane & 7) == 0) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) start_state[target][j] = s[j];
         start_dst[target] = ti.dst;
         start_cnt[target] = ti.cnt;
         start_fmt[target] = ti.fmt;
@@ -675,12 +659,14 @@ __global__ __launch_bounds__(1024) void k_batch_queue(BatchArgs a) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) u[j] = __builtin_amdgcn_readfirstlane(start_state[wib][j]);
       const uint64_t d = start_dst[wib], c = start_cnt[wib];
-      void* out = reinterpret_cast<void*>(readlane_u64(d, 0));
+      void* out = global_pointer(readlane_u64(d, 0));
       const uint64_t cnt = readlane_u64(c, 0);
+      const CoefRecord* lane_rec = a.lane;
+      asm("" : "+s"(lane_rec));  // read per tile: the records of both layouts held across the loop spill
       switch (__builtin_amdgcn_readfirstlane(start_fmt[wib])) {
-        case 0: batch_tile_alone<0>(out, cnt, u, a.lane); break;
-        case 1: batch_tile_alone<1>(out, cnt, u, a.lane); break;
-        default: batch_tile_alone<2>(out, cnt, u, a.lane); break;
+        case 0: batch_tile_alone<0>(out, cnt, u, lane_rec); break;
+        case 1: batch_tile_alone<1>(out, cnt, u, lane_rec); break;
+        default: batch_tile_alone<2>(out, cnt, u, lane_rec); break;
       }
     }
     __syncthreads();  // LDS and `group` are rewritten by the next group
@@ -697,79 +683,15 @@ __global__ __launch_bounds__(1024) void k_batch_queue(BatchArgs a) {
 
 // ---- bulk advance: many states, offsets of up to kAdvanceWords words --------
 
-// The value of v in the lanes l ^ 0 .. l ^ 7 of this lane's group of eight.
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
-}
-
-__device__ __forceinline__ void gather_xor(uint32_t v, uint32_t w[8]) {
-  constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kXor3 = 0x1B;  // quad_perm [1,0,3,2], [2,3,0,1], [3,2,1,0]
-  const uint32_t m = dpp<0x141>(v);                        // row_half_mirror: lane ^ 7
-  w[0] = v;
-  w[1] = dpp<kXor1>(v);
-  w[2] = dpp<kXor2>(v);
-  w[3] = dpp<kXor3>(v);
-  w[4] = dpp<kXor3>(m);
-  w[5] = dpp<kXor2>(m);
-  w[6] = dpp<kXor1>(m);
-  w[7] = m;
-}
-
-// This lane's row of a jump matrix (entries in the order of gather_xor).
-struct JumpRow {
-  int32_t c[8];
-};
-
-__device__ __forceinline__ JumpRow load_row(const int32_t* p) {  // p: the matrix + 4 * row
-  const u4_t a = *reinterpret_cast<const u4_t*>(p), b = *reinterpret_cast<const u4_t*>(p + 32);
-  return JumpRow{{(int32_t)a.x, (int32_t)a.y, (int32_t)a.z, (int32_t)a.w, (int32_t)b.x, (int32_t)b.y, (int32_t)b.z,
-                  (int32_t)b.w}};
-}
-
-// The next centred word from a row's sum (see jump_matrix_entries).
-__device__ __forceinline__ int32_t reduce_centred(uint64_t v) {
-  const uint64_t f = fold_hi((uint32_t)(v >> 32), (uint32_t)v);
-  return (int32_t)(((uint32_t)f & kP) + (uint32_t)(f >> 31) - kCenter);
-}
-
-// One product: this lane's centred word of (matrix) x (state), the state's
-// words being the centred e of the group's lanes.
-__device__ __forceinline__ int32_t jump_row(const JumpRow& m, int32_t e) {
-  uint32_t w[8];
-  gather_xor((uint32_t)e, w);
-  uint64_t v = kJumpBase;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) v += (uint64_t)((int64_t)m.c[k] * (int64_t)(int32_t)w[k]);
-  return reduce_centred(v);
-}
-
-__device__ __forceinline__ int32_t centre_word(uint32_t s) { return (int32_t)(s >= kCenter ? s - kP : s); }
-__device__ __forceinline__ uint32_t word_of(int32_t e) { return (uint32_t)(e > 0 ? e : e + (int32_t)kP); }  // in [1, p]
-
 __device__ __forceinline__ const int32_t* position_table(const AdvanceArgs& a, int k) {
   return k < kJumpPositions ? a.digits + k * kPositionInts : a.digits_wide + (k - kJumpPositions) * kPositionInts;
 }
 
-__device__ __forceinline__ uint32_t digit_of(uint32_t half, int k) { return (half >> (8 * (k & 3))) & 0xffu; }
-
-// The jump of a state that has a zero word (this lane's word s): bigDotProd
-// is 0 exactly where every product of a row is.  A state without one never
-// gets one (no row of a power of A is zero), so only waves that start with
-// such a state come here.
+// The jump of a state that has a zero word (see jump_zero_words).
 __device__ __forceinline__ uint32_t advance_zero_words(uint32_t s, const uint32_t* off, const AdvanceArgs& a) {
-  const int row = threadIdx.x & 7;
   for (int k = 0; k < 8 * (int)a.words; ++k) {
     const uint32_t d = digit_of(off[k / 4], k);
-    if (!__ballot(d != 0u)) continue;
-    const JumpRow m = load_row(position_table(a, k) + d * kJumpMatrixInts + 4 * row);
-    uint32_t w[8];
-    gather_xor(s, w);
-    bool any = false;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) any = any || (m.c[q] != 0 && w[q] != 0u);
-    const uint32_t y = word_of(jump_row(m, centre_word(s)));
-    s = any ? y : 0u;
+    if (__ballot(d != 0u)) s = jump_zero_words(s, d, position_table(a, k));
   }
   return s;
 }
@@ -781,19 +703,6 @@ __device__ __forceinline__ uint32_t advance_zero_words(uint32_t s, const uint32_
 // 256 bits: 5.5 and 8.1 us).  Positions where
 // no state of the wave has a digit are skipped.  A state is read before it is
 // written, so `in` and `out` may be the same buffer.
-__device__ __forceinline__ void load_rows4(JumpRow m[4], const AdvanceArgs& a, int half, uint32_t d, int row) {
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-    m[b] = load_row(position_table(a, 4 * half + b) + digit_of(d, b) * kJumpMatrixInts + 4 * row);
-}
-
-__device__ __forceinline__ int32_t apply_rows4(const JumpRow m[4], uint32_t d, int32_t e) {
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-    if (__ballot(digit_of(d, b) != 0u)) e = jump_row(m[b], e);
-  return e;
-}
-
 __global__ __launch_bounds__(256) void k_advance(AdvanceArgs a) {
   const int row = threadIdx.x & 7;
   const uint64_t item = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3;
@@ -807,15 +716,15 @@ __global__ __launch_bounds__(256) void k_advance(AdvanceArgs a) {
     int32_t e = centre_word(s);
     JumpRow m0[4], m1[4];
     uint32_t d0 = off[0], d1 = off[1];
-    load_rows4(m0, a, 0, d0, row);
+    load_rows4(m0, position_table(a, 0), d0);
     for (uint32_t w = 0; w < a.words; ++w) {
-      load_rows4(m1, a, 2 * w + 1, d1, row);
+      load_rows4(m1, position_table(a, 8 * w + 4), d1);
       e = apply_rows4(m0, d0, e);
       const uint32_t da = d1;
       if (w + 1 < a.words) {
         d0 = off[2 * w + 2];
         d1 = off[2 * w + 3];
-        load_rows4(m0, a, 2 * w + 2, d0, row);
+        load_rows4(m0, position_table(a, 8 * w + 8), d0);
       }
       e = apply_rows4(m1, da, e);
     }
@@ -1111,12 +1020,10 @@ __device__ __forceinline__ void mfma_tiles(const MfmaFillArgs& a, uint64_t t0, u
   // column n are the tile's outputs 128 n - 8 + q, from the tile state
   long B;
   {
+    const uint32_t word = jump_group(own_word(a.start.state), a.start.offset + a.head + t0 * kTile, a.digits);
     uint32_t s[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s[j] = a.start.state[j];
-    jump_groups(s, a.start.offset + a.head + t0 * kTile, a.jump);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s[j] = __builtin_amdgcn_readfirstlane(s[j]);
+    for (int j = 0; j < 8; ++j) s[j] = __builtin_amdgcn_readlane(word, j);
     Coef k2[2];
     const CoefRecord* fan = a.mfma_fan + (n ? n - 1 : 0) * 8 + wg;  // outputs COL n - 8 + q
     k2[0] = load_coef(fan);
@@ -1208,7 +1115,7 @@ template <int FMT, int COL, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void k_fill_mfma(MfmaFillArgs a) {
   __shared__ uint32_t stage[WAVES][kMfmaColumns * (COL + 4)];
   const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint64_t w = (uint64_t)blockIdx.x * WAVES + wib;
+  const uint64_t w = xcd_block(blockIdx.x, gridDim.x, a.xcds, a.xcd_group) * WAVES + wib;
   if (w < a.waves) {
     const uint64_t t0 = w * a.tiles_per_wave;
     mfma_tiles<FMT, COL>(a, t0, (uint32_t)min((uint64_t)a.tiles_per_wave, a.tiles - t0), stage[wib]);
@@ -1217,12 +1124,10 @@ __global__ __launch_bounds__(64 * WAVES) void k_fill_mfma(MfmaFillArgs a) {
   const uint64_t e = w - a.waves;
   if (e >= a.extra) return;
   const uint64_t first = a.extra_first[e], cnt = a.extra_count[e];
+  const uint32_t word = jump_group(own_word(a.start.state), a.start.offset + first, a.digits);
   uint32_t s[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) s[j] = a.start.state[j];
-  jump_groups(s, a.start.offset + first, a.jump);
-#pragma unroll
-  for (int j = 0; j < 8; ++j) s[j] = __builtin_amdgcn_readfirstlane(s[j]);
+  for (int j = 0; j < 8; ++j) s[j] = __builtin_amdgcn_readlane(word, j);
   Coef k[4];
   load_lane_coefs<FMT, 4>(k, a.lane);
   generate_run<FMT, 4>(static_cast<typename Out<FMT>::T*>(a.out) + first, cnt, s, k, a.lane);

@@ -16,8 +16,6 @@ constexpr int kLaneRows = 256;   // block rows kept on the device: up to 4 outpu
 constexpr int kJumpBits = 8;
 constexpr int kJumpPositions = 64 / kJumpBits;
 constexpr int kJumpValues = (1 << kJumpBits) - 1;  // non-zero digit values
-// Record index of row 0 of the identity, stored after the digit matrices.
-constexpr int kIdentityRec = kJumpPositions * kJumpValues * 8;
 // Bulk advances take offsets of up to kAdvanceWords 64-bit words; byte
 // positions kJumpPositions .. kWidePositions-1 live in a second table built
 // on first use.
@@ -34,12 +32,8 @@ constexpr uint64_t kMaxTile = 1ull << 40;
 // Per-device constant tables.
 struct DeviceTables {
   CoefRecord* lane = nullptr;  // kLaneRows records: row 0 of A^(k+1), support 0xff
-  // kJumpPositions * kJumpValues * 8 records: row r of A^(d 2^(kJumpBits k))
-  // at ((k * kJumpValues) + (d - 1)) * 8 + r; then the 8 rows of the
-  // identity at kIdentityRec + r
-  CoefRecord* jump = nullptr;
-  // Jump matrices of the bulk advance: A^(d 2^(kJumpBits k)) at
-  // k kPositionInts + d kJumpMatrixInts, positions 0..kJumpPositions-1
+  // Jump matrices: A^(d 2^(kJumpBits k)) at k kPositionInts + d
+  // kJumpMatrixInts, byte positions k = 0..kJumpPositions-1
   const int32_t* digits = nullptr;
   // the same for positions kJumpPositions..kWidePositions-1; null until the
   // first bulk advance with offsets wider than 64 bits
@@ -88,7 +82,7 @@ struct FillArgs {
   uint64_t head;            // outputs before the first 1 KiB boundary of out
   StreamStart start;        // the state, and the position (offset) of out[0]
   const CoefRecord* lane;
-  const CoefRecord* jump;
+  const int32_t* digits;    // jump matrices (DeviceTables::digits)
   uint32_t xcds;            // XCDs that blocks are dealt to in turn (block b runs on XCD b mod xcds)
   uint32_t xcd_group;       // consecutive blocks of output per XCD run (1: blocks in dispatch order)
 };
@@ -113,12 +107,14 @@ struct MfmaFillArgs {
   uint64_t extra_count[2];
   StreamStart start;
   const CoefRecord* lane;
-  const CoefRecord* jump;
+  const int32_t* digits;    // jump matrices (DeviceTables::digits)
   const uint32_t* mfma_a;
   const int32_t* mfma_c;
   const CoefRecord* mfma_fan;   // this column length's tables
   const uint32_t* mfma_next_a;  // kMfmaClasses x 64 x 2 words
   const uint32_t* mfma_next_k;  // 4 x 2
+  uint32_t xcds;                // as in FillArgs
+  uint32_t xcd_group;
 };
 
 // Waves of a fill of n >= 1 outputs.
@@ -209,7 +205,7 @@ struct BatchArgs {
   uint64_t tile;               // outputs per tile
   const uint32_t* states;      // resident per-stream states (8 words each), may be null
   const CoefRecord* lane;
-  const CoefRecord* jump;
+  const int32_t* digits;    // jump matrices (DeviceTables::digits)
   uint32_t xcds;               // as in FillArgs
   uint32_t xcd_group;
 };

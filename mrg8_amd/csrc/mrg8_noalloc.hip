@@ -91,11 +91,11 @@ extern "C" int mrg8_batch_generate_noalloc(int device, const mrg8_stream_desc* d
   a.tile = c.tile_outputs;
   a.states = nullptr;
   a.lane = ctx->tables.lane;
-  a.jump = ctx->tables.jump;
+  a.digits = ctx->tables.digits;
   a.xcds = (uint32_t)ctx->num_xcc;
-  a.xcd_group = xcd_run_blocks(*ctx, c.block_threads);
+  a.xcd_group = xcd_run_blocks(*ctx, c.blocks_per_cu ? c.block_threads : tile_block_threads(c.block_threads));
   // the staging copy above wrote the header's work counters as zero
-  e = c.blocks_per_cu == 0  ? launch_batch_tiles(a, nt, c.block_threads, s)
+  e = c.blocks_per_cu == 0  ? launch_batch_tiles(a, nt, tile_block_threads(c.block_threads), s)
       : c.blocks_per_cu < 0 ? launch_batch_queue(a, ctx->num_cu * -c.blocks_per_cu, c.block_threads, s)
                             : launch_batch(a, ctx->num_cu * c.blocks_per_cu, c.block_threads, s);
   if (e != hipSuccess) return hip_fail(e, "batch launch (no-alloc)");

@@ -114,14 +114,14 @@ BatchArgs BatchSlot::args(const LaunchConfig& cfg) const {
   a.tile = cfg.tile;
   a.states = states_;
   a.lane = ctx_->tables.lane;
-  a.jump = ctx_->tables.jump;
+  a.digits = ctx_->tables.digits;
   a.xcds = (uint32_t)ctx_->num_xcc;
-  a.xcd_group = xcd_run_blocks(*ctx_, cfg.block_threads);
+  a.xcd_group = xcd_run_blocks(*ctx_, cfg.blocks_per_cu ? cfg.block_threads : tile_block_threads(cfg.block_threads));
   return a;
 }
 
 hipError_t BatchSlot::launch(const LaunchConfig& cfg, hipStream_t stream) const {
-  if (cfg.blocks_per_cu == 0) return launch_batch_tiles(args(cfg), ntiles_, cfg.block_threads, stream);
+  if (cfg.blocks_per_cu == 0) return launch_batch_tiles(args(cfg), ntiles_, tile_block_threads(cfg.block_threads), stream);
   if (cfg.blocks_per_cu < 0)
     return launch_batch_queue(args(cfg), ctx_->num_cu * -cfg.blocks_per_cu, cfg.block_threads, stream);
   return launch_batch(args(cfg), ctx_->num_cu * cfg.blocks_per_cu, cfg.block_threads, stream);
