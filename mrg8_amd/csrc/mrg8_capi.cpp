@@ -301,19 +301,23 @@ int fill_mfma(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, void
   a.tiles = tiles;
   a.column = (uint32_t)column;
   a.waves_per_block = (uint32_t)(block_threads ? block_threads / 64 : format == MRG8_U32 ? 4 : 16);
-  // default: 32 KiB of output per wave for doubles and 16 KiB for words, fewer
-  // tiles when that would leave fewer than 8 waves per CU
-  const uint64_t bytes_per_wave = format == MRG8_U32 ? 16384 : 32768;
-  const uint64_t per = outputs_per_wave
-                           ? outputs_per_wave / tile
-                           : std::min<uint64_t>(bytes_per_wave / (uint64_t)esz / tile, tiles / ((uint64_t)ctx.num_cu * 8));
+  // default: 32 KiB of output per wave for doubles, fewer tiles when that
+  // would leave fewer than 8 waves per CU; for words 16 KiB (two tiles of
+  // 2048) from 32 waves per CU on, one tile below
+  const bool long_words = format == MRG8_U32 && tiles >= (uint64_t)ctx.num_cu * 64;
+  uint64_t per = format == MRG8_U32
+                     ? (long_words ? 16384 / (uint64_t)esz / tile : 1)
+                     : std::min<uint64_t>(32768 / (uint64_t)esz / tile, tiles / ((uint64_t)ctx.num_cu * 8));
+  if (outputs_per_wave) per = outputs_per_wave / tile;
   a.tiles_per_wave = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(per, 1), 1u << 20);
   a.waves = (tiles + a.tiles_per_wave - 1) / a.tiles_per_wave;
-  // blocks of four waves in XCD runs of 16 (1 MiB of words at the default
-  // run): 2^28 words 174-177 us; in dispatch order 190 us, 512-thread blocks
-  // of 8192 words per wave 179-181 us either way
+  // Blocks of four waves, in XCD runs of 16 (1 MiB of words) from 32 waves per
+  // CU on.  2^28 words: 171 us, in dispatch order 206 us, with one tile per
+  // wave 206 us, 512-thread blocks of 8192 words per wave 180 us; 2^26: 48.2
+  // us, 512-thread blocks the same; 2^24 with one tile per wave 14.9 us, two
+  // tiles 15.3 us.
   a.xcds = (uint32_t)ctx.num_xcc;
-  a.xcd_group = a.waves_per_block == 4 && a.waves >= (uint64_t)ctx.num_cu * 16 ? 16 : 1;
+  a.xcd_group = a.waves_per_block == 4 && a.waves >= (uint64_t)ctx.num_cu * 32 ? 16 : 1;
   const uint64_t tail_first = head + tiles * tile;
   if (head) {
     a.extra_first[a.extra] = 0;

@@ -934,8 +934,8 @@ __global__ __launch_bounds__(256) void k_stage(const u4_t* __restrict__ src, u4_
 //     carry the 2^30 sum R_j, the reference's -1 and the biases, so that
 //     t = C_0 + 2^8 C_1 and u = C_2 + 2^8 C_3 are non-negative and below
 //     2^29, and x = t + ((u << 16) & p) + (u >> 15) (2^16 u mod p is a 31-bit
-//     rotation) is the residue plus at most one p: eight 32-bit operations
-//     per output.
+//     rotation) is the residue plus at most one p: five 32-bit operations
+//     per output (mfma_step_residue).  2^28 words: 171 us, 176 us with eight.
 // MFMA layouts (gfx950; the fill's parity tests depend on them): lane
 // l = n + 16 g holds the 8 bytes of K-group g for row/column n, and result
 // register i of lane l is row 4 g + i of column n.  K-group g, byte i is word W(g) + i / 4, digit
@@ -971,12 +971,18 @@ __device__ __forceinline__ uint64_t mad_u64_u32(uint32_t a, uint32_t b, uint64_t
   return w;
 }
 
-// Residue in [0, p) of a step output (result register i of the four
-// classes, accumulators started from the step constants).
+// Residue in [0, p) of a step output (result register i of the four classes,
+// accumulators started from the step constants, class 2 taken twice): with
+// u = C_2 + 2^8 C_3, acc[2] + 2^9 acc[3] is 2 u, whose 16-bit halves are
+// 2 (u mod 2^15) and u >> 15, so one two-term dot product with (2^15, 1) adds
+// 2^16 u mod p, the 31-bit rotation of u, to t.  Five operations an output
+// (eight with the rotation from shifts and a mask).
+typedef unsigned short us2_t __attribute__((ext_vector_type(2)));
+
 __device__ __forceinline__ uint32_t mfma_step_residue(const v4i_t (&acc)[kMfmaClasses], int i) {
-  const uint32_t t = (uint32_t)acc[0][i] + ((uint32_t)acc[1][i] << 8);  // [0, 2 beta + 2^16)
-  const uint32_t u = (uint32_t)acc[2][i] + ((uint32_t)acc[3][i] << 8);  // [0, 2 beta + 2^15)
-  const uint32_t x = t + ((u << 16) & kP) + (u >> 15);                  // < 2 p
+  const uint32_t t = (uint32_t)acc[0][i] + ((uint32_t)acc[1][i] << 8);   // [0, 2 beta + 2^16)
+  const uint32_t u2 = (uint32_t)acc[2][i] + ((uint32_t)acc[3][i] << 9);  // 2 u, u in [0, 2 beta + 2^15)
+  const uint32_t x = __builtin_amdgcn_udot2(__builtin_bit_cast(us2_t, u2), us2_t{1u << 15, 1}, t, false);  // < 2 p
   return min(x, x - kP);
 }
 
@@ -1009,6 +1015,7 @@ __device__ __forceinline__ void mfma_tiles(const MfmaFillArgs& a, uint64_t t0, u
     A[q] = reinterpret_cast<const long*>(a.mfma_a)[q * 64 + lane];
     C0[q] = reinterpret_cast<const v4i_t*>(a.mfma_c)[q * 4 + g];
   }
+  C0[2] *= 2;
   long AJ[kMfmaClasses] = {};
   u2_t KJ = {};
   if (nt > 1) {
@@ -1068,6 +1075,7 @@ __device__ __forceinline__ void mfma_tiles(const MfmaFillArgs& a, uint64_t t0, u
       v4i_t acc[kMfmaClasses];
 #pragma unroll
       for (int q = 0; q < kMfmaClasses; ++q) acc[q] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A[q], B, C0[q], 0, 0, 0);
+      acc[2] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A[2], B, acc[2], 0, 0, 0);  // twice class 2: see mfma_step_residue
       uint32_t r[4];
 #pragma unroll
       for (int i = 3; i >= 0; --i) r[i] = mfma_step_residue(acc, i);  // registers 2, 3 first: the next operand
