@@ -21,13 +21,24 @@ from .capi import F64, F64_01, U32, Mrg8Error  # noqa: F401
 P = 2147483647
 
 
+_State = ctypes.c_uint32 * 8
+
+
 def _u32x8(state) -> "ctypes.Array":
+    # the common forms without numpy's conversions and reductions (a torch.ops.mrg8.fill_ call 23 -> 19 us)
+    kind = type(state)
+    if kind is np.ndarray:
+        if state.dtype == np.uint32 and state.shape == (8,):
+            return _State.from_buffer_copy(state.tobytes())
+    elif (kind is list or kind is tuple) and len(state) == 8 and all(
+            type(x) is int and 0 <= x <= 0xFFFFFFFF for x in state):
+        return _State(*state)
     a = np.asarray(state, dtype=np.int64)
     if a.shape != (8,):
         raise ValueError("state must have 8 words")
     if (a < 0).any() or (a > 0xFFFFFFFF).any():
         raise ValueError("state words must be 32-bit unsigned")
-    return (ctypes.c_uint32 * 8)(*[int(x) for x in a])
+    return _State(*[int(x) for x in a])
 
 
 def _bits200(bits) -> "ctypes.Array":
@@ -40,8 +51,9 @@ def _bits200(bits) -> "ctypes.Array":
 
 
 def _ptr(p) -> int:
-    if hasattr(p, "data_ptr"):
-        return int(p.data_ptr())  # torch tensor
+    data_ptr = getattr(p, "data_ptr", None)
+    if data_ptr is not None:
+        return data_ptr()  # torch tensor
     if hasattr(p, "ptr"):
         return int(p.ptr)  # mrg8_amd.hip.DeviceBuffer
     return int(p)
@@ -50,11 +62,12 @@ def _ptr(p) -> int:
 def _stream(s):
     if s is None:
         return None
-    if hasattr(s, "cuda_stream"):
-        return ctypes.c_void_p(int(s.cuda_stream))  # torch.cuda.Stream
+    stream = getattr(s, "cuda_stream", None)
+    if stream is not None:
+        return stream  # torch.cuda.Stream
     if hasattr(s, "handle"):
         return ctypes.c_void_p(s.handle)
-    return ctypes.c_void_p(int(s))
+    return int(s)
 
 
 class mrg8_cuda:
@@ -117,21 +130,20 @@ class mrg8_cuda:
         multiple of the tile).  Automatic: the matrix-core fill for word fills
         of 2^22 outputs or more, the vector kernel otherwise."""
         if block_threads or tile or per_lane:
-            capi.call("mrg8_generate_shape", self._h, ctypes.c_void_p(_ptr(dptr)), ctypes.c_uint64(n), fmt,
-                      _stream(stream), block_threads, ctypes.c_uint64(tile), per_lane)
+            capi.call("mrg8_generate_shape", self._h, _ptr(dptr), ctypes.c_uint64(n), fmt, _stream(stream), block_threads,
+                      ctypes.c_uint64(tile), per_lane)
         else:
-            capi.call("mrg8_generate", self._h, ctypes.c_void_p(_ptr(dptr)), ctypes.c_uint64(n), fmt,
-                      _stream(stream))
+            capi.call("mrg8_generate", self._h, _ptr(dptr), ctypes.c_uint64(n), fmt, _stream(stream))
 
     def mrg8_outer_32(self, d_ran, n: int, BS: int = 0, TNUM: int = 0) -> None:
         """cuda/mrg8_cuda.cu:414-436: blocking, [0,1) doubles.  TNUM = 0 (the
         default) takes the library's own launch shape; BS = 0 means 64, the
         reference's threads per block when only TNUM is given."""
-        capi.call("mrg8_outer_32", self._h, ctypes.c_void_p(_ptr(d_ran)), n, BS, TNUM)
+        capi.call("mrg8_outer_32", self._h, _ptr(d_ran), n, BS, TNUM)
 
     def mrg8_inner(self, d_ran, n: int, TNUM: int = 64 * 1024) -> None:
         """cuda/mrg8_cuda.cu:402-412: blocking, [0,1) doubles."""
-        capi.call("mrg8_inner", self._h, ctypes.c_void_p(_ptr(d_ran)), n, TNUM)
+        capi.call("mrg8_inner", self._h, _ptr(d_ran), n, TNUM)
 
     def state_cpy_DtH(self) -> None:
         capi.call("mrg8_state_cpy_DtH", self._h)
@@ -224,8 +236,8 @@ def advance_states(d_in, d_offsets, words: int, d_out, n: int, stream=None, devi
     """Device-side bulk jump: n states (8 uint32 words each, device memory)
     advanced by little-endian offsets of `words` uint64 words each (up to 256
     bits); stream-ordered.  See mrg8_advance_states in include/mrg8.h."""
-    capi.call("mrg8_advance_states", device, ctypes.c_void_p(_ptr(d_in)), ctypes.c_void_p(_ptr(d_offsets)),
-              ctypes.c_uint32(words), ctypes.c_void_p(_ptr(d_out)), ctypes.c_uint64(n), _stream(stream))
+    capi.call("mrg8_advance_states", device, _ptr(d_in), _ptr(d_offsets), ctypes.c_uint32(words), _ptr(d_out),
+              ctypes.c_uint64(n), _stream(stream))
 
 
 class Batch:

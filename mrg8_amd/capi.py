@@ -157,8 +157,14 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_functions: dict = {}
+
+
 def call(name: str, *args) -> int:
-    rc = getattr(lib(), name)(*args)
+    f = _functions.get(name)
+    if f is None:
+        f = _functions[name] = getattr(lib(), name)
+    rc = f(*args)
     if rc != OK:
         msg = lib().mrg8_last_error()
         raise Mrg8Error(rc, name, msg.decode() if msg else lib().mrg8_strerror(rc).decode())

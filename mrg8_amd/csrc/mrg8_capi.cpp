@@ -49,6 +49,11 @@ const JumpTable& host_jump_table() {
   return t;
 }
 
+const DigitTable& host_digit_table() {
+  static const DigitTable t(host_jump_table());
+  return t;
+}
+
 // ---- per-device state ------------------------------------------------------------
 
 namespace {
@@ -61,16 +66,21 @@ std::vector<std::unique_ptr<DeviceContext>> g_devices;
 bool build_digits(int first, int end, int32_t* out) {
   const JumpTable& jt = host_jump_table();
   for (int k = first; k < end; ++k) {
-    const int j = kJumpBits * k;
-    std::vector<uint32_t> m(jt.at(std::min(j, kNumJump - 1)), jt.at(std::min(j, kNumJump - 1)) + 64);
-    for (int q = kNumJump - 1; q < j; ++q) m = mat_mul(m.data(), m.data());
-    std::vector<uint32_t> p(64, 0);
-    for (int r = 0; r < 8; ++r) p[(size_t)r * 9] = 1;  // the identity: a digit 0 leaves the state as it is
-    for (int d = 0; d <= kJumpValues; ++d) {
-      if (d > 0) p = d > 1 ? mat_mul(p.data(), m.data()) : m;
-      if (!jump_matrix_entries(p.data(), out + (size_t)(k - first) * kPositionInts + (size_t)d * kJumpMatrixInts))
-        return false;
+    int32_t* const at = out + (size_t)(k - first) * kPositionInts;
+    std::vector<uint32_t> m(64, 0), p;
+    for (int r = 0; r < 8; ++r) m[(size_t)r * 9] = 1;  // the identity: a digit 0 leaves the state as it is
+    bool ok = jump_matrix_entries(m.data(), at);
+    if (k >= kJumpPositions) {
+      const int j = kJumpBits * k;
+      m.assign(jt.at(std::min(j, kNumJump - 1)), jt.at(std::min(j, kNumJump - 1)) + 64);
+      for (int q = kNumJump - 1; q < j; ++q) m = mat_mul(m.data(), m.data());
     }
+    for (int d = 1; d <= kJumpValues && ok; ++d) {
+      if (k >= kJumpPositions) p = d > 1 ? mat_mul(p.data(), m.data()) : m;
+      ok = jump_matrix_entries(k < kJumpPositions ? host_digit_table().at(k, d) : p.data(),
+                               at + (size_t)d * kJumpMatrixInts);
+    }
+    if (!ok) return false;
   }
   return true;
 }
@@ -548,7 +558,7 @@ extern "C" int mrg8_set_state(mrg8_gen_t g, const uint32_t state[8]) {
 extern "C" int mrg8_jump_ahead(mrg8_gen_t g, uint64_t step) {
   clear_error();
   if (!g) return fail(MRG8_ERR_ARG, "null generator");
-  jump64(host_jump_table(), step, g->state);
+  jump64(host_digit_table(), step, g->state);
   return MRG8_OK;
 }
 
@@ -564,7 +574,7 @@ extern "C" int mrg8_jump_state(mrg8_gen_t g, uint64_t step, uint32_t new_state[8
   if (!g || !new_state) return fail(MRG8_ERR_ARG, "null argument");
   uint32_t st[8];
   std::memcpy(st, g->state, sizeof st);
-  jump64(host_jump_table(), step, st);
+  jump64(host_digit_table(), step, st);
   std::memcpy(new_state, st, sizeof st);
   return MRG8_OK;
 }
@@ -592,7 +602,7 @@ extern "C" int mrg8_advance_state(const uint32_t state[8], uint64_t step, uint32
   if (!state_valid(state)) return fail(MRG8_ERR_ARG, "state words must be at most 2^31 - 1");
   uint32_t st[8];
   std::memcpy(st, state, sizeof st);
-  jump64(host_jump_table(), step, st);
+  jump64(host_digit_table(), step, st);
   std::memcpy(new_state, st, sizeof st);
   return MRG8_OK;
 }
@@ -622,7 +632,7 @@ static int generate_impl(mrg8_gen_t g, void* dptr, uint64_t n, int format, void*
   int rc = fill_device(*g->ctx, g->state, 0, dptr, n, format, s, block_threads, tile, per_lane);
   if (rc) return rc;
   if (std::find(g->streams.begin(), g->streams.end(), s) == g->streams.end()) g->streams.push_back(s);
-  jump64(host_jump_table(), n, g->state);  // the state after n outputs
+  jump64(host_digit_table(), n, g->state);  // the state after n outputs
   return MRG8_OK;
 }
 
@@ -749,7 +759,7 @@ static int host_fill(mrg8_gen_t g, void* host, uint64_t n, int format) {
     const uint64_t m = count(i);
     int rc = fill_device(*g->ctx, g->state, 0, g->pin_chunk[b], m, format, g->host_stream, 0, 0, 0);
     if (rc) return rc;
-    jump64(host_jump_table(), m, g->state);
+    jump64(host_digit_table(), m, g->state);
     hipError_t x = hipEventRecord(g->chunk_ready[b], g->host_stream);
     return x == hipSuccess ? MRG8_OK : hip_fail(x, "hipEventRecord(chunk)");
   };

@@ -54,6 +54,7 @@ int hip_fail(hipError_t e, const char* what);
 void clear_error();
 
 const JumpTable& host_jump_table();
+const DigitTable& host_digit_table();
 int device_context(int device, DeviceContext** out);
 // The device's context if mrg8_init_device (or any call that needs it) has
 // created it, else null; creates nothing.
