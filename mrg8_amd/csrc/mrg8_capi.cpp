@@ -128,8 +128,8 @@ int device_context(int device, DeviceContext** out) {
   // start records); a fan-out row with a zero entry would need the exact-zero
   // test, so such a table turns the matrix-core fill off.
   MfmaHostTables mt[2];
-  MfmaStrideTables mn[2];
-  bool mfma_ok = true;
+  MfmaStrideTables mn[2], skip;
+  bool mfma_ok = mfma_stride_tables(host_jump_table(), kBatchSkip, kMfmaClasses, kMfmaBeta, &skip);
   for (int i = 0; i < 2; ++i)
     mfma_ok = mfma_ok && mfma_host_tables(kMfmaColumns, kMfmaColumnLen[i], kMfmaClasses, kMfmaBeta, &mt[i]) &&
               mfma_stride_tables(host_jump_table(), (uint64_t)kMfmaColumns * kMfmaColumnLen[i], kMfmaClasses, kMfmaBeta,
@@ -148,7 +148,7 @@ int device_context(int device, DeviceContext** out) {
   void* p = nullptr;
   const size_t rec_bytes = sizeof(CoefRecord) * lane.size();
   // operand digits and accumulator start values do not depend on the column length
-  size_t mfma_bytes = sizeof(uint32_t) * (mt[0].a.size() + mt[0].c.size());
+  size_t mfma_bytes = sizeof(uint32_t) * (mt[0].a.size() + mt[0].c.size() + skip.a.size() + skip.k.size());
   for (int i = 0; i < 2; ++i)
     mfma_bytes += sizeof(CoefRecord) * mt[i].fan.size() + sizeof(uint32_t) * (mn[i].a.size() + mn[i].k.size());
   if (!mfma_ok) mfma_bytes = 0;
@@ -185,6 +185,8 @@ int device_context(int device, DeviceContext** out) {
       ctx->tables.mfma_next_k[i] =
           reinterpret_cast<const uint32_t*>(put(mn[i].k.data(), sizeof(uint32_t) * mn[i].k.size()));
     }
+    ctx->tables.mfma_skip_a = reinterpret_cast<const uint32_t*>(put(skip.a.data(), sizeof(uint32_t) * skip.a.size()));
+    ctx->tables.mfma_skip_k = reinterpret_cast<const uint32_t*>(put(skip.k.data(), sizeof(uint32_t) * skip.k.size()));
   }
   if (e != hipSuccess) {
     (void)hipFree(p);

@@ -986,6 +986,15 @@ __device__ __forceinline__ uint32_t mfma_step_residue(const v4i_t (&acc)[kMfmaCl
   return min(x, x - kP);
 }
 
+// The products of a step: class 2 twice (see mfma_step_residue); C0 holds the
+// step constants with class 2's doubled.
+__device__ __forceinline__ void mfma_step(v4i_t (&acc)[kMfmaClasses], const long (&A)[kMfmaClasses],
+                                          const v4i_t (&C0)[kMfmaClasses], long B) {
+#pragma unroll
+  for (int q = 0; q < kMfmaClasses; ++q) acc[q] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A[q], B, C0[q], 0, 0, 0);
+  acc[2] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A[2], B, acc[2], 0, 0, 0);
+}
+
 // Residue in [0, p) of a stride output (accumulators started from 0, k in
 // [kMfmaBeta, kMfmaBeta + p)).
 __device__ __forceinline__ uint32_t mfma_stride_residue(const v4i_t (&acc)[kMfmaClasses], int i, uint32_t k) {
@@ -1073,9 +1082,7 @@ __device__ __forceinline__ void mfma_tiles(const MfmaFillArgs& a, uint64_t t0, u
 #pragma unroll
     for (int step = 0; step < kSteps; ++step) {
       v4i_t acc[kMfmaClasses];
-#pragma unroll
-      for (int q = 0; q < kMfmaClasses; ++q) acc[q] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A[q], B, C0[q], 0, 0, 0);
-      acc[2] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A[2], B, acc[2], 0, 0, 0);  // twice class 2: see mfma_step_residue
+      mfma_step(acc, A, C0, B);
       uint32_t r[4];
 #pragma unroll
       for (int i = 3; i >= 0; --i) r[i] = mfma_step_residue(acc, i);  // registers 2, 3 first: the next operand
@@ -1139,6 +1146,191 @@ __global__ __launch_bounds__(64 * WAVES) void k_fill_mfma(MfmaFillArgs a) {
   Coef k[4];
   load_lane_coefs<FMT, 4>(k, a.lane);
   generate_run<FMT, 4>(static_cast<typename Out<FMT>::T*>(a.out) + first, cnt, s, k, a.lane);
+}
+
+// Persistent batched kernel for short tiles: a wave takes eight tiles at once,
+// eight lanes looking up and jumping each, and generates them together with
+// the matrix cores in sixteen columns: 256 outputs of every tile a run, the
+// two halves from the tile's state and from A^128 times it, 16 outputs of
+// every column a step (see the matrix-core fill).  A run goes through LDS and
+// leaves tile by tile.  In the vector kernel a short tile is mostly start:
+// eight lane broadcasts and two chains of eight multiply-adds, one tile after
+// the other, and nothing left to store when the next jumps wait for memory.
+// Here the next group is looked up before the current one's steps and jumped
+// before its stores (loads wait for all earlier stores), and what is left is
+// bound by the issue of the jumps' 64-bit multiply-adds and the residues.
+// Not kept: sixteen tiles in columns of their own with four lanes jumping each
+// (65536 x 256 words 20.8 us, but 2048 x 256 13.3 and 32768 x 512 30); halves
+// of fewer than 128 outputs where a tile needs no more (the rows then wait for
+// the lookup: 131072 x 256 words 42.7 against 40.4).
+// Which batches take it: see batch_kernel.
+constexpr uint32_t kShortGroup = 8;
+constexpr int kShortRun = kBatchSkip, kShortStride = kShortRun + 4;  // outputs of a column in a run, its LDS words
+
+// A run of a tile of cnt outputs from its output `done` on, the tile's two
+// columns at `col` and 8 columns on: four outputs a lane.
+struct RunWords {
+  uint32_t w[4];
+};
+
+template <int FMT>
+__device__ __forceinline__ uint32_t run_output(int i) {  // first output of this lane's pair i (of 2)
+  return FMT == 2 ? 4 * threadIdx.x + 2 * i : kShortRun * i + 2 * threadIdx.x;
+}
+
+template <int FMT>
+__device__ __forceinline__ RunWords read_run(const uint32_t* col) {
+  if constexpr (FMT == 2) {  // four consecutive outputs
+    const u4_t v = *reinterpret_cast<const u4_t*>(col + (threadIdx.x >> 5) * (8 * kShortStride) + 4 * (threadIdx.x & 31));
+    return RunWords{{v.x, v.y, v.z, v.w}};
+  } else {  // two of each half, so that each store of the wave is contiguous
+    const u2_t a = *reinterpret_cast<const u2_t*>(col + 2 * threadIdx.x);
+    const u2_t b = *reinterpret_cast<const u2_t*>(col + 8 * kShortStride + 2 * threadIdx.x);
+    return RunWords{{a.x, a.y, b.x, b.y}};
+  }
+}
+
+template <int FMT>
+__device__ __forceinline__ void store_run(void* out, uint64_t done, uint64_t cnt, const RunWords& r, bool zero) {
+  typedef typename Out<FMT>::T T;
+  typedef T pair_t __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+  typedef T quad_t __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  T v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = zero ? convert_zero<FMT>() : convert<FMT>(r.w[i]);
+  T* const p = static_cast<T*>(out) + done;
+  const uint64_t left = cnt - done;
+  if (FMT == 2 && run_output<FMT>(1) + 1 < left) {
+    __builtin_nontemporal_store(quad_t{v[0], v[1], v[2], v[3]}, reinterpret_cast<quad_t*>(p + run_output<FMT>(0)));
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t o = run_output<FMT>(i);
+    if (o + 1 < left) __builtin_nontemporal_store(pair_t{v[2 * i], v[2 * i + 1]}, reinterpret_cast<pair_t*>(p + o));
+    else if (o < left) __builtin_nontemporal_store(v[2 * i], p + o);
+  }
+}
+
+// A run of every tile of a group: tiles of one format, none with the all-zero
+// state, the LDS reads first.
+template <int FMT>
+__device__ __forceinline__ void store_runs(const TileInfo& ti, uint32_t ngrp, uint64_t done, const uint32_t* stage) {
+  RunWords v[kShortGroup];
+#pragma unroll
+  for (int t = 0; t < (int)kShortGroup; ++t) v[t] = read_run<FMT>(stage + t * kShortStride);
+#pragma unroll
+  for (int t = 0; t < (int)kShortGroup; ++t) {
+    const uint64_t cnt = (uint32_t)t < ngrp ? readlane_u64(ti.cnt, 8 * t) : 0;
+    if (done < cnt) store_run<FMT>(global_pointer(readlane_u64(ti.dst, 8 * t)), done, cnt, v[t], false);
+  }
+}
+
+__global__ __launch_bounds__(64) void k_batch_short(BatchArgs a) {
+  __shared__ __attribute__((aligned(16))) uint32_t stage[kMfmaColumns * kShortStride];
+  const uint32_t lane = threadIdx.x, n = lane & 15, g = lane >> 4;
+  const uint32_t wg = (g & 1) * 4 + (g >> 1) * 2;  // W(g), as in mfma_tiles
+  const uint32_t grp = lane >> 3;
+  const BatchTables tab = batch_tables(a.block);
+  const uint64_t ntiles = tab.ntiles;
+  // equal waves of full groups, but enough of them to reach every SIMD
+  const uint64_t round = (uint64_t)kShortGroup * gridDim.x;
+  const uint64_t per_wave = kShortGroup * ((ntiles + round - 1) / round);
+  const uint64_t nwaves = min((uint64_t)gridDim.x, max((ntiles + per_wave - 1) / per_wave, (uint64_t)a.min_waves));
+  const uint64_t wave = xcd_block(blockIdx.x, gridDim.x, a.xcds, a.xcd_group);
+  if (wave >= nwaves || wave >= ntiles) return;
+  long A[kMfmaClasses];
+  v4i_t C0[kMfmaClasses];
+#pragma unroll
+  for (int q = 0; q < kMfmaClasses; ++q) {
+    A[q] = reinterpret_cast<const long*>(a.mfma_a)[q * 64 + lane];
+    C0[q] = reinterpret_cast<const v4i_t*>(a.mfma_c)[q * 4 + g];
+  }
+  const JumpRow second = load_row(a.digits + kShortRun * kJumpMatrixInts + 4 * (lane & 7));  // A^128
+  const uint64_t total = (ntiles - wave + nwaves - 1) / nwaves;
+  auto group_size = [&](uint64_t j0) { return j0 < total ? (uint32_t)min<uint64_t>(kShortGroup, total - j0) : 0u; };
+  auto lookup = [&](uint64_t j0) { return lookup_tile(tab, a, (j0 + (grp < group_size(j0) ? grp : 0)) * nwaves + wave); };
+  uint32_t ngrp = group_size(0);
+  TileInfo ti = lookup(0);
+  uint32_t s = jump_group(ti.state[lane & 7], grp < ngrp ? ti.offset : 0, a.digits);
+  for (uint64_t j0 = 0; ngrp != 0; j0 += kShortGroup) {
+    const bool mine = grp < ngrp;
+    const uint32_t s2 = word_of(jump_row(second, centre_word(s)));
+    const uint32_t nnext = group_size(j0 + kShortGroup);
+    TileInfo tn = ti;
+    uint32_t sn = 0;
+    if (nnext) {
+      tn = lookup(j0 + kShortGroup);
+      sn = tn.state[lane & 7];
+    }
+    const uint64_t alive = __ballot(s != 0u);  // a tile's eight bits are 0: the all-zero state
+    const int32_t fmt = __builtin_amdgcn_readfirstlane(ti.fmt);
+    const bool plain = __ballot(((alive >> (lane & 56)) & 255u) == 0 || ti.fmt != fmt) == 0;
+    uint64_t most = mine ? ti.cnt : 0;
+#pragma unroll
+    for (int d = 8; d < 64; d *= 2) most = max(most, (uint64_t)__shfl_xor((unsigned long long)most, d));
+    most = readlane_u64(most, 0);
+    // column n (tile n mod 8, half n / 8): words W(g), W(g) + 1, oldest first
+    long B;
+    {
+      const int hi = (int)(4 * (8 * (n & 7) + 7 - wg)), lo = hi - 4;
+      auto from = [](int at, uint32_t v) { return (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)v); };
+      const uint32_t h0 = from(hi, s), h1 = from(hi, s2), l0 = from(lo, s), l1 = from(lo, s2);
+      B = mfma_operand(n & 8 ? h1 : h0, n & 8 ? l1 : l0);
+    }
+    if (j0 == 0) C0[2] *= 2;  // not before the jump's loads are issued
+    uint32_t* const col = stage + n * kShortStride;
+    for (uint64_t done = 0;;) {
+      const int steps = (int)min<uint64_t>(kShortRun / 16, (most - done + 15) / 16);
+#pragma unroll
+      for (int step = 0; step < kShortRun / 16; ++step) {
+        if (step >= steps) break;
+        v4i_t acc[kMfmaClasses];
+        mfma_step(acc, A, C0, B);
+        uint32_t x[4];
+#pragma unroll
+        for (int i = 3; i >= 0; --i) x[i] = mfma_step_residue(acc, i);
+        B = mfma_operand(x[2] + 1u, x[3] + 1u);
+        *reinterpret_cast<u2_t*>(col + 16 * step + 2 * g) = u2_t{x[0], x[1]};
+        *reinterpret_cast<u2_t*>(col + 16 * step + 8 + wg) = u2_t{x[2], x[3]};
+      }
+      // the next group's jumps before this run's stores: they would wait for them
+      if (done == 0 && nnext) sn = jump_group(sn, grp < nnext ? tn.offset : 0, a.digits);
+      if (plain) {
+        switch (fmt) {
+          case 0: store_runs<0>(ti, ngrp, done, stage); break;
+          case 1: store_runs<1>(ti, ngrp, done, stage); break;
+          default: store_runs<2>(ti, ngrp, done, stage); break;
+        }
+      } else {
+        for (uint32_t t = 0; t < ngrp; ++t) {
+          const uint64_t cnt = readlane_u64(ti.cnt, 8 * t);
+          if (done >= cnt) continue;
+          void* out = global_pointer(readlane_u64(ti.dst, 8 * t));
+          const bool zero = ((alive >> (8 * t)) & 255u) == 0;
+          const uint32_t* src = stage + t * kShortStride;
+          switch (__builtin_amdgcn_readlane(ti.fmt, 8 * t)) {
+            case 0: store_run<0>(out, done, cnt, read_run<0>(src), zero); break;
+            case 1: store_run<1>(out, done, cnt, read_run<1>(src), zero); break;
+            default: store_run<2>(out, done, cnt, read_run<2>(src), zero); break;
+          }
+        }
+      }
+      done += 2 * kShortRun;
+      if (done >= most) break;
+      // every column is at its other half's end of this run: A^128 once more
+      v4i_t acc[kMfmaClasses];
+#pragma unroll
+      for (int q = 0; q < kMfmaClasses; ++q)
+        acc[q] = __builtin_amdgcn_mfma_i32_16x16x32_i8(reinterpret_cast<const long*>(a.mfma_skip_a)[q * 64 + lane], B,
+                                                       v4i_t{}, 0, 0, 0);
+      const u2_t K = reinterpret_cast<const u2_t*>(a.mfma_skip_k)[g];
+      B = mfma_operand(mfma_stride_residue(acc, 0, K.x) + 1u, mfma_stride_residue(acc, 1, K.y) + 1u);
+    }
+    ti = tn;
+    s = sn;
+    ngrp = nnext;
+  }
 }
 
 template <int FMT, int PL>
@@ -1208,6 +1400,12 @@ hipError_t launch_fill_mfma(const MfmaFillArgs& a, int format, hipStream_t strea
     case 2: return fill_mfma_column<2>(a, blocks, stream);
     default: return hipErrorInvalidValue;
   }
+}
+
+hipError_t launch_batch_short(const BatchArgs& a, uint32_t waves, hipStream_t stream) {
+  if (!a.mfma_a || waves == 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_batch_short, dim3(waves), dim3(64), 0, stream, a);
+  return hipGetLastError();
 }
 
 hipError_t launch_batch(const BatchArgs& a, int grid, int block_threads, hipStream_t stream) {

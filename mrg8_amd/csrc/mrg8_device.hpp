@@ -49,6 +49,9 @@ struct DeviceTables {
   const CoefRecord* mfma_fan[2] = {nullptr, nullptr};
   const uint32_t* mfma_next_a[2] = {nullptr, nullptr};
   const uint32_t* mfma_next_k[2] = {nullptr, nullptr};
+  // A^kBatchSkip in the same form (k_batch_short)
+  const uint32_t* mfma_skip_a = nullptr;
+  const uint32_t* mfma_skip_k = nullptr;
 };
 
 // Matrix-core fill.  A tile is kMfmaColumns columns of `column` consecutive
@@ -59,6 +62,7 @@ struct DeviceTables {
 constexpr int kMfmaColumns = 16;
 constexpr int kMfmaColumnLen[2] = {64, 128};
 constexpr int kMfmaClasses = 4;   // byte digits of a coefficient
+constexpr int kBatchSkip = 128;   // outputs of a column in a run of k_batch_short
 // Word fills of at least this many outputs take the matrix-core fill by
 // default (measured on MI355X below).
 constexpr uint64_t kMfmaDefaultMinWords = 1ull << 22;
@@ -208,6 +212,14 @@ struct BatchArgs {
   const int32_t* digits;    // jump matrices (DeviceTables::digits)
   uint32_t xcds;               // as in FillArgs
   uint32_t xcd_group;
+  // k_batch_short: the step's operand digits and accumulator start values,
+  // A^128 in the same form with its combine constants, and the waves that a
+  // launch uses at least
+  const uint32_t* mfma_a;
+  const int32_t* mfma_c;
+  const uint32_t* mfma_skip_a;
+  const uint32_t* mfma_skip_k;
+  uint32_t min_waves;
 };
 
 // A bulk advance: out[8i..8i+7] = in[8i..8i+7] jumped ahead by the
@@ -227,6 +239,8 @@ hipError_t launch_fill(const FillArgs& a, int format, int per_lane, int block_th
 // Blocks of a.waves_per_block waves.
 hipError_t launch_fill_mfma(const MfmaFillArgs& a, int format, hipStream_t stream);
 hipError_t launch_batch(const BatchArgs& a, int grid, int block_threads, hipStream_t stream);
+// Persistent grid of `waves` one-wave blocks for short tiles.
+hipError_t launch_batch_short(const BatchArgs& a, uint32_t waves, hipStream_t stream);
 // Persistent grid of `grid` blocks taking groups of (waves per block)
 // consecutive tiles, in address order, from the counters in the batch
 // block's header.  Launches of one batch block must not overlap.

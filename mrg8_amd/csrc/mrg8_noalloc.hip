@@ -81,23 +81,18 @@ extern "C" int mrg8_batch_generate_noalloc(int device, const mrg8_stream_desc* d
   hipStream_t s = static_cast<hipStream_t>(stream);
   std::lock_guard<std::mutex> lk(g_host_mu);
   write_segments(reinterpret_cast<BatchSegment*>(g_host + sizeof(BatchHeader)), descs, count);
-  uint64_t nt = 0;
-  const size_t used = layout_batch_block(g_host, count, c.tile_outputs, tiles, &nt);
+  uint64_t nt = 0, weight = 0;
+  const size_t used = layout_batch_block(g_host, count, c.tile_outputs, tiles, &nt, &weight);
   // pageable source: the runtime has read g_host when the call returns
   hipError_t e = hipMemcpyAsync(ctx->noalloc_scratch, g_host, used, hipMemcpyHostToDevice, s);
   if (e != hipSuccess) return hip_fail(e, "scratch staging copy");
-  BatchArgs a{};
-  a.block = ctx->noalloc_scratch;
-  a.tile = c.tile_outputs;
-  a.states = nullptr;
-  a.lane = ctx->tables.lane;
-  a.digits = ctx->tables.digits;
-  a.xcds = (uint32_t)ctx->num_xcc;
-  a.xcd_group = xcd_run_blocks(*ctx, c.blocks_per_cu ? c.block_threads : tile_block_threads(c.block_threads));
+  LaunchConfig l;
+  l.block_threads = c.block_threads;
+  l.blocks_per_cu = c.blocks_per_cu;
+  l.tile = c.tile_outputs;
   // the staging copy above wrote the header's work counters as zero
-  e = c.blocks_per_cu == 0  ? launch_batch_tiles(a, nt, tile_block_threads(c.block_threads), s)
-      : c.blocks_per_cu < 0 ? launch_batch_queue(a, ctx->num_cu * -c.blocks_per_cu, c.block_threads, s)
-                            : launch_batch(a, ctx->num_cu * c.blocks_per_cu, c.block_threads, s);
+  e = launch_batch_kernel(*ctx, batch_args(*ctx, ctx->noalloc_scratch, l, nullptr), l,
+                          batch_kernel(*ctx, l, nt, weight), nt, s);
   if (e != hipSuccess) return hip_fail(e, "batch launch (no-alloc)");
   return MRG8_OK;
 }

@@ -74,15 +74,17 @@ size_t batch_block_bytes(uint32_t count, uint64_t ntiles) {
   return tile_seg_offset(count) + sizeof(uint32_t) * (size_t)ntiles;
 }
 
-size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t max_tiles, uint64_t* ntiles) {
+size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t max_tiles, uint64_t* ntiles,
+                          uint64_t* weight) {
   const size_t tb_off = tile_begin_offset(count), ts_off = tile_seg_offset(count);
   BatchHeader* hdr = reinterpret_cast<BatchHeader*>(mem);
   const BatchSegment* segs = reinterpret_cast<const BatchSegment*>(mem + sizeof(BatchHeader));
   uint64_t* tiles = reinterpret_cast<uint64_t*>(mem + tb_off);
   uint32_t* tile_seg = reinterpret_cast<uint32_t*>(mem + ts_off);
-  uint64_t t = 0;
+  uint64_t t = 0, total = 0;
   for (uint32_t i = 0; i < count; ++i) {
     tiles[i] = t;
+    total += segs[i].count * (segs[i].format == 2 ? 1 : kShortDouble);
     const uint64_t n = segment_tiles(segs[i].out, segs[i].format, segs[i].count, tile);
     const uint64_t end = std::min<uint64_t>(t + n, max_tiles);
     if (t < end) std::fill(tile_seg + t, tile_seg + end, i);
@@ -96,42 +98,85 @@ size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t 
   hdr->queue_next = 0;  // k_batch_queue's counters start at zero
   hdr->queue_done = 0;
   *ntiles = t;
+  *weight = total;
   return batch_block_bytes(count, std::min<uint64_t>(t, max_tiles));
 }
 
 uint64_t BatchSlot::finalise(uint32_t count, uint64_t tile) {
   uint64_t t = 0;
-  used_bytes_ = layout_batch_block(hmem_, count, tile, max_tiles_, &t);
+  used_bytes_ = layout_batch_block(hmem_, count, tile, max_tiles_, &t, &weight_);
   count_ = count;
   ntiles_ = t;
   dirty_ = true;
   return t;
 }
 
-BatchArgs BatchSlot::args(const LaunchConfig& cfg) const {
+BatchArgs batch_args(const DeviceContext& ctx, const uint8_t* block, const LaunchConfig& cfg, const uint32_t* states) {
   BatchArgs a{};
-  a.block = dmem_;
+  a.block = block;
   a.tile = cfg.tile;
-  a.states = states_;
-  a.lane = ctx_->tables.lane;
-  a.digits = ctx_->tables.digits;
-  a.xcds = (uint32_t)ctx_->num_xcc;
-  a.xcd_group = xcd_run_blocks(*ctx_, cfg.blocks_per_cu ? cfg.block_threads : tile_block_threads(cfg.block_threads));
+  a.states = states;
+  a.lane = ctx.tables.lane;
+  a.digits = ctx.tables.digits;
+  a.xcds = (uint32_t)ctx.num_xcc;
+  a.xcd_group = xcd_run_blocks(ctx, cfg.blocks_per_cu ? cfg.block_threads : tile_block_threads(cfg.block_threads));
+  a.mfma_a = ctx.tables.mfma_a;
+  a.mfma_c = ctx.tables.mfma_c;
+  a.mfma_skip_a = ctx.tables.mfma_skip_a;
+  a.mfma_skip_k = ctx.tables.mfma_skip_k;
+  a.min_waves = (uint32_t)ctx.num_cu * 4;  // one per SIMD
   return a;
 }
 
+// A striding grid of at least eight tiles for each SIMD takes the short-tile
+// kernel while its tiles average up to 1024 words or 128 doubles.  MI355X, us
+// per run, 63-bit offsets, striding (256 x 8 | 256 x 4) against short:
+//   tiles, outputs        striding       short
+//   65536 x  256 words    29.3 | 28.4    21.6
+//   65536 x   16 words    20.7 | 20.0    17.7
+//   65536 x 1024 words    73.4 | 69.4    64.8
+//    8192 x  256 words    12.2 |  9.0     6.8
+//    8192 x  512 words    13.8 | 10.8     9.0
+//    4096 x  512 words     8.6 |  8.5     8.2   (1024: 10.6 | 10.4, 11.7)
+//   65536 x  128 doubles  23.5 | 22.4    22.5
+//   32768 x  256 doubles  20.2 | 17.4    20.9   (512: 31.0 | 29.5, 34.3)
+// Doubles are bound by their stores from there on, and the vector kernel, with
+// four times the waves per SIMD, has more of them in flight.
+BatchKernel batch_kernel(const DeviceContext& ctx, const LaunchConfig& cfg, uint64_t ntiles, uint64_t weight) {
+  if (cfg.blocks_per_cu == 0) return BatchKernel::Tiles;
+  if (cfg.blocks_per_cu < 0) return BatchKernel::Queue;
+  const bool many = ntiles >= 8ull * 4 * ctx.num_cu, is_short = weight <= 1024 * ntiles;
+  return ctx.tables.mfma_a && many && is_short ? BatchKernel::Short : BatchKernel::Striding;
+}
+
+hipError_t launch_batch_kernel(const DeviceContext& ctx, BatchArgs a, const LaunchConfig& cfg, BatchKernel kernel,
+                               uint64_t ntiles, hipStream_t stream) {
+  switch (kernel) {
+    case BatchKernel::Tiles: return launch_batch_tiles(a, ntiles, tile_block_threads(cfg.block_threads), stream);
+    case BatchKernel::Queue: return launch_batch_queue(a, ctx.num_cu * -cfg.blocks_per_cu, cfg.block_threads, stream);
+    case BatchKernel::Striding: return launch_batch(a, ctx.num_cu * cfg.blocks_per_cu, cfg.block_threads, stream);
+    case BatchKernel::Short:
+      // at most the three waves per SIMD that its registers allow: what a
+      // larger grid costs to start is not hidden (65536 x 256 words, 12 waves
+      // per CU 21.6 us, 8 22.2, 16 24.4)
+      a.xcd_group = xcd_run_blocks(ctx, 64);
+      return launch_batch_short(a, (uint32_t)(ctx.num_cu * std::min(12, cfg.blocks_per_cu * (cfg.block_threads / 64))), stream);
+  }
+  return hipErrorInvalidValue;
+}
+
 hipError_t BatchSlot::launch(const LaunchConfig& cfg, hipStream_t stream) const {
-  if (cfg.blocks_per_cu == 0) return launch_batch_tiles(args(cfg), ntiles_, tile_block_threads(cfg.block_threads), stream);
-  if (cfg.blocks_per_cu < 0)
-    return launch_batch_queue(args(cfg), ctx_->num_cu * -cfg.blocks_per_cu, cfg.block_threads, stream);
-  return launch_batch(args(cfg), ctx_->num_cu * cfg.blocks_per_cu, cfg.block_threads, stream);
+  return launch_batch_kernel(*ctx_, batch_args(*ctx_, dmem_, cfg, states_), cfg,
+                             batch_kernel(*ctx_, cfg, ntiles_, weight_), ntiles_, stream);
 }
 
 int BatchSlot::capture(const LaunchConfig& cfg) {
-  // a one-tile-per-wave grid depends on the tile count, a persistent one of
-  // either kind does not (its kernel reads the count from the device block)
+  // a one-tile-per-wave grid depends on the tile count, a persistent one does
+  // not (its kernel reads the count from the device block); the striding grid's
+  // kernel depends on how short the staged tiles are
   if (have_graph_ && cfg.block_threads == captured_.block_threads && cfg.blocks_per_cu == captured_.blocks_per_cu &&
-      cfg.tile == captured_.tile && (cfg.blocks_per_cu != 0 || captured_ntiles_ == ntiles_))
+      cfg.tile == captured_.tile && (cfg.blocks_per_cu != 0 || captured_ntiles_ == ntiles_) &&
+      captured_kernel_ == batch_kernel(*ctx_, cfg, ntiles_, weight_))
     return MRG8_OK;
   if (int rc = wait_done()) return rc;  // the old graph may still be running
   if (exec_) (void)hipGraphExecDestroy(exec_);
@@ -153,6 +198,7 @@ int BatchSlot::capture(const LaunchConfig& cfg) {
   if (e != hipSuccess) return hip_fail(e, "graph capture");
   captured_ = cfg;
   captured_ntiles_ = ntiles_;
+  captured_kernel_ = batch_kernel(*ctx_, cfg, ntiles_, weight_);
   have_graph_ = true;
   return MRG8_OK;
 }

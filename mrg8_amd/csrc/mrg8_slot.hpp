@@ -37,8 +37,19 @@ size_t batch_block_bytes(uint32_t count, uint64_t ntiles);
 // Lays out the batch block at `mem` whose `count` segments are already
 // written after its header: prefix sums of tiles of `tile` outputs, the
 // tile -> segment map (at most `max_tiles` entries) and the header.  Sets
-// *ntiles to the tile count and returns the bytes in use.
-size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t max_tiles, uint64_t* ntiles);
+// *ntiles to the tile count and *weight to all segments' outputs, a double
+// as kShortDouble words, and returns the bytes in use.
+constexpr uint64_t kShortDouble = 8;
+size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t max_tiles, uint64_t* ntiles,
+                          uint64_t* weight);
+
+// The kernel of a launch of a batch block with `ntiles` (> 0) tiles and the
+// weight that its layout set, its arguments, and its launch.
+enum class BatchKernel { Tiles, Queue, Striding, Short };
+BatchKernel batch_kernel(const DeviceContext& ctx, const LaunchConfig& cfg, uint64_t ntiles, uint64_t weight);
+BatchArgs batch_args(const DeviceContext& ctx, const uint8_t* block, const LaunchConfig& cfg, const uint32_t* states);
+hipError_t launch_batch_kernel(const DeviceContext& ctx, BatchArgs a, const LaunchConfig& cfg, BatchKernel kernel,
+                               uint64_t ntiles, hipStream_t stream);
 
 class BatchSlot {
  public:
@@ -79,7 +90,6 @@ class BatchSlot {
   int capture(const LaunchConfig& cfg);
   // Records the completion event behind the last run if it is not there yet.
   hipError_t mark_last_run();
-  BatchArgs args(const LaunchConfig& cfg) const;
   hipError_t launch(const LaunchConfig& cfg, hipStream_t stream) const;
 
   DeviceContext* ctx_ = nullptr;
@@ -96,11 +106,12 @@ class BatchSlot {
   bool last_marked_ = true;            // run_done_ is recorded behind the last run
   bool last_queue_ = false;            // the last run was an address-order grid (work counters)
   uint32_t count_ = 0;
-  uint64_t ntiles_ = 0;
+  uint64_t ntiles_ = 0, weight_ = 0;
   hipGraph_t graph_ = nullptr;
   hipGraphExec_t exec_ = nullptr;
   LaunchConfig captured_{};
   uint64_t captured_ntiles_ = 0;
+  BatchKernel captured_kernel_ = BatchKernel::Tiles;
   bool have_graph_ = false;
 };
 

@@ -57,3 +57,71 @@ def test_jump_digits_and_zero_words(gpu, oracle_mod, grid):
         want, _ = oracle_mod.generate(oracle_mod.jump(np.asarray(st, np.uint32), off), cnt, fmt)
         have = got[p:p + cnt * want.itemsize]
         assert np.array_equal(have, want.view(np.uint8)), (list(st), off, fmt)
+
+
+SHORT_LENGTHS = [1, 2, 3, 15, 16, 17, 63, 127, 128, 129, 130, 255, 256, 257, 258, 300, 511, 512, 513, 0, 769]
+
+
+@pytest.mark.parametrize("grid,fmts,more", [((256, 8, 2048), (2,), 0), ((256, 4, 256), (2,), 5), ((64, 1, 2048), (2, 2, 2, 0), 1),
+                                            ((128, 2, 256), (0,), 8), ((256, 8, 512), (1, 2, 2, 0, 2), 16399)])
+def test_many_short_tiles(gpu, oracle_mod, grid, fmts, more):
+    """Batches of at least 32 tiles per CU on a striding grid: tiles of less,
+    exactly and more than a run of 256 outputs, groups of one and of several
+    formats, zero words and the all-zero state, alignments of one element; the
+    graph across a restaging with too few tiles, and the no-alloc entry point."""
+    import ctypes
+
+    import torch
+    from mrg8_amd import capi
+
+    rng = np.random.default_rng(7)
+    few = fmts == (0,)
+    lengths = [n for n in SHORT_LENGTHS if not few or n <= 256]
+    states = [rng.integers(1, P + 1, size=8) for _ in range(3)]
+    states += [np.array([0, 0, 0, 0, 0, 0, 0, 5]), np.zeros(8, int)]
+    kinds = []
+    for i in range(5 * len(lengths)):  # 5 states x 21 (or 14) lengths, every pair
+        off = [0, 1, 255, 1 << 32, int(rng.integers(0, 2**63))][(i // 3) % 5]
+        kinds.append((states[i % 5], off, lengths[i % len(lengths)], fmts[i % len(fmts)]))
+    want = [np.frombuffer(oracle_mod.generate(oracle_mod.jump(np.asarray(st, np.uint32), off), n, f)[0].tobytes(), np.uint8)
+            for st, off, n, f in kinds]
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    n = (32 * cus + more) * len(lengths) // (len(lengths) - (0 in lengths)) + 1  # empty segments have no tile
+    place, at = [], 0
+    for i in range(n):
+        place.append(at := at + (-at) % (4 if kinds[i % len(kinds)][3] == 2 else 8))
+        at += want[i % len(kinds)].size
+    weight = sum((1 if f == 2 else 8) * c for _, _, c, f in kinds) / sum(c > 0 for _, _, c, f in kinds)
+    assert weight <= 1024
+    expected = np.full(at + 64, 0xA5, np.uint8)
+    for i in range(n):
+        expected[place[i]:place[i] + want[i % len(kinds)].size] = want[i % len(kinds)]
+
+    buf = gpu.hip.DeviceBuffer(at + 64)
+    b = gpu.Batch(n, 8 * n)
+    b.set_config(*grid)
+    b.use_graph(True)
+    for count in (n, 300, n):
+        buf.fill_byte(0xA5)
+        b.set((*kinds[i % len(kinds)][:3], buf.ptr + place[i], kinds[i % len(kinds)][3]) for i in range(count))
+        say("short tiles", grid, fmts, count)
+        b.run()
+        b.run()
+        gpu.hip.synchronize()
+        got = buf.copy_to_host(np.uint8, at + 64)
+        end = place[count] if count < n else at
+        assert np.array_equal(got[:end], expected[:end]), np.flatnonzero(got[:end] != expected[:end])[:8]
+        assert (got[end:] == 0xA5).all()
+    b.close()
+    if more == 5:
+        arr = (capi.StreamDesc * n)()
+        for i in range(n):
+            st, off, cnt, f = kinds[i % len(kinds)]
+            arr[i].state = (ctypes.c_uint32 * 8)(*[int(x) for x in st])
+            arr[i].offset, arr[i].count, arr[i].out, arr[i].format = off, cnt, buf.ptr + place[i], f
+        buf.fill_byte(0xA5)
+        say("short tiles", "noalloc", grid, n)
+        capi.call("mrg8_batch_generate_noalloc", 0, arr, ctypes.c_uint32(n), ctypes.byref(capi.BatchConfig(*grid)), None)
+        gpu.hip.synchronize()
+        assert np.array_equal(buf.copy_to_host(np.uint8, at + 64), expected)
+    buf.free()
