@@ -313,21 +313,29 @@ int fill_mfma(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, void
   a.tiles = tiles;
   a.column = (uint32_t)column;
   a.waves_per_block = (uint32_t)(block_threads ? block_threads / 64 : format == MRG8_U32 ? 4 : 16);
-  // default: 32 KiB of output per wave for doubles, fewer tiles when that
-  // would leave fewer than 8 waves per CU; for words 16 KiB (two tiles of
-  // 2048) from 32 waves per CU on, one tile below
-  const bool long_words = format == MRG8_U32 && tiles >= (uint64_t)ctx.num_cu * 64;
-  uint64_t per = format == MRG8_U32
-                     ? (long_words ? 16384 / (uint64_t)esz / tile : 1)
-                     : std::min<uint64_t>(32768 / (uint64_t)esz / tile, tiles / ((uint64_t)ctx.num_cu * 8));
+  // Default, doubles: 32 KiB of output per wave, fewer tiles when that would
+  // leave fewer than 8 waves per CU.  Words: 4 tiles (of 2048) per wave, fewer
+  // while at most 12 waves per CU hold the fill (16 fit the LDS), and two, in
+  // XCD runs of 16 blocks (1 MiB), from 32 such waves per CU on.
+  // us with 1 | 2 | 4 tiles in dispatch order | 2 in runs of 16:
+  //   2^22.6 words (12 tiles per CU)  8.5 |   8.7 |   9.2 |   8.9
+  //   2^23                           10.4 |   9.7 |   9.9 |  10.1
+  //   2^24                           15.9 |  16.2 |  15.1 |  16.4
+  //   2^24.6                         22.3 |  23.2 |  21.1 |  22.4
+  //   2^25 (64 tiles per CU)         28.0 |  29.3 |  27.2 |  27.1
+  //   2^26                           53.9 |  56.3 |  50.7 |  48.9
+  //   2^28                           209  |   206 |   190 |   174
+  // (512-thread blocks of 4 tiles: 2^26 48.9, 2^28 181.)
+  const uint64_t cu = (uint64_t)ctx.num_cu;
+  const bool long_words = format == MRG8_U32 && tiles >= 64 * cu;
+  uint64_t per = format != MRG8_U32 ? std::min<uint64_t>(32768 / (uint64_t)esz / tile, tiles / (8 * cu))
+                 : long_words       ? 16384 / (uint64_t)esz / tile
+                 : tiles <= 12 * cu ? 1
+                 : tiles <= 24 * cu ? 2
+                                    : 32768 / (uint64_t)esz / tile;
   if (outputs_per_wave) per = outputs_per_wave / tile;
   a.tiles_per_wave = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(per, 1), 1u << 20);
   a.waves = (tiles + a.tiles_per_wave - 1) / a.tiles_per_wave;
-  // Blocks of four waves, in XCD runs of 16 (1 MiB of words) from 32 waves per
-  // CU on.  2^28 words: 171 us, in dispatch order 206 us, with one tile per
-  // wave 206 us, 512-thread blocks of 8192 words per wave 180 us; 2^26: 48.2
-  // us, 512-thread blocks the same; 2^24 with one tile per wave 14.9 us, two
-  // tiles 15.3 us.
   a.xcds = (uint32_t)ctx.num_xcc;
   a.xcd_group = a.waves_per_block == 4 && a.waves >= (uint64_t)ctx.num_cu * 32 ? 16 : 1;
   const uint64_t tail_first = head + tiles * tile;

@@ -125,3 +125,18 @@ def test_many_short_tiles(gpu, oracle_mod, grid, fmts, more):
         gpu.hip.synchronize()
         assert np.array_equal(buf.copy_to_host(np.uint8, at + 64), expected)
     buf.free()
+
+
+@pytest.mark.parametrize("tiles,more,pad", [(12, 2047, 0), (12, 2048, 1), (24, 0, 0), (24, 2049, 3), (64, -1, 0), (64, 1, 2)])
+def test_word_fill_tiles_per_wave(gpu, oracle_mod, tiles, more, pad):
+    """The matrix-core fill where its tiles per wave and its XCD runs change
+    (12, 24 and 64 tiles of 2048 words per CU)."""
+    import torch
+
+    n = tiles * torch.cuda.get_device_properties(0).multi_processor_count * 2048 + more + (-pad) % 256
+    say("word fill", n, pad)
+    g = gpu.mrg8_cuda(SEED + tiles)
+    got = run_device(gpu, g, n, 2, pad_elems=pad)
+    want, st = oracle_mod.generate(oracle_mod.seed_state(SEED + tiles), n, 2)
+    assert np.array_equal(got, want)
+    assert np.array_equal(g.get_state(), st)
