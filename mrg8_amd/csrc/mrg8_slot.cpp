@@ -132,16 +132,17 @@ BatchArgs batch_args(const DeviceContext& ctx, const uint8_t* block, const Launc
 // kernel while its tiles average up to 1024 words or 128 doubles.  MI355X, us
 // per run, 63-bit offsets, striding (256 x 8 | 256 x 4) against short:
 //   tiles, outputs        striding       short
-//   65536 x  256 words    29.3 | 28.4    21.6
-//   65536 x   16 words    20.7 | 20.0    17.7
-//   65536 x 1024 words    73.4 | 69.4    64.8
-//    8192 x  256 words    12.2 |  9.0     6.8
-//    8192 x  512 words    13.8 | 10.8     9.0
-//    4096 x  512 words     8.6 |  8.5     8.2   (1024: 10.6 | 10.4, 11.7)
-//   65536 x  128 doubles  23.5 | 22.4    22.5
-//   32768 x  256 doubles  20.2 | 17.4    20.9   (512: 31.0 | 29.5, 34.3)
+//   65536 x  256 words    30.6 | 28.7    20.9
+//   65536 x   16 words    20.6 | 19.9    16.2
+//   65536 x 1024 words    72.8 | 70.5    61.5
+//   51205 x  128 words    19.8 | 19.1    17.2
+//    8192 x  256 words    12.1 |  8.8     7.1
+//    8192 x 1024 words    17.2 | 14.2    13.2
+//    4096 x  512 words     8.7 |  8.5     8.4   (1024: 10.5 | 10.3, 12.0)
+//   65536 x  128 doubles  23.5 | 22.5    21.2   (256: 34.1 | 30.8, 31.4)
+//   32768 x  128 doubles  17.0 | 13.8    13.7   (256: 20.5 | 17.6, 18.3)
 // Doubles are bound by their stores from there on, and the vector kernel, with
-// four times the waves per SIMD, has more of them in flight.
+// more waves per SIMD, has more of them in flight (32768 x 512: 29 against 34).
 BatchKernel batch_kernel(const DeviceContext& ctx, const LaunchConfig& cfg, uint64_t ntiles, uint64_t weight) {
   if (cfg.blocks_per_cu == 0) return BatchKernel::Tiles;
   if (cfg.blocks_per_cu < 0) return BatchKernel::Queue;
@@ -158,7 +159,7 @@ hipError_t launch_batch_kernel(const DeviceContext& ctx, BatchArgs a, const Laun
     case BatchKernel::Short:
       // at most the three waves per SIMD that its registers allow: what a
       // larger grid costs to start is not hidden (65536 x 256 words, 12 waves
-      // per CU 21.6 us, 8 22.2, 16 24.4)
+      // per CU 20.9 us, 8 22.5, 16 24.6)
       a.xcd_group = xcd_run_blocks(ctx, 64);
       return launch_batch_short(a, (uint32_t)(ctx.num_cu * std::min(12, cfg.blocks_per_cu * (cfg.block_threads / 64))), stream);
   }
