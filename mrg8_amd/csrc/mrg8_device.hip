@@ -616,14 +616,20 @@ __global__ __launch_bounds__(1024) void k_batch_tiles(BatchArgs a) {
 }
 
 // Persistent batched kernel that takes its work in address order: each block
-// in turn takes the next group of (waves per block) consecutive tiles from a
-// counter in the batch block's header, and then works on it as k_batch_tiles
+// works on groups of (waves per block) consecutive tiles as k_batch_tiles
 // works on its block's tiles (waves 0-1 look up and jump the group's start
-// states and leave them in LDS, every wave generates one tile).  Blocks stay
-// resident, but the grid writes its tiles in the order a one-tile-per-wave
-// grid is dispatched in.  The last block to finish sets the counters back to
-// zero for the next launch; the counters make launches of one batch block
-// that overlap in time incorrect, which the host prevents.
+// states and leave them in LDS, every wave generates one tile).  A block's
+// first group is its index, every further one the next from a counter in the
+// batch block's header, taken while the current group is worked on.  Blocks
+// stay resident, but the grid writes its tiles in the order a
+// one-tile-per-wave grid is dispatched in.  The counter makes launches of one
+// batch block that overlap in time incorrect, which the host prevents.
+// The counter's atomics are its cost: some 13 ns each, one after the other.
+// With one for every group, waited for before its lookups, and another at
+// every block's end, 768 blocks took 20 us for one segment of 2048 doubles
+// (now 4.9), 54.8 for 500 of 32768 (31.4) and 139 for 2600 (116).  Striding
+// through the groups without a counter: 26.7 and 120 us, and 4013 segments of
+// 256 to 2^19 doubles 430 against 375 us.
 __global__ __launch_bounds__(1024) void k_batch_queue(BatchArgs a) {
   __shared__ uint32_t start_state[16][8];
   __shared__ uint64_t start_dst[16], start_cnt[16];
@@ -635,17 +641,20 @@ __global__ __launch_bounds__(1024) void k_batch_queue(BatchArgs a) {
   const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t nw = blockDim.x >> 6;
   const uint64_t ngroups = (tab.ntiles + nw - 1) / nw;
-  for (;;) {
-    if (threadIdx.x == 0) group = atomicAdd(&hdr->queue_next, 1u);
-    __syncthreads();
-    const uint64_t g = group;  // the same value in every wave: the block leaves the loop together
-    if (g >= ngroups) break;
+  for (uint64_t g = blockIdx.x; g < ngroups;) {  // the same value in every wave: the block leaves the loop together
     const uint64_t tile0 = g * nw;
+    // read per group: addresses and records held across the loop spill
+    const int32_t* digits = a.digits;
+    const CoefRecord* lane_rec = a.lane;
+    asm("" : "+s"(digits), "+s"(lane_rec));
+    const bool takes = ngroups > gridDim.x && threadIdx.x == blockDim.x - 64;
+    uint32_t taken = 0;
+    if (takes) taken = atomicAdd(&hdr->queue_next, 1u);
     if (wib * 8 < nw) {
       const uint32_t target = wib * 8 + (lane >> 3);
       const bool mine = target < nw && tile0 + target < tab.ntiles;
       const TileInfo ti = lookup_tile(tab, a, mine ? tile0 + target : tile0);
-      const uint32_t s = jump_group<2>(ti.state[lane & 7], mine ? ti.offset : 0, a.digits);
+      const uint32_t s = jump_group(ti.state[lane & 7], mine ? ti.offset : 0, digits);
       if (mine) start_state[target][lane & 7] = s;
       if (mine && (lane & 7) == 0) {
         start_dst[target] = ti.dst;
@@ -661,23 +670,21 @@ __global__ __launch_bounds__(1024) void k_batch_queue(BatchArgs a) {
       const uint64_t d = start_dst[wib], c = start_cnt[wib];
       void* out = global_pointer(readlane_u64(d, 0));
       const uint64_t cnt = readlane_u64(c, 0);
-      const CoefRecord* lane_rec = a.lane;
-      asm("" : "+s"(lane_rec));  // read per tile: the records of both layouts held across the loop spill
       switch (__builtin_amdgcn_readfirstlane(start_fmt[wib])) {
         case 0: batch_tile_alone<0>(out, cnt, u, lane_rec); break;
         case 1: batch_tile_alone<1>(out, cnt, u, lane_rec); break;
         default: batch_tile_alone<2>(out, cnt, u, lane_rec); break;
       }
     }
-    __syncthreads();  // LDS and `group` are rewritten by the next group
-  }
-  if (threadIdx.x == 0) {
-    __threadfence();  // this block's last take from the counter comes before its count of done blocks
-    if (atomicAdd(&hdr->queue_done, 1u) == gridDim.x - 1) {
-      // every block has left the loop: no block takes from the counter again
-      atomicExch(&hdr->queue_next, 0u);
-      atomicExch(&hdr->queue_done, 0u);
+    if (ngroups <= gridDim.x) return;
+    if (takes) {
+      group = gridDim.x + taken;
+      // the grid takes ngroups times: all but the first gridDim.x groups, and
+      // once in vain in every block
+      if (taken == ngroups - 1) atomicExch(&hdr->queue_next, 0u);
     }
+    __syncthreads();  // LDS is rewritten by the next group
+    g = group;
   }
 }
 

@@ -191,15 +191,14 @@ struct BatchHeader {
   uint64_t tile_begin_off;  // bytes from the block start
   uint64_t tile_seg_off;
   uint64_t pad0[12];
-  // Work counters of k_batch_queue: the next group of tiles to hand out and
-  // the blocks that have finished.  Zero when the block is staged; the last
-  // block of every launch sets them back to zero.  They have a 128-byte
-  // cache line of their own: every block's atomic adds on them would
-  // otherwise contend with the reads of the header and of the first
-  // segments (a single 2^28-double segment: 1.46 ms with the counters
-  // beside the header, 0.35 ms on a line of their own).
+  // Work counter of k_batch_queue: groups of tiles handed out beyond the
+  // blocks' first ones.  Zero when the block is staged; every launch that
+  // counts sets it back to zero.  It has a 128-byte cache line of its own:
+  // the atomic adds on it would otherwise contend with the reads of the
+  // header and of the first segments (a single 2^28-double segment: 1.46 ms
+  // with the counter beside the header, 0.35 ms on a line of its own).
   uint32_t queue_next;
-  uint32_t queue_done;
+  uint32_t reserved1;
   uint64_t pad1[15];
 };
 static_assert(sizeof(BatchHeader) == 256 && offsetof(BatchHeader, queue_next) == 128, "header layout");

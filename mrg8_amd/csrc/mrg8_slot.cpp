@@ -95,8 +95,7 @@ size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t 
   hdr->ntiles = t;
   hdr->tile_begin_off = tb_off;
   hdr->tile_seg_off = ts_off;
-  hdr->queue_next = 0;  // k_batch_queue's counters start at zero
-  hdr->queue_done = 0;
+  hdr->queue_next = 0;  // k_batch_queue's counter starts at zero
   *ntiles = t;
   *weight = total;
   return batch_block_bytes(count, std::min<uint64_t>(t, max_tiles));

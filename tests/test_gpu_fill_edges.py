@@ -140,3 +140,29 @@ def test_word_fill_tiles_per_wave(gpu, oracle_mod, tiles, more, pad):
     want, st = oracle_mod.generate(oracle_mod.seed_state(SEED + tiles), n, 2)
     assert np.array_equal(got, want)
     assert np.array_equal(g.get_state(), st)
+
+
+@pytest.mark.parametrize("threads", [64, 512])
+@pytest.mark.parametrize("groups", [-1, 0, 1, 777])
+@pytest.mark.parametrize("graph", [False, True])
+def test_address_order_counter(gpu, oracle_mod, threads, groups, graph):
+    """An address-order grid of one block per CU around the group count from
+    which its blocks take further groups from the counter, run after run."""
+    import torch
+
+    tiles = (torch.cuda.get_device_properties(0).multi_processor_count + groups) * (threads // 64)
+    n = tiles * 256 - 5
+    buf = gpu.hip.DeviceBuffer(n * 4)
+    b = gpu.Batch(1, tiles + 1)
+    b.set_config(threads, -1, 256)
+    b.use_graph(graph)
+    want, _ = oracle_mod.generate(oracle_mod.jump(oracle_mod.seed_state(SEED), 1 << 33), n, 2)
+    b.set([(oracle_mod.seed_state(SEED), 1 << 33, n, buf.ptr, 2)])
+    for run in range(3):
+        say("address order", threads, groups, graph, run)
+        buf.fill_byte(0xA5)
+        b.run()
+        gpu.hip.synchronize()
+        assert np.array_equal(buf.copy_to_host(np.uint32, n), want)
+    b.close()
+    buf.free()
