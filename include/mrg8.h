@@ -297,11 +297,10 @@ typedef struct mrg8_server_config {
   uint64_t step_outputs;       /* target outputs per launch (0 = automatic) */
   uint64_t tile_outputs;       /* outputs per work item, multiple of 256, at most 2^40
                                   (0 = automatic) */
-  int32_t block_threads;       /* 0 = automatic */
-  int32_t blocks_per_cu;       /* 0 = automatic (a persistent grid striding over the tiles, 1 block
-                                  per CU); as in mrg8_batch_config otherwise: < 0 takes the tiles in
-                                  address order (measured slower for the serving loop's short
-                                  request chunks) */
+  int32_t block_threads;       /* 0 = automatic: 768 threads, or 256 when blocks_per_cu is given */
+  int32_t blocks_per_cu;       /* 0 = automatic: one block per CU taking the tiles in address order,
+                                  or striding over them when block_threads is given; as in
+                                  mrg8_batch_config otherwise */
   uint32_t steps_in_flight;    /* launches in flight at once, 1..8 (0 = 3) */
   uint32_t age_limit_us;       /* requests admitted longer ago than this are served first,
                                   in admission order; the rest shortest-remaining first (0 = 1000) */

@@ -284,18 +284,28 @@ extern "C" int mrg8_server_create(int device, const mrg8_server_config* cfg, uin
   s->cfg.max_output_bytes = s->cfg.max_output_bytes / kAlign * kAlign;
   if (!s->cfg.max_inflight) s->cfg.max_inflight = 4096;
   // Defaults measured on MI355X with the log-uniform request mix at 300-680
-  // G samples/s offered: 4096-output tiles, one 512-thread block per CU,
-  // 2^26-output steps (8 tiles per wave), three steps in flight, 1 ms age
-  // limit.  Two waves per SIMD and step: with one (256 threads) a step alone
-  // on the card leaves its SIMDs waiting for the recurrence, p99 0.44, 0.66,
-  // 0.95 and 1.61 ms at 300, 490, 600 and 680 G samples/s against 0.36, 0.54,
-  // 0.77 and 1.57 ms, a burst of 48 requests 0.79 against 0.72 ms; with three
-  // or more the steps in flight get in each other's way (p99 3 ms and more at
-  // 680).  2^25-output steps stop keeping up above ~600 G samples/s;
-  // 2^27-output steps add ~0.2-0.4 ms to p99.
+  // G samples/s offered: 4096-output tiles, an address-order grid of one
+  // 768-thread block per CU, 2^26-output steps, three in flight, 1 ms age
+  // limit.  p99 at 300, 490, 600 and 680 G samples/s and the time of a burst
+  // of 48 requests (3.4 GB):
+  //   768 threads, address order      0.28 0.38 0.52 0.71 ms   0.66 ms
+  //   512 threads, address order      0.34 0.47 0.58 0.81      0.66
+  //   1024 threads, address order     0.31 0.43 0.60 1.04      0.72
+  //   512 threads, striding           0.37 0.54 0.78 1.57      0.73
+  //   256 threads, striding           0.44 0.66 0.95 1.61      0.79
+  //   768 threads, striding           0.35 0.63 3.55 23        0.80
+  // The striding grid's waves each write a place of their own for each step,
+  // and three of its steps at once get in each other's way.  With 768 threads:
+  // two or four steps in flight 0.76 and 0.92 ms at 680; 2^25-output steps
+  // stop keeping up there, 3 * 2^25 0.66 ms but 0.02 ms more at 490 and 600;
+  // 2048-output tiles 1.45 ms at 680.
   if (!s->cfg.tile_outputs) s->cfg.tile_outputs = 4096;
   if (!s->cfg.step_outputs) s->cfg.step_outputs = 1ull << 26;
-  if (!s->cfg.block_threads) s->cfg.block_threads = s->cfg.blocks_per_cu ? 256 : 512;
+  if (!s->cfg.block_threads && !s->cfg.blocks_per_cu) {
+    s->cfg.block_threads = 768;
+    s->cfg.blocks_per_cu = -1;
+  }
+  if (!s->cfg.block_threads) s->cfg.block_threads = 256;
   if (!s->cfg.blocks_per_cu) s->cfg.blocks_per_cu = 1;
   if (!s->cfg.steps_in_flight) s->cfg.steps_in_flight = 3;
   if (!s->cfg.age_limit_us) s->cfg.age_limit_us = 1000;
