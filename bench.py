@@ -136,7 +136,7 @@ def timed_series(step, stream, warmup, steps):
 def write_ceiling(buf, nbytes, s, reps=10):
     """Store-bandwidth ceiling over the same buffer: this project's probe
     (d[i] = i, the counterpart of cuda/stream.cu) with the double fill's 1 KiB
-    non-temporal wave stores (512-thread blocks in XCD runs), with the same
+    non-temporal wave stores (2048 per wave, 512-thread blocks in XCD runs), with the same
     runs in 1024-thread blocks in dispatch order, and in the reference's
     one-element-per-thread form, and the runtime's own fill kernel
     (hipMemsetAsync)."""
@@ -580,15 +580,15 @@ def main():
                      "frac": round(achieved / PEAK_GBS, 4),
                      "traffic": traffic,
                      "kernel": "k_fill<F64,4>",
-                     "shape": "default: 512-thread blocks, 2048 outputs per wave, 4 per lane, blocks in XCD runs "
+                     "shape": "default: 64-thread blocks, 1024 outputs per wave, 4 per lane, blocks in XCD runs "
                               "of 64 (each XCD writes 64 consecutive blocks' output)",
                      "kernel_ms": round(f64["kernel_ms"], 4),
                      "per_launch_ms": [round(x, 4) for x in f64["per_launch_ms"]],
                      "valu_busy_pct": valu_busy_from_profiles("fill_f64_2e28_counters.txt", "k_fill<F64,4>"),
                      "algorithmic_bytes_per_launch": f64["bytes"]},
         "u32": {"gsps": round(N_SINGLE * args.steps / single["u32"]["wall_s"] / 1e9, 2),
-                "kernel": "k_fill_mfma<U32,128,8>: the matrix-core fill (int8 MFMA), the default for words; "
-                          "512-thread blocks, 8192 words per wave",
+                "kernel": "k_fill_mfma<U32,128,4>: the matrix-core fill (int8 MFMA), the default for words; "
+                          "256-thread blocks in XCD runs of 16, 4096 words per wave",
                 "kernel_ms": round(single["u32"]["kernel_ms"], 4),
                 "vector_kernel_ms": round(single["u32_vector"]["kernel_ms"], 4),
                 "vector_per_launch_ms": [round(x, 4) for x in single["u32_vector"]["per_launch_ms"]],
@@ -607,8 +607,9 @@ def main():
             "per_launch_ms": [round(x, 4) for x in single["f64_matrix_core"]["per_launch_ms"]]},
         "small_2e24_f64": {k: round(v, 4) for k, v in single["small"].items()},
         "write_ceiling": {"kernel": "mrg8_probe_write: d[i] = i over the same 2 GiB with the fill's 1 KiB "
-                                    "non-temporal wave stores, 512-thread blocks in XCD runs of 64 (the "
-                                    "counterpart of cuda/stream.cu), measured just before the float64 leg",
+                                    "non-temporal wave stores, runs of 2048 doubles per wave, 512-thread "
+                                    "blocks in XCD runs of 64 (the counterpart of cuda/stream.cu), measured "
+                                    "just before the float64 leg",
                           "gbs": ceiling["gbs"], "frac": round(ceiling["gbs"] / PEAK_GBS, 4),
                           "fill_frac_of_ceiling": round(achieved / ceiling["gbs"], 4),
                           "dispatch_order_gbs": single["ceiling"]["probe_dispatch_order"]["gbs"],

@@ -208,7 +208,7 @@ int mrg8_check_jump_matrix(const char* path);
  * All pointers are device memory; d_in and d_out may be the same buffer
  * (other overlaps are not allowed); state words must be at most 2^31 - 1.
  * Stream-ordered on `stream`.  The first call with words > 1 builds a
- * 2.3 MiB table for byte positions 8..31 on the device (kept for the
+ * 1.5 MiB table for byte positions 8..31 on the device (kept for the
  * process). */
 int mrg8_advance_states(int device, const uint32_t* d_in, const uint64_t* d_offsets, uint32_t words,
                         uint32_t* d_out, uint64_t n, void* stream);
@@ -227,7 +227,9 @@ typedef struct mrg8_stream_desc {
 } mrg8_stream_desc;
 
 /* Launch configuration (picked by mrg8_batch_autotune or set by hand; a new
- * batch starts with 1024 threads, one tile per wave, 2048-output tiles). */
+ * batch starts with 1024 threads, one tile per wave, 2048-output tiles; a
+ * one-tile-per-wave grid runs in blocks of at most 256 threads whatever is
+ * asked for). */
 typedef struct mrg8_batch_config {
   int32_t block_threads;  /* 64..1024, multiple of 64 */
   int32_t blocks_per_cu;  /* 0: one tile per wave (grid from the tile count; best for long
@@ -238,7 +240,10 @@ typedef struct mrg8_batch_config {
                              streams; the counter is 32 bits: a run with more groups of
                              tiles than that is MRG8_ERR_CAPACITY); > 0: persistent grid
                              of CUs * blocks_per_cu blocks
-                             (best for many short segments with long jumps) */
+                             (best for many short segments with long jumps; with 32 or more
+                             tiles per CU that average up to 1024 words or 128 doubles, waves
+                             of the same grid take eight tiles at a time, at most 12 waves
+                             per CU) */
   uint64_t tile_outputs;  /* outputs per work item, multiple of 256, at most 2^40 */
 } mrg8_batch_config;
 

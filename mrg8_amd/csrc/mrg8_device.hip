@@ -21,7 +21,10 @@
 //   * k_fill: one stream, one tile per wave, each wave on its own (no LDS, no
 //     barrier).
 //   * k_batch: many streams (segments), a persistent grid striding over
-//     tiles, tables and counts read from one device block.
+//     tiles, tables and counts read from one device block; k_batch_short the
+//     same for many short tiles, eight at a time on the matrix cores;
+//     k_batch_tiles one tile per wave; k_batch_queue a persistent grid that
+//     takes its tiles in address order.
 //   * Blocks reach their part of the output through xcd_block: the
 //     dispatcher deals blocks to the XCDs in turn, and large grids give each
 //     XCD runs of consecutive blocks' output instead.
@@ -950,10 +953,11 @@ __global__ __launch_bounds__(256) void k_stage(const u4_t* __restrict__ src, u4_
 // i < 2 and 8 + W(g) + i - 2 for i >= 2.  So the step's last eight outputs
 // (positions 8..15, the column's next state) are registers 2 and 3 of
 // exactly the lanes whose K-group needs them: no lane exchange.
-// A wave makes a few consecutive tiles (32 KiB of output: the store
+// A wave makes a few consecutive tiles (up to 32 KiB of output: the store
 // pattern of short-lived waves in address order, which persistent waves
-// striding over the tiles did not match: 427-474 against 339 us for 2^28
-// doubles).  The 16 column states of the wave's next tile are the current
+// striding over the tiles, with a product by A^(2048 waves) from one to the
+// next, do not match: 192-217 against 170 us for 2^28 words, 371-480 against
+// 325 us for doubles).  The 16 column states of the wave's next tile are the current
 // ones times A^2048: one more product of the same form, whose rows put the
 // new words in registers 0 and 1 of the lanes that need them.  Only a
 // wave's first tile computes its column states from the tile state (the

@@ -90,7 +90,7 @@ extern "C" int mrg8_batch_generate_noalloc(int device, const mrg8_stream_desc* d
   l.block_threads = c.block_threads;
   l.blocks_per_cu = c.blocks_per_cu;
   l.tile = c.tile_outputs;
-  // the staging copy above wrote the header's work counters as zero
+  // the staging copy above wrote the header's work counter as zero
   e = launch_batch_kernel(*ctx, batch_args(*ctx, ctx->noalloc_scratch, l, nullptr), l,
                           batch_kernel(*ctx, l, nt, weight), nt, s);
   if (e != hipSuccess) return hip_fail(e, "batch launch (no-alloc)");

@@ -229,7 +229,7 @@ int BatchSlot::run(const LaunchConfig& cfg, hipStream_t stream, bool graph, bool
   hipError_t e = hipSuccess;
   // The device block may be overwritten once this slot's previous launch has
   // finished, and an address-order grid (blocks_per_cu < 0) may start only
-  // after the previous one has reset the work counters in it: on the same
+  // after the previous one has reset the work counter in it: on the same
   // stream both are ordered after the previous launch; on another stream
   // they wait for it.  Runs next to an address-order run wait as well, so
   // that two such runs are never apart by one unordered run in between.

@@ -104,7 +104,7 @@ class BatchSlot {
   bool copy_pending_ = false, run_pending_ = false, dirty_ = false;
   hipStream_t last_stream_ = nullptr;  // stream of the last run
   bool last_marked_ = true;            // run_done_ is recorded behind the last run
-  bool last_queue_ = false;            // the last run was an address-order grid (work counters)
+  bool last_queue_ = false;            // the last run was an address-order grid (work counter)
   uint32_t count_ = 0;
   uint64_t ntiles_ = 0, weight_ = 0;
   hipGraph_t graph_ = nullptr;
