@@ -143,7 +143,7 @@ int device_context(int device, DeviceContext** out) {
     (void)hipGetLastError();  // not reported by a later launch check
     xcc = 1;
   }
-  if (xcc < 1) xcc = 1;
+  if (xcc < 1 || (xcc & (xcc - 1))) xcc = 1;  // xcd_block's counts are powers of two
   ctx->num_xcc = xcc;
   void* p = nullptr;
   const size_t rec_bytes = sizeof(CoefRecord) * lane.size();

@@ -221,16 +221,17 @@ __device__ __forceinline__ uint32_t jump_group(uint32_t s, uint64_t off, const i
   return word_of(e);
 }
 
-// This lane's word (lane & 7) of a state in uniform registers.
+// A state in uniform registers, its word j in lane j < 8 (jump_group's first
+// lane group; the other lanes hold 1, no zero word).  Eight lane writes: a
+// select by lane takes 23 operations, and a load by lane waits for memory.
+// The wait states are for a DPP read of the result.
 __device__ __forceinline__ uint32_t own_word(const uint32_t st[8]) {
-  const uint32_t row = threadIdx.x & 7;
-  uint32_t w = st[0];
-#pragma unroll
-  for (int j = 1; j < 8; ++j) {
-    uint32_t x = st[j];
-    asm("" : "+s"(x));  // a select between registers, not a load at a computed address
-    w = row == (uint32_t)j ? x : w;
-  }
+  uint32_t w = 1;
+  asm("v_writelane_b32 %0, %1, 0\n\tv_writelane_b32 %0, %2, 1\n\tv_writelane_b32 %0, %3, 2\n\t"
+      "v_writelane_b32 %0, %4, 3\n\tv_writelane_b32 %0, %5, 4\n\tv_writelane_b32 %0, %6, 5\n\t"
+      "v_writelane_b32 %0, %7, 6\n\tv_writelane_b32 %0, %8, 7\n\ts_nop 1"
+      : "+v"(w)
+      : "s"(st[0]), "s"(st[1]), "s"(st[2]), "s"(st[3]), "s"(st[4]), "s"(st[5]), "s"(st[6]), "s"(st[7]));
   return w;
 }
 
@@ -425,13 +426,14 @@ __device__ __forceinline__ uint64_t fill_first(const FillArgs& a, uint64_t w) { 
 // (b mod x alike) instead take runs of g consecutive blocks' output within
 // every span of x g blocks, whatever r is.  Blocks past the last whole span
 // keep their own part.  Either way every part is written by exactly one
-// block.
+// block.  x and g are powers of two: with divisions this was 60 scalar and 15
+// vector operations at the start of every wave, now nine scalar ones.
 __device__ __forceinline__ uint64_t xcd_block(uint32_t b, uint32_t nb, uint32_t x, uint32_t g) {
-  if (g <= 1 || x == 0) return b;
-  const uint32_t span = x * g, whole = nb / span * span;
-  if (b >= whole) return b;
-  const uint32_t q = b / x;
-  return (uint64_t)(q / g * span + (b - q * x) * g + q % g);
+  if (g <= 1) return b;
+  const uint32_t lx = __builtin_ctz(x), lg = __builtin_ctz(g), span = lx + lg;
+  if (b >= nb >> span << span) return b;
+  const uint32_t q = b >> lx;
+  return (q >> lg << span) + ((b & (x - 1)) << lg) + (q & (g - 1));
 }
 
 // Bound by the store stream for long fills and by the latency of a wave's

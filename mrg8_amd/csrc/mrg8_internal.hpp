@@ -34,7 +34,9 @@ struct DeviceContext {
 // Blocks per XCD run for kernels that map blocks through xcd_block: runs of
 // 32768 threads (64 blocks of 512) on a device with more than one XCD.
 inline uint32_t xcd_run_blocks(const DeviceContext& ctx, int block_threads) {
-  return ctx.num_xcc > 1 && block_threads > 0 ? (uint32_t)std::max(1, 32768 / block_threads) : 1;
+  uint32_t run = ctx.num_xcc > 1 && block_threads > 0 ? (uint32_t)std::max(1, 32768 / block_threads) : 1;
+  while (run & (run - 1)) run &= run - 1;  // xcd_block's counts are powers of two
+  return run;
 }
 
 // Threads per block of a one-tile-per-wave grid: at most 256 of the
