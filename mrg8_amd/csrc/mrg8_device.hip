@@ -221,6 +221,56 @@ __device__ __forceinline__ uint32_t jump_group(uint32_t s, uint64_t off, const i
   return word_of(e);
 }
 
+// A pointer that the compiler takes as read anew, still to global memory (a
+// flat access counts as an LDS access too, and waits for those).
+template <typename T>
+__device__ __forceinline__ const T* opaque(const T* p) {
+  uint64_t address = reinterpret_cast<uint64_t>(p);
+  asm("" : "+s"(address));
+  return (const T*)(const __attribute__((address_space(1))) T*)address;
+}
+
+// jump_group with one uniform offset, for the state in a wave's first lane
+// group: digits and row addresses stay scalar (nothing is counted over the
+// lanes, no address is added in vector registers).  2^28 doubles 323 -> 320
+// us at full clock, 365 -> 351 us in launches 6 to 25 after idle, where the
+// power manager holds the clock down by the work of the vector units; 2^22
+// 8.0 -> 8.2 us.
+__device__ __forceinline__ uint32_t jump_uniform(uint32_t s, uint64_t off, const int32_t* digits) {
+  if (off == 0) return s;
+  const uint32_t lo = (uint32_t)off;
+  uint32_t hi = (uint32_t)(off >> 32);
+  const uint32_t row = 4 * (threadIdx.x & 7);
+  auto load = [&](int k) {
+    return load_row(opaque(digits + k * kPositionInts + digit_of(k < 4 ? lo : hi, k) * kJumpMatrixInts) + row);
+  };
+  JumpRow m[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) m[k] = load(k);
+  if (__ballot(s == 0u)) {
+#pragma unroll 1
+    for (int k = 0; k < kJumpPositions; ++k) {
+      const uint32_t d = digit_of(k < 4 ? lo : hi, k);
+      if (d) s = jump_zero_words(s, d, digits + k * kPositionInts);
+    }
+    return s;
+  }
+  int32_t e = centre_word(s);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (digit_of(lo, k)) e = jump_row(m[k], e);
+    asm("" : "+s"(hi));  // compared anew: one comparison kept for all is kept in vector registers
+    if (hi) m[k] = load(k + 4);
+  }
+  asm("" : "+s"(hi));
+  if (hi) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (digit_of(hi, k)) e = jump_row(m[k], e);
+  }
+  return word_of(e);
+}
+
 // A state in uniform registers, its word j in lane j < 8 (jump_group's first
 // lane group; the other lanes hold 1, no zero word).  Eight lane writes: a
 // select by lane takes 23 operations, and a load by lane waits for memory.
@@ -453,7 +503,7 @@ __global__ __launch_bounds__(1024) void k_fill(FillArgs a) {
   const uint64_t first = fill_first(a, w);
   if (first >= a.n) return;
   const uint64_t cnt = min(a.head + (w + 1) * a.tile, a.n) - first;
-  const uint32_t word = jump_group(own_word(a.start.state), a.start.offset + first, a.digits);
+  const uint32_t word = jump_uniform(own_word(a.start.state), a.start.offset + first, a.digits);
   uint32_t s[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) s[j] = __builtin_amdgcn_readlane(word, j);
@@ -649,9 +699,8 @@ __global__ __launch_bounds__(1024) void k_batch_queue(BatchArgs a) {
   for (uint64_t g = blockIdx.x; g < ngroups;) {  // the same value in every wave: the block leaves the loop together
     const uint64_t tile0 = g * nw;
     // read per group: addresses and records held across the loop spill
-    const int32_t* digits = a.digits;
-    const CoefRecord* lane_rec = a.lane;
-    asm("" : "+s"(digits), "+s"(lane_rec));
+    const int32_t* digits = opaque(a.digits);
+    const CoefRecord* lane_rec = opaque(a.lane);
     const bool takes = ngroups > gridDim.x && threadIdx.x == blockDim.x - 64;
     uint32_t taken = 0;
     if (takes) taken = atomicAdd(&hdr->queue_next, 1u);
@@ -1049,7 +1098,7 @@ __device__ __forceinline__ void mfma_tiles(const MfmaFillArgs& a, uint64_t t0, u
   // column n are the tile's outputs 128 n - 8 + q, from the tile state
   long B;
   {
-    const uint32_t word = jump_group(own_word(a.start.state), a.start.offset + a.head + t0 * kTile, a.digits);
+    const uint32_t word = jump_uniform(own_word(a.start.state), a.start.offset + a.head + t0 * kTile, a.digits);
     uint32_t s[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] = __builtin_amdgcn_readlane(word, j);
@@ -1152,7 +1201,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_fill_mfma(MfmaFillArgs a) {
   const uint64_t e = w - a.waves;
   if (e >= a.extra) return;
   const uint64_t first = a.extra_first[e], cnt = a.extra_count[e];
-  const uint32_t word = jump_group(own_word(a.start.state), a.start.offset + first, a.digits);
+  const uint32_t word = jump_uniform(own_word(a.start.state), a.start.offset + first, a.digits);
   uint32_t s[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) s[j] = __builtin_amdgcn_readlane(word, j);
