@@ -420,11 +420,20 @@ __device__ __forceinline__ void peel_to_boundary(typename Out<FMT>::T*& dst, uin
 // first output) is s, into dst[0..cnt), with this lane's records k (and the
 // lane records, for the outputs before the first 1 KiB boundary).  `cnt` and
 // s must be wave-uniform; dst need only be element-aligned.
-template <int FMT, int PL, uintptr_t ALIGN = kStoreAlign>
+// NARROW keeps the coefficients 32 bits wide: the compiler otherwise widens
+// them ahead of the loop, half of them with a copy each.  It frees some 25
+// registers, which pays where a group's start is waited for (address-order
+// grid: 133 to 709 segments 2 to 4 % faster, 17 GB the same) and not where
+// more resident waves loosen the order of the stores (2^28 doubles 352 against
+// 320 us, one tile per wave 2 to 3 % slower for large batches).
+template <int FMT, int PL, uintptr_t ALIGN = kStoreAlign, bool NARROW = false>
 __device__ __forceinline__ void generate_run(typename Out<FMT>::T* __restrict__ dst, uint64_t cnt, uint32_t s[8],
-                                             const Coef (&k)[PL], const CoefRecord* __restrict__ lane_rec) {
+                                             const Coef (&k0)[PL], const CoefRecord* __restrict__ lane_rec) {
   typedef LaneLayout<FMT, PL> L;
   constexpr int kPer = 64 * PL;
+  Coef k[PL];
+#pragma unroll
+  for (int i = 0; i < PL; ++i) k[i] = k0[i];
   const uint32_t lane = threadIdx.x & 63;
   uint32_t any = 0;
 #pragma unroll
@@ -438,6 +447,12 @@ __device__ __forceinline__ void generate_run(typename Out<FMT>::T* __restrict__ 
   const uint64_t full = cnt / kPer;
   const uint64_t rem = cnt - full * kPer;
   for (uint64_t it = 0; it < full; ++it) {
+    if constexpr (NARROW) {
+#pragma unroll
+      for (int i = 0; i < PL; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) asm("" : "+v"(k[i].c[j]));
+    }
     int32_t e[8];
     centre(s, e);
     uint32_t r[PL];
@@ -516,10 +531,10 @@ __global__ __launch_bounds__(1024) void k_fill(FillArgs a) {
 // the first ALIGN-byte boundary; only tile 0 of a segment can have any).  The
 // persistent kernel passes ALIGN = 16: with the 1 KiB peel it ran 10 % slower
 // on the 4096-stream batch.
-template <int FMT, int PL, uintptr_t ALIGN = kStoreAlign>
+template <int FMT, int PL, uintptr_t ALIGN = kStoreAlign, bool NARROW = false>
 __device__ __forceinline__ void batch_tile(void* out, uint64_t cnt, uint32_t s[8], const Coef (&k)[PL],
                                            const CoefRecord* __restrict__ lane_rec) {
-  if (cnt) generate_run<FMT, PL, ALIGN>(static_cast<typename Out<FMT>::T*>(out), cnt, s, k, lane_rec);
+  if (cnt) generate_run<FMT, PL, ALIGN, NARROW>(static_cast<typename Out<FMT>::T*>(out), cnt, s, k, lane_rec);
 }
 
 __device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int lane) {
@@ -621,12 +636,12 @@ __global__ __launch_bounds__(1024) void k_batch(BatchArgs a) {
 }
 
 // One tile of a batch with the fill's layout (4 outputs per lane).
-template <int FMT>
+template <int FMT, bool NARROW = false>
 __device__ __forceinline__ void batch_tile_alone(void* out, uint64_t cnt, uint32_t s[8],
                                                  const CoefRecord* __restrict__ lane_rec) {
   Coef k[4];
   load_lane_coefs<FMT, 4>(k, lane_rec);
-  batch_tile<FMT, 4>(out, cnt, s, k, lane_rec);
+  batch_tile<FMT, 4, kStoreAlign, NARROW>(out, cnt, s, k, lane_rec);
 }
 
 // Batched kernel with one tile per wave (grid = tiles / waves per block):
@@ -725,9 +740,9 @@ __global__ __launch_bounds__(1024) void k_batch_queue(BatchArgs a) {
       void* out = global_pointer(readlane_u64(d, 0));
       const uint64_t cnt = readlane_u64(c, 0);
       switch (__builtin_amdgcn_readfirstlane(start_fmt[wib])) {
-        case 0: batch_tile_alone<0>(out, cnt, u, lane_rec); break;
-        case 1: batch_tile_alone<1>(out, cnt, u, lane_rec); break;
-        default: batch_tile_alone<2>(out, cnt, u, lane_rec); break;
+        case 0: batch_tile_alone<0, true>(out, cnt, u, lane_rec); break;
+        case 1: batch_tile_alone<1, true>(out, cnt, u, lane_rec); break;
+        default: batch_tile_alone<2, true>(out, cnt, u, lane_rec); break;
       }
     }
     if (ngroups <= gridDim.x) return;
