@@ -420,20 +420,18 @@ __device__ __forceinline__ void peel_to_boundary(typename Out<FMT>::T*& dst, uin
 // first output) is s, into dst[0..cnt), with this lane's records k (and the
 // lane records, for the outputs before the first 1 KiB boundary).  `cnt` and
 // s must be wave-uniform; dst need only be element-aligned.
-// NARROW keeps the coefficients 32 bits wide: the compiler otherwise widens
-// them ahead of the loop, half of them with a copy each.  It frees some 25
-// registers, which pays where a group's start is waited for (address-order
-// grid: 133 to 709 segments 2 to 4 % faster, 17 GB the same) and not where
-// more resident waves loosen the order of the stores (2^28 doubles 352 against
-// 320 us, one tile per wave 2 to 3 % slower for large batches).
+// NARROW (k a variable of the caller) keeps the coefficients 32 bits wide: the
+// compiler otherwise widens them ahead of the loop, half of them with a copy
+// each.  It frees some 25 registers, which pays where a group's start is waited
+// for (address-order grid: batches of less than 2^26 outputs 2 to 5 % faster,
+// 17 GB the same) and not where more resident waves loosen the order of the
+// stores (2^28 doubles 352 against 320 us, one tile per wave 2 to 3 % slower
+// for large batches).
 template <int FMT, int PL, uintptr_t ALIGN = kStoreAlign, bool NARROW = false>
 __device__ __forceinline__ void generate_run(typename Out<FMT>::T* __restrict__ dst, uint64_t cnt, uint32_t s[8],
-                                             const Coef (&k0)[PL], const CoefRecord* __restrict__ lane_rec) {
+                                             const Coef (&k)[PL], const CoefRecord* __restrict__ lane_rec) {
   typedef LaneLayout<FMT, PL> L;
   constexpr int kPer = 64 * PL;
-  Coef k[PL];
-#pragma unroll
-  for (int i = 0; i < PL; ++i) k[i] = k0[i];
   const uint32_t lane = threadIdx.x & 63;
   uint32_t any = 0;
 #pragma unroll
@@ -451,7 +449,7 @@ __device__ __forceinline__ void generate_run(typename Out<FMT>::T* __restrict__ 
 #pragma unroll
       for (int i = 0; i < PL; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) asm("" : "+v"(k[i].c[j]));
+        for (int j = 0; j < 8; ++j) asm("" : "+v"(const_cast<Coef&>(k[i]).c[j]));
     }
     int32_t e[8];
     centre(s, e);
