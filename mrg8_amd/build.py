@@ -28,7 +28,7 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", "-Wall", "-Wextra", "-Wno-unused-paramet
 # not needed here and some forms have proven unreliable on this hardware).
 # MFMA results go to ordinary VGPRs: the matrix-core fill reads every result
 # with VALU instructions, and results left in AGPRs cost one v_accvgpr_read
-# per value (four per output) -- 189 VGPRs either way fit its two waves per SIMD.
+# per value (four per output); 100 VGPRs leave room for four waves per SIMD.
 DEVICE = ["-x", "hip", "--offload-arch=" + ARCH,
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
           "-mllvm", "-amdgpu-mfma-vgpr-form"]
