@@ -241,9 +241,9 @@ typedef struct mrg8_batch_config {
                              tiles than that is MRG8_ERR_CAPACITY); > 0: persistent grid
                              of CUs * blocks_per_cu blocks
                              (best for many short segments with long jumps; with 32 or more
-                             tiles per CU that average up to 1024 words or 128 doubles, waves
-                             of the same grid take eight tiles at a time, at most 12 waves
-                             per CU) */
+                             tiles per CU that average up to 1024 words or 128 doubles, the
+                             longest not far above the average, waves of the same grid take
+                             eight tiles at a time, at most 12 waves per CU) */
   uint64_t tile_outputs;  /* outputs per work item, multiple of 256, at most 2^40 */
 } mrg8_batch_config;
 

@@ -81,8 +81,8 @@ extern "C" int mrg8_batch_generate_noalloc(int device, const mrg8_stream_desc* d
   hipStream_t s = static_cast<hipStream_t>(stream);
   std::lock_guard<std::mutex> lk(g_host_mu);
   write_segments(reinterpret_cast<BatchSegment*>(g_host + sizeof(BatchHeader)), descs, count);
-  uint64_t nt = 0, weight = 0;
-  const size_t used = layout_batch_block(g_host, count, c.tile_outputs, tiles, &nt, &weight);
+  BatchWork work;
+  const size_t used = layout_batch_block(g_host, count, c.tile_outputs, tiles, &work);
   // pageable source: the runtime has read g_host when the call returns
   hipError_t e = hipMemcpyAsync(ctx->noalloc_scratch, g_host, used, hipMemcpyHostToDevice, s);
   if (e != hipSuccess) return hip_fail(e, "scratch staging copy");
@@ -92,7 +92,7 @@ extern "C" int mrg8_batch_generate_noalloc(int device, const mrg8_stream_desc* d
   l.tile = c.tile_outputs;
   // the staging copy above wrote the header's work counter as zero
   e = launch_batch_kernel(*ctx, batch_args(*ctx, ctx->noalloc_scratch, l, nullptr), l,
-                          batch_kernel(*ctx, l, nt, weight), nt, s);
+                          batch_kernel(*ctx, l, work), work.tiles, s);
   if (e != hipSuccess) return hip_fail(e, "batch launch (no-alloc)");
   return MRG8_OK;
 }

@@ -74,18 +74,31 @@ size_t batch_block_bytes(uint32_t count, uint64_t ntiles) {
   return tile_seg_offset(count) + sizeof(uint32_t) * (size_t)ntiles;
 }
 
-size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t max_tiles, uint64_t* ntiles,
-                          uint64_t* weight) {
+size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t max_tiles, BatchWork* work) {
   const size_t tb_off = tile_begin_offset(count), ts_off = tile_seg_offset(count);
   BatchHeader* hdr = reinterpret_cast<BatchHeader*>(mem);
   const BatchSegment* segs = reinterpret_cast<const BatchSegment*>(mem + sizeof(BatchHeader));
   uint64_t* tiles = reinterpret_cast<uint64_t*>(mem + tb_off);
   uint32_t* tile_seg = reinterpret_cast<uint32_t*>(mem + ts_off);
-  uint64_t t = 0, total = 0;
+  uint64_t t = 0;
+  BatchWork w;
+  auto add = [&](uint64_t outputs, uint64_t times) {
+    const uint64_t runs = outputs / kShortRunOutputs + (outputs % kShortRunOutputs != 0);
+    w.runs += runs * times;
+    w.longest = std::max(w.longest, runs);
+  };
   for (uint32_t i = 0; i < count; ++i) {
     tiles[i] = t;
-    total += segs[i].count * (segs[i].format == 2 ? 1 : kShortDouble);
-    const uint64_t n = segment_tiles(segs[i].out, segs[i].format, segs[i].count, tile);
+    const uint64_t c = segs[i].count, n = segment_tiles(segs[i].out, segs[i].format, c, tile);
+    w.weight += c * (segs[i].format == 2 ? 1 : kShortDouble);
+    if (n == 1) {
+      add(c, 1);
+    } else if (n) {  // the first tile with the head, whole ones, the last
+      const uint64_t first = segment_head(segs[i].out, segs[i].format, c, tile) + tile;
+      add(first, 1);
+      if (n > 2) add(tile, n - 2);
+      add(c - first - (n - 2) * tile, 1);
+    }
     const uint64_t end = std::min<uint64_t>(t + n, max_tiles);
     if (t < end) std::fill(tile_seg + t, tile_seg + end, i);
     t += n;
@@ -96,18 +109,16 @@ size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t 
   hdr->tile_begin_off = tb_off;
   hdr->tile_seg_off = ts_off;
   hdr->queue_next = 0;  // k_batch_queue's counter starts at zero
-  *ntiles = t;
-  *weight = total;
+  w.tiles = t;
+  *work = w;
   return batch_block_bytes(count, std::min<uint64_t>(t, max_tiles));
 }
 
 uint64_t BatchSlot::finalise(uint32_t count, uint64_t tile) {
-  uint64_t t = 0;
-  used_bytes_ = layout_batch_block(hmem_, count, tile, max_tiles_, &t, &weight_);
+  used_bytes_ = layout_batch_block(hmem_, count, tile, max_tiles_, &work_);
   count_ = count;
-  ntiles_ = t;
   dirty_ = true;
-  return t;
+  return work_.tiles;
 }
 
 BatchArgs batch_args(const DeviceContext& ctx, const uint8_t* block, const LaunchConfig& cfg, const uint32_t* states) {
@@ -142,11 +153,23 @@ BatchArgs batch_args(const DeviceContext& ctx, const uint8_t* block, const Launc
 //   32768 x  128 doubles  17.0 | 13.8    13.7   (256: 20.5 | 17.6, 18.3)
 // Doubles are bound by their stores from there on, and the vector kernel, with
 // more waves per SIMD, has more of them in flight (32768 x 512: 29 against 34).
-BatchKernel batch_kernel(const DeviceContext& ctx, const LaunchConfig& cfg, uint64_t ntiles, uint64_t weight) {
+// A wave works on eight tiles until the longest of them is done, so the longest may
+// take 2.8 times the mean's runs of 256 outputs (or two of them, which cost
+// little more than one).  us, 256 x 8, striding against short:
+//   longest / mean   tiles                               striding  short
+//   2.0              16384: 512 words, 15872: 16           12.4     10.3
+//   2.6              65536, log-uniform in 8 to 1023       46.4     42.3
+//   2.9              65536: 8192 of 1024, the rest 16      34.6     40.1
+//   3.7              65536: 2048 of 1024, the rest 16      26.8     33.8
+//   3.9              65536, log-uniform in 8 to 2047       58.5     69.1
+//   6.8              32768: 128 of 2048, the rest 128      19.6     32.8
+//   43               32768: 128 of 16384, the rest 128     46.4    192
+BatchKernel batch_kernel(const DeviceContext& ctx, const LaunchConfig& cfg, const BatchWork& work) {
   if (cfg.blocks_per_cu == 0) return BatchKernel::Tiles;
   if (cfg.blocks_per_cu < 0) return BatchKernel::Queue;
-  const bool many = ntiles >= 8ull * 4 * ctx.num_cu, is_short = weight <= 1024 * ntiles;
-  return ctx.tables.mfma_a && many && is_short ? BatchKernel::Short : BatchKernel::Striding;
+  const bool many = work.tiles >= 8ull * 4 * ctx.num_cu, is_short = work.weight <= 1024 * work.tiles;
+  const bool even = work.longest <= 2 || 5 * work.longest * work.tiles <= 14 * work.runs;
+  return ctx.tables.mfma_a && many && is_short && even ? BatchKernel::Short : BatchKernel::Striding;
 }
 
 hipError_t launch_batch_kernel(const DeviceContext& ctx, BatchArgs a, const LaunchConfig& cfg, BatchKernel kernel,
@@ -167,7 +190,7 @@ hipError_t launch_batch_kernel(const DeviceContext& ctx, BatchArgs a, const Laun
 
 hipError_t BatchSlot::launch(const LaunchConfig& cfg, hipStream_t stream) const {
   return launch_batch_kernel(*ctx_, batch_args(*ctx_, dmem_, cfg, states_), cfg,
-                             batch_kernel(*ctx_, cfg, ntiles_, weight_), ntiles_, stream);
+                             batch_kernel(*ctx_, cfg, work_), work_.tiles, stream);
 }
 
 int BatchSlot::capture(const LaunchConfig& cfg) {
@@ -175,8 +198,8 @@ int BatchSlot::capture(const LaunchConfig& cfg) {
   // not (its kernel reads the count from the device block); the striding grid's
   // kernel depends on how short the staged tiles are
   if (have_graph_ && cfg.block_threads == captured_.block_threads && cfg.blocks_per_cu == captured_.blocks_per_cu &&
-      cfg.tile == captured_.tile && (cfg.blocks_per_cu != 0 || captured_ntiles_ == ntiles_) &&
-      captured_kernel_ == batch_kernel(*ctx_, cfg, ntiles_, weight_))
+      cfg.tile == captured_.tile && (cfg.blocks_per_cu != 0 || captured_ntiles_ == work_.tiles) &&
+      captured_kernel_ == batch_kernel(*ctx_, cfg, work_))
     return MRG8_OK;
   if (int rc = wait_done()) return rc;  // the old graph may still be running
   if (exec_) (void)hipGraphExecDestroy(exec_);
@@ -197,8 +220,8 @@ int BatchSlot::capture(const LaunchConfig& cfg) {
   (void)hipStreamDestroy(cs);
   if (e != hipSuccess) return hip_fail(e, "graph capture");
   captured_ = cfg;
-  captured_ntiles_ = ntiles_;
-  captured_kernel_ = batch_kernel(*ctx_, cfg, ntiles_, weight_);
+  captured_ntiles_ = work_.tiles;
+  captured_kernel_ = batch_kernel(*ctx_, cfg, work_);
   have_graph_ = true;
   return MRG8_OK;
 }
@@ -211,17 +234,17 @@ hipError_t BatchSlot::mark_last_run() {
 }
 
 int BatchSlot::run(const LaunchConfig& cfg, hipStream_t stream, bool graph, bool track) {
-  if (count_ == 0 || ntiles_ == 0) return MRG8_OK;
-  if (ntiles_ > max_tiles_) return fail(MRG8_ERR_CAPACITY, "staged work needs more than max_tiles tiles");
+  if (count_ == 0 || work_.tiles == 0) return MRG8_OK;
+  if (work_.tiles > max_tiles_) return fail(MRG8_ERR_CAPACITY, "staged work needs more than max_tiles tiles");
   const uint64_t wpb = (uint64_t)cfg.block_threads / 64;
   if (cfg.blocks_per_cu == 0) {  // one wave per tile: the grid (work-items in total) is a 32-bit quantity
-    if ((ntiles_ + wpb - 1) / wpb * (uint64_t)cfg.block_threads > 0xffffffffull)
+    if ((work_.tiles + wpb - 1) / wpb * (uint64_t)cfg.block_threads > 0xffffffffull)
       return fail(MRG8_ERR_CAPACITY, "%llu tiles need more than 2^32 - 1 work-items at one tile per wave; use larger "
-                  "tiles or a persistent grid", (unsigned long long)ntiles_);
+                  "tiles or a persistent grid", (unsigned long long)work_.tiles);
   } else if (cfg.blocks_per_cu < 0) {  // the work counter is 32 bits: groups plus one last take per block
-    if ((ntiles_ + wpb - 1) / wpb + (uint64_t)ctx_->num_cu * (uint64_t)-cfg.blocks_per_cu > 0xffffffffull)
+    if ((work_.tiles + wpb - 1) / wpb + (uint64_t)ctx_->num_cu * (uint64_t)-cfg.blocks_per_cu > 0xffffffffull)
       return fail(MRG8_ERR_CAPACITY, "%llu tiles are more groups than the address-order grid counts; use larger tiles",
-                  (unsigned long long)ntiles_);
+                  (unsigned long long)work_.tiles);
   }
   DeviceGuard dg(ctx_->device);
   int rc = graph ? capture(cfg) : MRG8_OK;

@@ -37,16 +37,21 @@ size_t batch_block_bytes(uint32_t count, uint64_t ntiles);
 // Lays out the batch block at `mem` whose `count` segments are already
 // written after its header: prefix sums of tiles of `tile` outputs, the
 // tile -> segment map (at most `max_tiles` entries) and the header.  Sets
-// *ntiles to the tile count and *weight to all segments' outputs, a double
-// as kShortDouble words, and returns the bytes in use.
+// *work to what the launch rules read and returns the bytes in use.
+struct BatchWork {
+  uint64_t tiles = 0;
+  uint64_t weight = 0;   // all outputs, a double as kShortDouble words
+  uint64_t runs = 0;     // all tiles' runs of kShortRunOutputs outputs
+  uint64_t longest = 0;  // the longest tile's runs
+};
 constexpr uint64_t kShortDouble = 8;
-size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t max_tiles, uint64_t* ntiles,
-                          uint64_t* weight);
+constexpr uint64_t kShortRunOutputs = 2 * kBatchSkip;  // k_batch_short: outputs of a tile at a time
+size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t max_tiles, BatchWork* work);
 
-// The kernel of a launch of a batch block with `ntiles` (> 0) tiles and the
-// weight that its layout set, its arguments, and its launch.
+// The kernel of a launch of a batch block with the (non-empty) work that its
+// layout set, its arguments, and its launch.
 enum class BatchKernel { Tiles, Queue, Striding, Short };
-BatchKernel batch_kernel(const DeviceContext& ctx, const LaunchConfig& cfg, uint64_t ntiles, uint64_t weight);
+BatchKernel batch_kernel(const DeviceContext& ctx, const LaunchConfig& cfg, const BatchWork& work);
 BatchArgs batch_args(const DeviceContext& ctx, const uint8_t* block, const LaunchConfig& cfg, const uint32_t* states);
 hipError_t launch_batch_kernel(const DeviceContext& ctx, BatchArgs a, const LaunchConfig& cfg, BatchKernel kernel,
                                uint64_t ntiles, hipStream_t stream);
@@ -73,7 +78,7 @@ class BatchSlot {
   // sums, tile -> segment map).  Returns the number of tiles; the caller
   // keeps it <= max_tiles.
   uint64_t finalise(uint32_t count, uint64_t tile);
-  uint64_t staged_tiles() const { return ntiles_; }
+  uint64_t staged_tiles() const { return work_.tiles; }
   uint32_t staged_count() const { return count_; }
 
   // Copies the staged block (when it changed) and launches on `stream`:
@@ -106,7 +111,7 @@ class BatchSlot {
   bool last_marked_ = true;            // run_done_ is recorded behind the last run
   bool last_queue_ = false;            // the last run was an address-order grid (work counter)
   uint32_t count_ = 0;
-  uint64_t ntiles_ = 0, weight_ = 0;
+  BatchWork work_;
   hipGraph_t graph_ = nullptr;
   hipGraphExec_t exec_ = nullptr;
   LaunchConfig captured_{};

@@ -166,3 +166,32 @@ def test_address_order_counter(gpu, oracle_mod, threads, groups, graph):
         assert np.array_equal(buf.copy_to_host(np.uint32, n), want)
     b.close()
     buf.free()
+
+
+def test_striding_grid_with_uneven_tiles(gpu, oracle_mod):
+    """More than 32 tiles per CU on a striding grid, one of 16384 outputs among
+    sixteen tiny ones (which the short-tile kernel leaves alone), against the
+    oracle."""
+    from mrg8_amd.hip import DeviceBuffer
+
+    import torch
+
+    rng = np.random.default_rng(17)
+    tiny = 34 * torch.cuda.get_device_properties(0).multi_processor_count
+    state = rng.integers(1, P + 1, size=8)
+    words, _ = oracle_mod.generate(oracle_mod.jump(np.asarray(state, np.uint32), 1 << 40), 20000, 2)
+    lengths = [16384 if i % 17 == 0 else 1 + i % 90 for i in range(tiny)]
+    skip = [i % 1000 for i in range(tiny)]  # segment i starts this far into `words`
+    place = np.concatenate([[0], np.cumsum(lengths)])
+    buf = DeviceBuffer(int(place[-1]) * 4)
+    b = gpu.Batch(tiny, 2 * tiny)
+    b.set_config(256, 8, 16384)
+    b.set((state, (1 << 40) + k, n, buf.ptr + 4 * int(at), 2) for k, n, at in zip(skip, lengths, place))
+    say("uneven tiles", tiny)
+    b.run()
+    gpu.hip.synchronize()
+    got = buf.copy_to_host(np.uint32, int(place[-1]))
+    b.close()
+    buf.free()
+    for k, n, at in zip(skip, lengths, place):
+        assert np.array_equal(got[at:at + n], words[k:k + n]), (k, n)

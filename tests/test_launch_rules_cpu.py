@@ -1,0 +1,92 @@
+"""The host's launch rules, called in the library with a device context made up here (256 CUs, 8 XCDs, no device)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "mrg8_amd", "libmrg8_amd.so")
+ROCM = "/opt/rocm"
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None or not os.path.exists(ROCM + "/include/hip/hip_runtime.h"),
+                                reason="needs g++ and the HIP headers")
+
+HEAD = r"""
+#include <cstdio>
+#include <cstring>
+#include <vector>
+#include "mrg8_slot.hpp"
+using namespace mrg8;
+static int bad = 0;
+#define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); bad = 1; } } while (0)
+"""
+
+MAIN = r"""
+int main() {
+  static DeviceContext ctx;
+  ctx.num_cu = 256;
+  ctx.num_xcc = 8;
+  static uint32_t table;
+  ctx.tables.mfma_a = &table;
+  run(ctx);
+  if (!bad) std::printf("ok\n");
+  return bad;
+}
+"""
+
+
+def check(tmp_path, body):
+    src, exe = tmp_path / "rules.cpp", tmp_path / "rules"
+    src.write_text(HEAD + "#line 1\n" + body + MAIN)
+    r = subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", f"-I{ROCM}/include",
+                        "-I" + os.path.join(ROOT, "mrg8_amd", "csrc"), str(src), LIB, f"-L{ROCM}/lib", "-lamdhip64",
+                        "-Wl,-rpath," + os.path.dirname(LIB), f"-Wl,-rpath,{ROCM}/lib", "-o", str(exe)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr
+
+
+def test_short_tile_kernel_takes_even_batches_only(tmp_path):
+    """Batches of 10240 segments on a striding grid: the short-tile kernel works
+    on eight tiles until the longest is done, so one long tile among many short
+    ones goes to the other striding kernel, whatever the average."""
+    check(tmp_path, r"""
+static BatchKernel kernel_of(const DeviceContext& ctx, uint64_t usual, uint64_t other, uint32_t every, int format, uint64_t tile,
+                             uint32_t count = 10240, uint64_t misalign = 0) {
+  std::vector<uint8_t> mem(batch_block_bytes(count, 1 << 20));
+  BatchSegment* segs = reinterpret_cast<BatchSegment*>(mem.data() + sizeof(BatchHeader));
+  for (uint32_t i = 0; i < count; ++i) {
+    segs[i].count = every && i % every == 0 ? other : usual;
+    segs[i].out = reinterpret_cast<void*>((uintptr_t(1) << 40) + (uintptr_t(i) << 24) + misalign);
+    segs[i].format = format;
+  }
+  BatchWork work;
+  layout_batch_block(mem.data(), count, tile, 1 << 20, &work);
+  LaunchConfig cfg;
+  cfg.block_threads = 256;
+  cfg.blocks_per_cu = 8;
+  cfg.tile = tile;
+  return batch_kernel(ctx, cfg, work);
+}
+static void run(const DeviceContext& ctx) {
+  for (uint64_t n : {1, 16, 256, 257, 512, 1024}) CHECK(kernel_of(ctx, n, 0, 0, 2, 2048) == BatchKernel::Short);
+  CHECK(kernel_of(ctx, 1025, 0, 0, 2, 2048) == BatchKernel::Striding);
+  CHECK(kernel_of(ctx, 128, 0, 0, 0, 2048) == BatchKernel::Short);
+  CHECK(kernel_of(ctx, 129, 0, 0, 0, 2048) == BatchKernel::Striding);
+  CHECK(kernel_of(ctx, 16, 0, 0, 2, 2048, 8191) == BatchKernel::Striding);
+  // two runs of 256 are always close enough; from three on, 2.8 times the average
+  CHECK(kernel_of(ctx, 16, 512, 10240, 2, 2048) == BatchKernel::Short);
+  CHECK(kernel_of(ctx, 16, 513, 10240, 2, 2048) == BatchKernel::Striding);
+  CHECK(kernel_of(ctx, 16, 1024, 2, 2, 2048) == BatchKernel::Short);
+  CHECK(kernel_of(ctx, 16, 1024, 8, 2, 2048) == BatchKernel::Striding);
+  CHECK(kernel_of(ctx, 64, 16384, 17, 2, 16384) == BatchKernel::Striding);
+  CHECK(kernel_of(ctx, 64, 16384, 10240, 2, 16384) == BatchKernel::Striding);
+  // long segments cut into equal tiles, and one whose first tile has a long head
+  CHECK(kernel_of(ctx, 1024 * 20, 0, 0, 2, 1024) == BatchKernel::Short);
+  CHECK(kernel_of(ctx, 1024 * 20, 0, 0, 2, 1024, 512) == BatchKernel::Short);
+  CHECK(kernel_of(ctx, 1024 * 20, 0, 0, 2, 1024, 10240, 8) == BatchKernel::Short);
+  CHECK(kernel_of(ctx, 64, 1024 + 700, 10240, 2, 1024, 10240, 4 * 324) == BatchKernel::Striding);
+}
+""")
