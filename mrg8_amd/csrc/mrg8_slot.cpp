@@ -44,17 +44,14 @@ void BatchSlot::release() {
   DeviceGuard dg(ctx_->device);
   if (copy_pending_ && staged_) (void)hipEventSynchronize(staged_);
   if (run_pending_ && run_done_) (void)wait_done();
-  if (exec_) (void)hipGraphExecDestroy(exec_);
-  if (graph_) (void)hipGraphDestroy(graph_);
+  for (Captured& c : captured_) c.release();
   if (staged_) (void)hipEventDestroy(staged_);
   if (run_done_) (void)hipEventDestroy(run_done_);
   if (hmem_) (void)hipHostFree(hmem_);
   if (dmem_) (void)hipFree(dmem_);
-  exec_ = nullptr;
-  graph_ = nullptr;
   staged_ = run_done_ = nullptr;
   hmem_ = dmem_ = nullptr;
-  copy_pending_ = run_pending_ = have_graph_ = false;
+  copy_pending_ = run_pending_ = false;
   last_stream_ = nullptr;
   last_marked_ = true;
   last_queue_ = false;
@@ -193,36 +190,44 @@ hipError_t BatchSlot::launch(const LaunchConfig& cfg, hipStream_t stream) const 
                              batch_kernel(*ctx_, cfg, work_), work_.tiles, stream);
 }
 
-int BatchSlot::capture(const LaunchConfig& cfg) {
-  // a one-tile-per-wave grid depends on the tile count, a persistent one does
-  // not (its kernel reads the count from the device block); the striding grid's
-  // kernel depends on how short the staged tiles are
-  if (have_graph_ && cfg.block_threads == captured_.block_threads && cfg.blocks_per_cu == captured_.blocks_per_cu &&
-      cfg.tile == captured_.tile && (cfg.blocks_per_cu != 0 || captured_ntiles_ == work_.tiles) &&
-      captured_kernel_ == batch_kernel(*ctx_, cfg, work_))
+void BatchSlot::Captured::release() {
+  if (exec) (void)hipGraphExecDestroy(exec);
+  if (graph) (void)hipGraphDestroy(graph);
+  *this = Captured{};
+}
+
+// A one-tile-per-wave grid depends on the tile count, a persistent one does
+// not (its kernel reads the count from the device block).  The striding
+// grid's kernel depends on how short the staged tiles are: it has a graph for
+// each, so that restaging from one kind to the other neither waits for the
+// runs before it nor captures anew (165 us of host time a run, 52 us without).
+int BatchSlot::capture(const LaunchConfig& cfg, hipGraphExec_t* exec) {
+  Captured& c = captured_[batch_kernel(*ctx_, cfg, work_) == BatchKernel::Short ? 0 : 1];
+  if (c.exec && cfg.block_threads == c.cfg.block_threads && cfg.blocks_per_cu == c.cfg.blocks_per_cu &&
+      cfg.tile == c.cfg.tile && (cfg.blocks_per_cu != 0 || c.ntiles == work_.tiles)) {
+    *exec = c.exec;
     return MRG8_OK;
+  }
   if (int rc = wait_done()) return rc;  // the old graph may still be running
-  if (exec_) (void)hipGraphExecDestroy(exec_);
-  if (graph_) (void)hipGraphDestroy(graph_);
-  exec_ = nullptr;
-  graph_ = nullptr;
-  have_graph_ = false;
+  c.release();
   hipStream_t cs = nullptr;
   hipError_t e = hipStreamCreateWithFlags(&cs, hipStreamNonBlocking);
   if (e != hipSuccess) return hip_fail(e, "hipStreamCreate(capture)");
   e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
   if (e == hipSuccess) {
     hipError_t e1 = launch(cfg, cs);
-    hipError_t e2 = hipStreamEndCapture(cs, &graph_);
+    hipError_t e2 = hipStreamEndCapture(cs, &c.graph);
     e = e1 != hipSuccess ? e1 : e2;
   }
-  if (e == hipSuccess) e = hipGraphInstantiate(&exec_, graph_, nullptr, nullptr, 0);
+  if (e == hipSuccess) e = hipGraphInstantiate(&c.exec, c.graph, nullptr, nullptr, 0);
   (void)hipStreamDestroy(cs);
-  if (e != hipSuccess) return hip_fail(e, "graph capture");
-  captured_ = cfg;
-  captured_ntiles_ = work_.tiles;
-  captured_kernel_ = batch_kernel(*ctx_, cfg, work_);
-  have_graph_ = true;
+  if (e != hipSuccess) {
+    c.release();
+    return hip_fail(e, "graph capture");
+  }
+  c.cfg = cfg;
+  c.ntiles = work_.tiles;
+  *exec = c.exec;
   return MRG8_OK;
 }
 
@@ -247,7 +252,8 @@ int BatchSlot::run(const LaunchConfig& cfg, hipStream_t stream, bool graph, bool
                   (unsigned long long)work_.tiles);
   }
   DeviceGuard dg(ctx_->device);
-  int rc = graph ? capture(cfg) : MRG8_OK;
+  hipGraphExec_t exec = nullptr;
+  int rc = graph ? capture(cfg, &exec) : MRG8_OK;
   if (rc) return rc;
   hipError_t e = hipSuccess;
   // The device block may be overwritten once this slot's previous launch has
@@ -268,7 +274,7 @@ int BatchSlot::run(const LaunchConfig& cfg, hipStream_t stream, bool graph, bool
     copy_pending_ = true;
     dirty_ = false;
   }
-  e = graph ? hipGraphLaunch(exec_, stream) : launch(cfg, stream);
+  e = graph ? hipGraphLaunch(exec, stream) : launch(cfg, stream);
   if (e != hipSuccess) return hip_fail(e, graph ? "hipGraphLaunch" : "batch launch");
   run_pending_ = true;
   last_stream_ = stream;

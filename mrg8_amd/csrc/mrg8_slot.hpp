@@ -8,7 +8,7 @@
 // launches the kernel directly or
 // replays a captured graph holding it; the kernel reads the counts and table
 // offsets from the header, so a graph is captured once per launch
-// configuration.
+// configuration and kernel.
 //
 // Completion of a run is an event recorded behind it on its stream.  A
 // tracked run records it at once (the serving loop polls it); otherwise it
@@ -92,7 +92,15 @@ class BatchSlot {
   int wait_done();
 
  private:
-  int capture(const LaunchConfig& cfg);
+  // A captured launch of the staged work.
+  struct Captured {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    LaunchConfig cfg{};
+    uint64_t ntiles = 0;
+    void release();
+  };
+  int capture(const LaunchConfig& cfg, hipGraphExec_t* exec);
   // Records the completion event behind the last run if it is not there yet.
   hipError_t mark_last_run();
   hipError_t launch(const LaunchConfig& cfg, hipStream_t stream) const;
@@ -112,12 +120,7 @@ class BatchSlot {
   bool last_queue_ = false;            // the last run was an address-order grid (work counter)
   uint32_t count_ = 0;
   BatchWork work_;
-  hipGraph_t graph_ = nullptr;
-  hipGraphExec_t exec_ = nullptr;
-  LaunchConfig captured_{};
-  uint64_t captured_ntiles_ = 0;
-  BatchKernel captured_kernel_ = BatchKernel::Tiles;
-  bool have_graph_ = false;
+  Captured captured_[2];  // k_batch_short's, and any other kernel's
 };
 
 }  // namespace mrg8

@@ -195,3 +195,51 @@ def test_striding_grid_with_uneven_tiles(gpu, oracle_mod):
     buf.free()
     for k, n, at in zip(skip, lengths, place):
         assert np.array_equal(got[at:at + n], words[k:k + n]), (k, n)
+
+
+def test_graph_of_each_striding_kernel_is_kept(gpu, oracle_mod):
+    """A striding grid's runs as graph replays, restaged from long tiles to many
+    short ones and back: once both graphs are there, a run returns while the
+    runs before it still execute."""
+    import ctypes
+
+    import torch
+    from mrg8_amd import capi
+
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    state = oracle_mod.seed_state(SEED)
+    long, short = (64, 1 << 20), (40 * cus, 20)  # segments, words each
+    bufs = [gpu.hip.DeviceBuffer(4 * k * n) for k, n in (long, short)]
+    descs = []
+    for (k, n), buf in zip((long, short), bufs):
+        arr = (capi.StreamDesc * k)()
+        for i in range(k):
+            arr[i].state = (ctypes.c_uint32 * 8)(*state.tolist())
+            arr[i].offset, arr[i].count, arr[i].out, arr[i].format = i * n, n, buf.ptr + 4 * i * n, 2
+        descs.append((arr, ctypes.c_uint32(k)))
+    b = gpu.Batch(40 * cus, 1 << 17)
+    b.set_config(256, 8, 2048)
+    b.use_graph(True)
+    stream, issued = torch.cuda.Stream(), torch.cuda.Event()
+    for which in (0, 1, 0, 1, 0):
+        capi.call("mrg8_batch_set", b._h, *descs[which])
+        b.run(stream)
+    stream.synchronize()
+    for repeat in range(3):
+        for buf in bufs:
+            buf.fill_byte(0xA5)
+        capi.call("mrg8_batch_set", b._h, *descs[0])
+        say("graph of each kernel", repeat)
+        for _ in range(600):  # some 30 ms
+            b.run(stream)
+        issued.record(stream)
+        capi.call("mrg8_batch_set", b._h, *descs[1])
+        b.run(stream)
+        assert not issued.query(), "the run waited for those before it"
+        stream.synchronize()
+        for (k, n), buf in zip((long, short), bufs):
+            want, _ = oracle_mod.generate(state, k * n, 2)
+            assert np.array_equal(buf.copy_to_host(np.uint32, k * n), want)
+    b.close()
+    for buf in bufs:
+        buf.free()
