@@ -279,10 +279,24 @@ void default_shape(const DeviceContext& ctx, uint64_t n, int format, int per_lan
 // MI355X with the default shape, runs of 1, 16, 64 and 256 blocks: 2^28
 // doubles 382, 335, 318 and 326 us, 2^24 24.5, 25.6, 24.0 and 25.3 us, 2^22
 // 8.5, 8.8, 8.4 and 9.1 us; 2^21 (8 waves per CU) 5.5, 5.8, 5.7 and 5.9 us.
-// Word fills were slower in runs and are left in dispatch order.
-uint32_t fill_xcd_group(const DeviceContext& ctx, int format, uint64_t waves, int block_threads) {
-  if (format == MRG8_U32 || ctx.num_xcc <= 1 || waves < (uint64_t)ctx.num_cu * 16) return 1;
+// Larger blocks and longer waves have longer runs, which pay from 64 waves per
+// CU on (at 16, in runs | in dispatch order: 64 threads of 65536 outputs per
+// wave, 2^28 473 | 413 us; 256 of 2048, 2^23 16.1 | 14.3; 256 of 1024, 2^22
+// 10.0 | 8.9).  Word fills were slower in runs and are left in dispatch order.
+uint32_t fill_xcd_group(const DeviceContext& ctx, int format, uint64_t waves, int block_threads, uint64_t tile) {
+  const uint64_t per_cu = block_threads == 64 && tile <= 1024 ? 16 : 64;
+  if (format == MRG8_U32 || ctx.num_xcc <= 1 || waves < (uint64_t)ctx.num_cu * per_cu) return 1;
   return std::min(64u, xcd_run_blocks(ctx, block_threads));
+}
+
+// Whether the waves of a block wait for one another before their outputs.  In
+// XCD runs of blocks with several waves of 2048 to 8192 doubles they do: apart,
+// their stores leave the address order (with the barrier | without: 512 threads
+// of 2048, 2^26 91.1 | 92.9 us, 2^28 344 | 349; 1024 of 2048, 2^28 344 | 358;
+// one wave jumping for all of its block 343 and 353).  Shorter waves lose by it
+// (512 threads of 1024, 2^28 366 | 341 us), longer ones neither.
+bool fill_in_step(uint32_t xcd_group, int block_threads, uint64_t tile) {
+  return xcd_group > 1 && block_threads > 64 && tile >= 2048 && tile <= 8192;
 }
 
 namespace {
@@ -436,7 +450,8 @@ int fill_device(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, vo
   a.lane = ctx.tables.lane;
   a.digits = ctx.tables.digits;
   a.xcds = (uint32_t)ctx.num_xcc;
-  a.xcd_group = fill_xcd_group(ctx, format, fill_waves(n, head, tile), block_threads);
+  a.xcd_group = fill_xcd_group(ctx, format, fill_waves(n, head, tile), block_threads, tile);
+  a.in_step = fill_in_step(a.xcd_group, block_threads, tile);
   int prev = 0;
   (void)hipGetDevice(&prev);
   if (prev != ctx.device) (void)hipSetDevice(ctx.device);

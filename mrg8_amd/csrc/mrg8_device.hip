@@ -514,9 +514,10 @@ __global__ __launch_bounds__(1024) void k_fill(FillArgs a) {
   const uint32_t nw = blockDim.x >> 6;
   const uint64_t w = xcd_block(blockIdx.x, gridDim.x, a.xcds, a.xcd_group) * nw + wib;
   const uint64_t first = fill_first(a, w);
+  const uint32_t word = jump_uniform(own_word(a.start.state), a.start.offset + first, a.digits);
+  if (a.in_step) __syncthreads();  // every wave of the block, with outputs or not
   if (first >= a.n) return;
   const uint64_t cnt = min(a.head + (w + 1) * a.tile, a.n) - first;
-  const uint32_t word = jump_uniform(own_word(a.start.state), a.start.offset + first, a.digits);
   uint32_t s[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) s[j] = __builtin_amdgcn_readlane(word, j);

@@ -89,6 +89,7 @@ struct FillArgs {
   const int32_t* digits;    // jump matrices (DeviceTables::digits)
   uint32_t xcds;            // XCDs that blocks are dealt to in turn (block b runs on XCD b mod xcds)
   uint32_t xcd_group;       // consecutive blocks of output per XCD run (1: blocks in dispatch order)
+  uint32_t in_step;         // a block's waves start their outputs together
 };
 
 // A matrix-core fill: `tiles` whole tiles of 16 x `column` outputs at

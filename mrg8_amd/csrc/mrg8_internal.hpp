@@ -70,6 +70,11 @@ int format_size(int format);
 int fill_device(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, void* dptr, uint64_t n, int format,
                 hipStream_t stream, int block_threads, uint64_t tile, int per_lane);
 
+// Blocks per XCD run of a vector-kernel fill (1: blocks in dispatch order).
+uint32_t fill_xcd_group(const DeviceContext& ctx, int format, uint64_t waves, int block_threads, uint64_t tile);
+// Whether the waves of a block of such a fill start their outputs together.
+bool fill_in_step(uint32_t xcd_group, int block_threads, uint64_t tile);
+
 // Batch descriptors (include/mrg8.h): checks a launch configuration; checks
 // `count` descriptors and sums their tiles (of `tile` outputs) and outputs;
 // converts them to the device segment layout (inline states).

@@ -243,3 +243,29 @@ def test_graph_of_each_striding_kernel_is_kept(gpu, oracle_mod):
     b.close()
     for buf in bufs:
         buf.free()
+
+
+@pytest.mark.parametrize("threads,tile,more,pad", [(128, 2048, -1, 0), (512, 2048, 5 * 2048 + 3, 1), (1024, 2048, 1, 127),
+                                                   (256, 8192, 3 * 8192 - 1, 3)])
+def test_fill_blocks_in_step(gpu, oracle_mod, threads, tile, more, pad):
+    """Blocks whose waves wait for one another (64 or more waves of 2048 to 8192
+    doubles per CU), the last block with waves that have no outputs."""
+    import torch
+
+    n = 64 * torch.cuda.get_device_properties(0).multi_processor_count * tile + more
+    say("in step", threads, tile, n, pad)
+    buf = gpu.hip.DeviceBuffer((n + pad) * 8)
+    g = gpu.mrg8_cuda(SEED + threads)
+    g.generate(buf.ptr + 8 * pad, n, 0, block_threads=threads, tile=tile, per_lane=4)
+    gpu.hip.synchronize()
+    state = oracle_mod.seed_state(SEED + threads)
+    for first in (0, tile * (threads // 64) - 200, n // 2, n - 3 * tile - 7):  # windows across waves and blocks
+        count = min(400 if first < n // 2 else 3 * tile + 7, n - first)
+        want, _ = oracle_mod.generate(oracle_mod.jump(state, first), count, 0)
+        got = buf.copy_to_host(np.float64, count, 8 * (pad + first))
+        assert np.array_equal(got.view(np.uint64), want.view(np.uint64)), first
+    got = buf.copy_to_host(np.float64, n, 8 * pad)
+    buf.free()
+    assert oracle_mod.wsum(got) == int(oracle_mod.stream_wsums(state[None], np.zeros(1, np.uint64), np.array([n], np.uint64),
+                                                               np.zeros(1, np.int32))[0])
+    assert np.array_equal(g.get_state(), oracle_mod.jump(state, n))

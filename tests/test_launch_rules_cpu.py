@@ -90,3 +90,23 @@ static void run(const DeviceContext& ctx) {
   CHECK(kernel_of(ctx, 64, 1024 + 700, 10240, 2, 1024, 10240, 4 * 324) == BatchKernel::Striding);
 }
 """)
+
+
+def test_xcd_runs_of_fills(tmp_path):
+    """Only one-wave blocks of up to 1024 doubles run on the XCDs in runs below
+    64 waves per CU; blocks of several waves in such runs start in step."""
+    check(tmp_path, r"""
+static void run(const DeviceContext& ctx) {
+  CHECK(fill_xcd_group(ctx, MRG8_F64, 4096, 64, 1024) == 64);
+  CHECK(fill_xcd_group(ctx, MRG8_F64, 4095, 64, 1024) == 1);
+  CHECK(fill_xcd_group(ctx, MRG8_F64_01, 4096, 64, 65536) == 1);
+  CHECK(fill_xcd_group(ctx, MRG8_F64, 4096, 256, 1024) == 1);
+  CHECK(fill_xcd_group(ctx, MRG8_F64, 16383, 512, 2048) == 1);
+  CHECK(fill_xcd_group(ctx, MRG8_F64, 16384, 512, 2048) == 64);
+  CHECK(fill_xcd_group(ctx, MRG8_F64, 16384, 1024, 2048) == 32);
+  CHECK(fill_xcd_group(ctx, MRG8_U32, 1 << 20, 256, 2048) == 1);
+  CHECK(fill_in_step(64, 512, 2048) && fill_in_step(32, 1024, 8192));
+  CHECK(!fill_in_step(1, 512, 2048) && !fill_in_step(64, 64, 2048));
+  CHECK(!fill_in_step(64, 512, 1024) && !fill_in_step(64, 512, 16384));
+}
+""")
