@@ -136,11 +136,13 @@ typedef struct mrg8_fill_shape {
 /* Autotuner for single-stream fills: times threads-per-block x outputs-per-
  * lane (vector kernel and matrix-core fill) x outputs-per-wave on `device` for
  * fills of about n outputs in
- * `format` (a scratch buffer of n outputs is allocated for the trials) and
- * makes the fastest the default shape of mrg8_generate for that format and
+ * `format` (a scratch buffer of n outputs is allocated for the trials), puts
+ * the fastest in `best` (may be NULL) and, where it is faster than the
+ * automatic shape, makes it the default of mrg8_generate for that format and
  * size class (floor(log2 n)) on that device.  `cache_path` (may be NULL) is a
  * text file of results keyed by device, format and size class; a cached
- * entry is used without timing.  The counterpart of the reference's manual
+ * entry is used without timing (entries of versions that did not time the
+ * automatic shape are not used).  The counterpart of the reference's manual
  * TNUM x BS sweep (cuda/tests/test_mrg8_outer.cu:50-53). */
 int mrg8_tune_fill(int device, int format, uint64_t n, const char* cache_path, mrg8_fill_shape* best);
 

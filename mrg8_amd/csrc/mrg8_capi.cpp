@@ -381,26 +381,25 @@ int fill_mfma(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, void
 int fill_device(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, void* dptr, uint64_t n, int format,
                 hipStream_t stream, int block_threads, uint64_t tile, int per_lane) {
   if (n == 0) return MRG8_OK;
-  const int esz = format_size(format);
-  const int cls = 63 - __builtin_clzll(n);
-  TunedShape tuned;
-  {
+  if (!per_lane) {  // the tuned shape of this size class, where the caller leaves it open
     std::lock_guard<std::mutex> lk(ctx.tuned_mu);
-    tuned = ctx.tuned[format][cls];
-  }
-  // The shape: the caller's, else the tuned one for this size class, else
-  // the default (the matrix-core fill for large word fills, the vector
-  // kernel otherwise).
-  int pl = per_lane;
-  if (!pl) {
+    const TunedShape& tuned = ctx.tuned[format][63 - __builtin_clzll(n)];
     if (tuned.valid) {
-      pl = tuned.per_lane;
+      per_lane = tuned.per_lane;
       if (block_threads <= 0) block_threads = tuned.block_threads;
       if (tile == 0) tile = tuned.tile;
-    } else if (format == MRG8_U32 && n >= kMfmaDefaultMinWords && block_threads <= 0 && tile == 0) {
-      pl = 32;
     }
   }
+  return fill_shaped(ctx, state, offset, dptr, n, format, stream, block_threads, tile, per_lane);
+}
+
+// A fill of n >= 1 outputs in the given shape, 0: automatic (the matrix-core
+// fill for large word fills, the vector kernel otherwise).
+int fill_shaped(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, void* dptr, uint64_t n, int format,
+                hipStream_t stream, int block_threads, uint64_t tile, int per_lane) {
+  const int esz = format_size(format);
+  int pl = per_lane;
+  if (!pl && format == MRG8_U32 && n >= kMfmaDefaultMinWords && block_threads <= 0 && tile == 0) pl = 32;
   if (pl == 16 || pl == 32) {  // the matrix-core fill, columns of 4 pl outputs
     const int column = 4 * pl;
     if (block_threads > 0 && block_threads != 256 && block_threads != 512 && block_threads != 1024)
@@ -966,7 +965,8 @@ std::string fill_key(const DeviceContext& ctx, int format, int cls) {
   hipDeviceProp_t prop;
   (void)hipGetDeviceProperties(&prop, ctx.device);
   char buf[256];
-  std::snprintf(buf, sizeof buf, "%s:%d:fill:fmt%d:n2^%d", prop.gcnArchName, prop.multiProcessorCount, format, cls);
+  // not ":fill:", whose entries come from a sweep without the automatic shape
+  std::snprintf(buf, sizeof buf, "%s:%d:shape:fmt%d:n2^%d", prop.gcnArchName, prop.multiProcessorCount, format, cls);
   std::string k = buf;
   for (char& c : k)
     if (c == ' ') c = '_';
@@ -974,6 +974,25 @@ std::string fill_key(const DeviceContext& ctx, int format, int cls) {
 }
 
 }  // namespace
+
+std::vector<TunedShape> mrg8::fill_candidates(int format) {
+  std::vector<TunedShape> out(1);
+  auto add = [&](int threads, int per_lane, uint64_t tile) { out.push_back({true, threads, per_lane, tile}); };
+  const uint64_t esz = (uint64_t)format_size(format);
+  const int blocks[] = {256, 512, 1024};
+  // vector kernel: 1, 2 or 4 outputs per lane per iteration, four iterations
+  // or more; matrix-core fill: 16 or 32 outputs per lane per tile (columns of
+  // 64 or 128), 64 KiB per wave or less
+  for (int pl : {1, 2, 4})
+    for (int bt : blocks)
+      for (uint64_t tile : {1024, 2048, 4096, 8192, 16384})
+        if (tile >= 64ull * pl * 4) add(bt, pl, tile);
+  for (int pl : {16, 32})
+    for (int bt : blocks)
+      for (uint64_t tile : {2048, 4096, 8192, 16384})
+        if (tile % (64ull * pl) == 0 && tile * esz <= 65536) add(bt, pl, tile);
+  return out;
+}
 
 extern "C" int mrg8_tune_fill(int device, int format, uint64_t n, const char* cache_path, mrg8_fill_shape* best) {
   clear_error();
@@ -985,7 +1004,9 @@ extern "C" int mrg8_tune_fill(int device, int format, uint64_t n, const char* ca
   if (rc) return rc;
   const int cls = 63 - __builtin_clzll(n);
   const std::string key = fill_key(*ctx, format, cls);
+  // an entry's key ends in ":auto" where the automatic shape was as fast
   TunedShape found;
+  bool automatic = false;
   if (cache_path) {
     std::FILE* f = std::fopen(cache_path, "r");
     if (f) {
@@ -994,12 +1015,13 @@ extern "C" int mrg8_tune_fill(int device, int format, uint64_t n, const char* ca
       unsigned long long tile = 0;
       double ms = 0;
       while (std::fscanf(f, "%255s %d %d %llu %lf", k, &bt, &pl, &tile, &ms) == 5)
-        if (key == k && bt >= 64 && bt <= 1024 && bt % 64 == 0 && (pl == 1 || pl == 2 || pl == 4 || pl == 16 || pl == 32) &&
-            tile) {
+        if ((key == k || key + ":auto" == k) && bt >= 64 && bt <= 1024 && bt % 64 == 0 &&
+            (pl == 1 || pl == 2 || pl == 4 || pl == 16 || pl == 32) && tile) {
           found.valid = true;
           found.block_threads = bt;
           found.per_lane = pl;
           found.tile = tile;
+          automatic = key != k;
         }
       std::fclose(f);
     }
@@ -1020,53 +1042,59 @@ extern "C" int mrg8_tune_fill(int device, int format, uint64_t n, const char* ca
     }
     uint32_t st[8];
     seed_state(13579u, st);
+    // ms per fill of `reps` in a row
+    auto measure = [&](const TunedShape& c, int reps) {
+      auto fill = [&] {
+        if (rc == MRG8_OK) rc = fill_shaped(*ctx, st, 0, buf, n, format, nullptr, c.block_threads, c.tile, c.per_lane);
+      };
+      fill();  // warm-up
+      (void)hipEventRecord(e0, nullptr);
+      for (int r = 0; r < reps; ++r) fill();
+      (void)hipEventRecord(e1, nullptr);
+      (void)hipEventSynchronize(e1);
+      float ms = 0;
+      (void)hipEventElapsedTime(&ms, e0, e1);
+      return (double)ms / reps;
+    };
     double best_ms = 1e30;
-    const int blocks[] = {256, 512, 1024};
-    const uint64_t tiles[] = {2048, 4096, 8192, 16384};
-    // vector kernel: 1, 2 or 4 outputs per lane per iteration; matrix-core
-    // fill: 16 or 32 outputs per lane per tile (columns of 64 or 128)
-    const int pls[] = {1, 2, 4, 16, 32};
-    for (int pl : pls) {
-      for (int bt : blocks)
-        for (uint64_t tile : tiles) {
-          if (pl <= 4 ? tile < 64ull * pl * 8 : (bt == 256 || tile % (64ull * pl) || tile * esz > 65536)) continue;
-          rc = fill_device(*ctx, st, 0, buf, n, format, nullptr, bt, tile, pl);  // warm-up
-          if (rc) break;
-          (void)hipEventRecord(e0, nullptr);
-          const int reps = 4;
-          for (int r = 0; r < reps && rc == MRG8_OK; ++r) rc = fill_device(*ctx, st, 0, buf, n, format, nullptr, bt, tile, pl);
-          (void)hipEventRecord(e1, nullptr);
-          (void)hipEventSynchronize(e1);
-          float ms = 0;
-          (void)hipEventElapsedTime(&ms, e0, e1);
-          ms /= reps;
-          if (rc == MRG8_OK && ms < best_ms) {
-            best_ms = ms;
-            found.valid = true;
-            found.block_threads = bt;
-            found.per_lane = pl;
-            found.tile = tile;
-          }
-        }
+    for (const TunedShape& c : fill_candidates(format)) {
+      if (!c.valid) continue;
+      const double ms = measure(c, 4);
       if (rc) break;
+      if (ms < best_ms) {
+        best_ms = ms;
+        found = c;
+      }
+    }
+    // the fastest against the automatic shape in turn, some milliseconds each:
+    // it has to be 2 % faster, more than fills of one shape differ
+    if (rc == MRG8_OK) {
+      const int reps = (int)std::min(200.0, std::max(4.0, 2.0 / best_ms));
+      double auto_ms = 1e30;
+      best_ms = 1e30;
+      for (int round = 0; round < 5; ++round) {
+        auto_ms = std::min(auto_ms, measure(TunedShape{}, reps));
+        best_ms = std::min(best_ms, measure(found, reps));
+      }
+      automatic = best_ms > 0.98 * auto_ms;
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     (void)hipFree(buf);
     (void)hipSetDevice(prev);
     if (rc) return rc;
-    if (cache_path && found.valid) {
+    if (cache_path) {
       std::FILE* f = std::fopen(cache_path, "a");
       if (f) {
-        std::fprintf(f, "%s %d %d %llu %.6f\n", key.c_str(), found.block_threads, found.per_lane,
-                     (unsigned long long)found.tile, best_ms);
+        std::fprintf(f, "%s%s %d %d %llu %.6f\n", key.c_str(), automatic ? ":auto" : "", found.block_threads,
+                     found.per_lane, (unsigned long long)found.tile, best_ms);
         std::fclose(f);
       }
     }
   }
   {
     std::lock_guard<std::mutex> lk(ctx->tuned_mu);
-    ctx->tuned[format][cls] = found;
+    ctx->tuned[format][cls] = automatic ? TunedShape{} : found;
   }
   if (best) {
     best->block_threads = found.block_threads;

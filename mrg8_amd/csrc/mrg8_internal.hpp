@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <mutex>
+#include <vector>
 
 #include "../../include/mrg8.h"
 #include "mrg8_device.hpp"
@@ -69,6 +70,13 @@ int format_size(int format);
 // default.
 int fill_device(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, void* dptr, uint64_t n, int format,
                 hipStream_t stream, int block_threads, uint64_t tile, int per_lane);
+
+// The same without a look at the tuned shapes; n >= 1.
+int fill_shaped(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, void* dptr, uint64_t n, int format,
+                hipStream_t stream, int block_threads, uint64_t tile, int per_lane);
+
+// What mrg8_tune_fill times: the automatic shape (not valid, all 0) first.
+std::vector<TunedShape> fill_candidates(int format);
 
 // Blocks per XCD run of a vector-kernel fill (1: blocks in dispatch order).
 uint32_t fill_xcd_group(const DeviceContext& ctx, int format, uint64_t waves, int block_threads, uint64_t tile);

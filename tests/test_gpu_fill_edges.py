@@ -269,3 +269,24 @@ def test_fill_blocks_in_step(gpu, oracle_mod, threads, tile, more, pad):
     assert oracle_mod.wsum(got) == int(oracle_mod.stream_wsums(state[None], np.zeros(1, np.uint64), np.array([n], np.uint64),
                                                                np.zeros(1, np.int32))[0])
     assert np.array_equal(g.get_state(), oracle_mod.jump(state, n))
+
+
+def test_fill_tuner_cache_entries(gpu, oracle_mod, tmp_path):
+    """Cache entries of a tuned and of the automatic shape are used; those of the
+    sweep that did not time the automatic shape are not."""
+    say("tuner cache")
+    n, cache = 1 << 21, tmp_path / "shapes.txt"
+    gpu.tune_fill(0, n, cache_path=str(cache))
+    key = cache.read_text().split()[0].removesuffix(":auto")
+    old = tmp_path / "old.txt"
+    old.write_text(key.replace(":shape:", ":fill:") + " 1024 1 16384 0.000001\n")
+    assert list(gpu.tune_fill(0, n, cache_path=str(old)).values()) != [1024, 1, 16384]
+    assert len(old.read_text().splitlines()) == 2
+    want, _ = oracle_mod.generate(oracle_mod.seed_state(SEED), n, 0)
+    for suffix in ("", ":auto"):
+        kept = tmp_path / ("kept" + suffix[1:])
+        kept.write_text(f"{key}{suffix} 512 2 4096 0.1\n")
+        assert list(gpu.tune_fill(0, n, cache_path=str(kept)).values()) == [512, 2, 4096]
+        got = run_device(gpu, gpu.mrg8_cuda(SEED), n, 0)
+        assert np.array_equal(got.view(np.uint64), want.view(np.uint64))
+    assert len(kept.read_text().splitlines()) == 1

@@ -110,3 +110,23 @@ static void run(const DeviceContext& ctx) {
   CHECK(!fill_in_step(64, 512, 1024) && !fill_in_step(64, 512, 16384));
 }
 """)
+
+
+def test_fill_tuner_times_the_automatic_shape(tmp_path):
+    """The automatic shape is a candidate, and so are the shapes that large fills of either kernel do best with."""
+    check(tmp_path, r"""
+static void run(const DeviceContext&) {
+  for (int format : {MRG8_F64, MRG8_F64_01, MRG8_U32}) {
+    const std::vector<TunedShape> all = fill_candidates(format);
+    CHECK(!all[0].valid && !all[0].block_threads && !all[0].per_lane && !all[0].tile);
+    bool short_waves = false, small_mfma = false;
+    for (size_t i = 1; i < all.size(); ++i) {
+      const TunedShape& c = all[i];
+      CHECK(c.valid && c.block_threads >= 256 && c.tile);
+      short_waves |= c.block_threads == 256 && c.per_lane == 4 && c.tile == 1024;
+      small_mfma |= c.block_threads == 256 && c.per_lane == 32 && c.tile == 4096;
+    }
+    CHECK(short_waves && small_mfma);
+  }
+}
+""")
