@@ -297,7 +297,7 @@ def bench_batched(args):
     for label, shapes in (("queue_graph", [(512, -2, 2048), (512, -3, 2048), (1024, -1, 2048), (256, -4, 2048)]),
                           ("persistent_graph", [(256, 4, 4096), (256, 8, 4096), (512, 2, 4096), (256, 4, 8192),
                                                 (1024, 1, 4096), (256, 8, 2048)]),
-                          ("tiles_graph", [(1024, 0, 2048)])):
+                          ("tiles_graph", [(256, 0, 2048)])):
         best = None
         for shape in shapes:
             b.set_config(*shape)

@@ -229,7 +229,7 @@ typedef struct mrg8_stream_desc {
 } mrg8_stream_desc;
 
 /* Launch configuration (picked by mrg8_batch_autotune or set by hand; a new
- * batch starts with 1024 threads, one tile per wave, 2048-output tiles; a
+ * batch starts with 256 threads, one tile per wave, 2048-output tiles; a
  * one-tile-per-wave grid runs in blocks of at most 256 threads whatever is
  * asked for). */
 typedef struct mrg8_batch_config {
@@ -279,7 +279,7 @@ int mrg8_batch_autotune(mrg8_batch_t b, void* stream, const char* cache_path, mr
  * reference: for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
  * same generation as mrg8_batch_set + mrg8_batch_run with configuration
- * `cfg` (NULL: the batch default, 1024 threads and one 2048-output tile per
+ * `cfg` (NULL: the batch default, 256 threads and one 2048-output tile per
  * wave): identical outputs, stream-ordered on `stream`.  The batch block
  * (segments, tile prefix sums, tile map) goes to a fixed device scratch area
  * of MRG8_NOALLOC_SCRATCH_BYTES that the library holds on every device it

@@ -11,6 +11,7 @@
 #include <fstream>
 #include <sstream>
 #include <string>
+#include <vector>
 
 #include "../../include/mrg8.h"
 #include "mrg8_internal.hpp"
@@ -28,7 +29,7 @@ struct mrg8_batch {
   // address-order grid takes 2.58 ms, but runs of one batch are serialised,
   // and batches of many short segments with long jumps are faster on a
   // striding grid (mrg8_batch_autotune tries all three)
-  mrg8_batch_config cfg{1024, 0, 2048};
+  mrg8_batch_config cfg = kDefaultBatchConfig;
   // Direct launches by default: on MI355X a replay of the captured one-kernel
   // graph costs ~10 us more per launch than launching the kernel (0.047 ms
   // against 0.037 ms for 65536 jumps + 256 words each).
@@ -228,6 +229,22 @@ void cache_store(const char* path, const std::string& key, const mrg8_batch_conf
 
 }  // namespace
 
+// The counterpart of the reference's manual TNUM x BS sweep
+// (cuda/tests/test_mrg8_outer.cu:50-53).  Waves per CU 0: one tile per wave,
+// in the one block size that such a grid runs in at most; > 0: persistent grid
+// striding over the tiles; < 0: persistent grid taking the tiles in address
+// order.
+std::vector<mrg8_batch_config> mrg8::batch_candidates() {
+  std::vector<mrg8_batch_config> out;
+  for (int threads : {256, 512, 1024})
+    for (int waves_per_cu : {0, 4, 8, 16, 32, -16, -24}) {
+      const int waves = threads / 64;
+      if (waves_per_cu ? waves_per_cu % waves != 0 : threads != kTileBlockThreads) continue;
+      for (uint64_t tile : {2048, 4096, 8192, 16384}) out.push_back({threads, waves_per_cu / waves, tile});
+    }
+  return out;
+}
+
 extern "C" int mrg8_batch_autotune(mrg8_batch_t b, void* stream, const char* cache_path, mrg8_batch_config* best) {
   clear_error();
   if (!b) return fail(MRG8_ERR_ARG, "null batch");
@@ -249,42 +266,31 @@ extern "C" int mrg8_batch_autotune(mrg8_batch_t b, void* stream, const char* cac
     if (e0) (void)hipEventDestroy(e0);
     return hip_fail(ce, "hipEventCreate");
   }
-  // threads-per-block x waves-per-CU x tile size, the counterpart of the
-  // reference's manual TNUM x BS sweep (cuda/tests/test_mrg8_outer.cu:50-53)
-  // waves per CU 0: one tile per wave; > 0: persistent grid striding over
-  // the tiles; < 0: persistent grid taking the tiles in address order
-  const int blocks[] = {256, 512, 1024};
-  const int waves_per_cu[] = {0, 4, 8, 16, 32, -16, -24};
-  const uint64_t tiles[] = {2048, 4096, 8192, 16384};
   double best_ms = 1e30;
   mrg8_batch_config best_cfg = b->cfg;
   int rc = MRG8_OK;
-  for (int bt : blocks)
-    for (int w : waves_per_cu)
-      for (uint64_t t : tiles) {
-        if (rc) break;
-        const mrg8_batch_config c{bt, w / (bt / 64), t};
-        if ((w != 0 && (c.blocks_per_cu == 0 || w % (bt / 64))) || validate_batch_config(c) != MRG8_OK) continue;
-        const uint64_t nt = count_tiles(b->slot.segs(), b->slot.staged_count(), t);
-        if (nt > b->max_tiles) continue;
-        if (w == 0 && (nt + bt / 64 - 1) / (bt / 64) * (uint64_t)bt > 0xffffffffull) continue;  // 32-bit grid
-        if ((rc = mrg8_batch_set_config(b, &c)) != MRG8_OK) break;
-        if ((rc = mrg8_batch_run(b, s)) != MRG8_OK) break;  // warm-up (and capture)
-        hipError_t e = hipEventRecord(e0, s);
-        const int reps = 3;
-        for (int r = 0; r < reps && rc == MRG8_OK; ++r) rc = mrg8_batch_run(b, s);
-        if (e == hipSuccess) e = hipEventRecord(e1, s);
-        if (e == hipSuccess) e = hipEventSynchronize(e1);
-        float ms = 0;
-        if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-        if (rc == MRG8_OK && e != hipSuccess) rc = hip_fail(e, "autotune timing");
-        if (rc) break;
-        ms /= reps;
-        if (ms < best_ms) {
-          best_ms = ms;
-          best_cfg = c;
-        }
-      }
+  for (const mrg8_batch_config& c : batch_candidates()) {
+    const uint64_t wpb = (uint64_t)c.block_threads / 64;
+    const uint64_t nt = count_tiles(b->slot.segs(), b->slot.staged_count(), c.tile_outputs);
+    if (nt > b->max_tiles) continue;
+    if (c.blocks_per_cu == 0 && (nt + wpb - 1) / wpb * (uint64_t)c.block_threads > 0xffffffffull) continue;  // 32-bit grid
+    if ((rc = mrg8_batch_set_config(b, &c)) != MRG8_OK) break;
+    if ((rc = mrg8_batch_run(b, s)) != MRG8_OK) break;  // warm-up (and capture)
+    hipError_t e = hipEventRecord(e0, s);
+    const int reps = 3;
+    for (int r = 0; r < reps && rc == MRG8_OK; ++r) rc = mrg8_batch_run(b, s);
+    if (e == hipSuccess) e = hipEventRecord(e1, s);
+    if (e == hipSuccess) e = hipEventSynchronize(e1);
+    float ms = 0;
+    if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
+    if (rc == MRG8_OK && e != hipSuccess) rc = hip_fail(e, "autotune timing");
+    if (rc) break;
+    ms /= reps;
+    if (ms < best_ms) {
+      best_ms = ms;
+      best_cfg = c;
+    }
+  }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (rc) return rc;

@@ -645,20 +645,21 @@ __device__ __forceinline__ void batch_tile_alone(void* out, uint64_t cnt, uint32
 
 // Batched kernel with one tile per wave (grid = tiles / waves per block):
 // wave 0 of a block looks up and jumps the start states of the block's tiles
-// (8-lane groups; wave 1 too in blocks of more than eight waves) and leaves
-// them in LDS; every wave then generates its own tile and exits.
-__global__ __launch_bounds__(1024) void k_batch_tiles(BatchArgs a) {
-  __shared__ uint32_t start_state[16][8];
-  __shared__ uint64_t start_dst[16], start_cnt[16];
-  __shared__ int32_t start_fmt[16];
+// (8-lane groups) and leaves them in LDS; every wave then generates its own
+// tile and exits.
+__global__ __launch_bounds__(kTileBlockThreads) void k_batch_tiles(BatchArgs a) {
+  constexpr int kWaves = kTileBlockThreads / 64;
+  __shared__ uint32_t start_state[kWaves][8];
+  __shared__ uint64_t start_dst[kWaves], start_cnt[kWaves];
+  __shared__ int32_t start_fmt[kWaves];
   const int lane = threadIdx.x & 63;
   const BatchTables tab = batch_tables(a.block);
   const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t nw = blockDim.x >> 6;
   // < ntiles: the grid covers the tiles exactly
   const uint64_t tile0 = xcd_block(blockIdx.x, gridDim.x, a.xcds, a.xcd_group) * nw;
-  if (wib * 8 < nw) {
-    const uint32_t target = wib * 8 + (lane >> 3);
+  if (wib == 0) {
+    const uint32_t target = lane >> 3;
     const bool mine = target < nw && tile0 + target < tab.ntiles;
     const TileInfo ti = lookup_tile(tab, a, mine ? tile0 + target : tile0);
     const uint32_t s = jump_group(ti.state[lane & 7], mine ? ti.offset : 0, a.digits);
@@ -1540,6 +1541,7 @@ hipError_t launch_stage(const void* src, void* dst, size_t bytes, hipStream_t st
 }
 
 hipError_t launch_batch_tiles(const BatchArgs& a, uint64_t ntiles, int block_threads, hipStream_t stream) {
+  if (block_threads > kTileBlockThreads) return hipErrorInvalidConfiguration;
   const uint64_t wpb = (uint64_t)block_threads / 64;
   const uint64_t blocks = (ntiles + wpb - 1) / wpb;
   if (blocks == 0) return hipSuccess;

@@ -29,6 +29,12 @@ constexpr int kPositionInts = (kJumpValues + 1) * kJumpMatrixInts;
 // bounds within 64 bits.
 constexpr uint64_t kMaxTile = 1ull << 40;
 
+// Threads per block of a one-tile-per-wave grid, at most.  Larger blocks wait
+// for their slowest wave before the next block starts: 4096 streams of uneven
+// length 2.68 ms at 256, 2.70 ms at 512 and 2.76 ms at 1024; 65536 jumps and
+// 256 words each 74 and 81 us at 256 and 1024.
+constexpr int kTileBlockThreads = 256;
+
 // Per-device constant tables.
 struct DeviceTables {
   CoefRecord* lane = nullptr;  // kLaneRows records: row 0 of A^(k+1), support 0xff

@@ -40,12 +40,14 @@ inline uint32_t xcd_run_blocks(const DeviceContext& ctx, int block_threads) {
   return run;
 }
 
-// Threads per block of a one-tile-per-wave grid: at most 256 of the
-// configured ones.  Larger blocks wait for their slowest wave before the next
-// block starts: 4096 streams of uneven length 2.68 ms at 256, 2.70 ms at 512
-// and 2.76 ms at 1024; 65536 jumps and 256 words each 74 and 81 us at 256 and
-// 1024.
-inline int tile_block_threads(int block_threads) { return std::min(block_threads, 256); }
+// Threads per block of a one-tile-per-wave grid with these configured ones.
+inline int tile_block_threads(int block_threads) { return std::min(block_threads, kTileBlockThreads); }
+
+// A new batch's launch configuration.
+constexpr mrg8_batch_config kDefaultBatchConfig{kTileBlockThreads, 0, 2048};
+
+// What mrg8_batch_autotune times: threads per block x waves per CU x tile size.
+std::vector<mrg8_batch_config> batch_candidates();
 
 // Builds the table of byte positions kJumpPositions..kWidePositions-1 on the
 // context's device if it is not there yet.

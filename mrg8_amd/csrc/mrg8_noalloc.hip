@@ -54,7 +54,7 @@ extern "C" int mrg8_batch_generate_noalloc(int device, const mrg8_stream_desc* d
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return fail(MRG8_ERR_NODEVICE, "no HIP device available");
   if (device < 0 || device >= ndev) return fail(MRG8_ERR_ARG, "device %d out of range (have %d)", device, ndev);
-  const mrg8_batch_config c = cfg ? *cfg : mrg8_batch_config{1024, 0, 2048};
+  const mrg8_batch_config c = cfg ? *cfg : kDefaultBatchConfig;
   int rc = validate_batch_config(c);
   if (rc) return rc;
   uint64_t tiles = 0, total = 0;

@@ -85,7 +85,7 @@ def main():
                for i in range(len(lengths))])
         # the batch default (one tile per wave), then the persistent grid that
         # takes the tiles in address order
-        for shape in ((1024, 0, 2048), (512, -2, 2048)):
+        for shape in ((256, 0, 2048), (512, -2, 2048)):
             b.set_config(*shape)
             for _ in range(args.warmup + args.reps):
                 b.run()

@@ -290,3 +290,26 @@ def test_fill_tuner_cache_entries(gpu, oracle_mod, tmp_path):
         got = run_device(gpu, gpu.mrg8_cuda(SEED), n, 0)
         assert np.array_equal(got.view(np.uint64), want.view(np.uint64))
     assert len(kept.read_text().splitlines()) == 1
+
+
+@pytest.mark.parametrize("threads", [None, 64, 128, 192, 256, 320, 1024])
+def test_tile_per_wave_block_sizes(gpu, oracle_mod, threads):
+    """One tile per wave in every size of block, a last block with idle waves;
+    a new batch says the block size that it runs in."""
+    tiles = 4 * 7 + 1
+    n = tiles * 256 - 9
+    buf = gpu.hip.DeviceBuffer(n * 8)
+    b = gpu.Batch(1, tiles + 1)
+    assert b.config == {"block_threads": 256, "blocks_per_cu": 0, "tile_outputs": 2048}
+    if threads:
+        b.set_config(threads, 0, 256)
+        assert b.config["block_threads"] == threads
+    b.set([(oracle_mod.seed_state(SEED), 1 << 20, n, buf.ptr, 0)])
+    say("tile per wave", threads)
+    buf.fill_byte(0xA5)
+    b.run()
+    gpu.hip.synchronize()
+    want, _ = oracle_mod.generate(oracle_mod.jump(oracle_mod.seed_state(SEED), 1 << 20), n, 0)
+    assert np.array_equal(buf.copy_to_host(np.uint64, n), want.view(np.uint64))
+    b.close()
+    buf.free()

@@ -130,3 +130,23 @@ static void run(const DeviceContext&) {
   }
 }
 """)
+
+
+def test_batch_tuner_times_no_launch_twice(tmp_path):
+    """Candidates are valid and their launches differ; a one-tile-per-wave grid says the block size that it runs in,
+    and so does the configuration of a new batch."""
+    check(tmp_path, r"""
+static void run(const DeviceContext&) {
+  const std::vector<mrg8_batch_config> all = batch_candidates();
+  bool kinds[3] = {};
+  for (size_t i = 0; i < all.size(); ++i) {
+    const mrg8_batch_config& c = all[i];
+    CHECK(validate_batch_config(c) == MRG8_OK);
+    CHECK(c.blocks_per_cu || tile_block_threads(c.block_threads) == c.block_threads);
+    for (size_t j = 0; j < i; ++j) CHECK(std::memcmp(&all[j], &c, sizeof c) != 0);
+    kinds[(c.blocks_per_cu > 0) - (c.blocks_per_cu < 0) + 1] = true;
+  }
+  CHECK(kinds[0] && kinds[1] && kinds[2]);
+  CHECK(tile_block_threads(kDefaultBatchConfig.block_threads) == kDefaultBatchConfig.block_threads);
+}
+""")
