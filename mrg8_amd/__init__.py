@@ -51,20 +51,21 @@ def _bits200(bits) -> "ctypes.Array":
 
 
 def _ptr(p) -> int:
-    data_ptr = getattr(p, "data_ptr", None)
-    if data_ptr is not None:
-        return data_ptr()  # torch tensor
-    if hasattr(p, "ptr"):
-        return int(p.ptr)  # mrg8_amd.hip.DeviceBuffer
-    return int(p)
+    # int: an address of another integer type, which ctypes takes for no pointer
+    try:
+        data_ptr = p.data_ptr  # torch tensor
+    except AttributeError:
+        return int(p.ptr if hasattr(p, "ptr") else p)  # mrg8_amd.hip.DeviceBuffer
+    return int(data_ptr())
 
 
 def _stream(s):
     if s is None:
         return None
-    stream = getattr(s, "cuda_stream", None)
-    if stream is not None:
-        return stream  # torch.cuda.Stream
+    try:
+        return int(s.cuda_stream)  # torch.cuda.Stream
+    except AttributeError:
+        pass
     if hasattr(s, "handle"):
         return ctypes.c_void_p(s.handle)
     return int(s)

@@ -1,4 +1,7 @@
-"""The forms a state can be passed in, and host jumps by bytes of the step."""
+"""The forms a state, an address and a stream can be passed in, and host jumps by bytes of the step."""
+import ctypes
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -25,3 +28,20 @@ def test_bad_states_are_refused(bad):
 @pytest.mark.parametrize("state", [WORDS, [0] * 8, [P] * 8, [0, 0, 0, 0, 0, 0, 0, 9], [0, 3, 0, 0, 0, 0, 0, 0]])
 def test_host_jump_bytes(step, state, oracle_mod):
     assert mrg8_amd.advance_state(state, step).tolist() == oracle_mod.jump(np.array(state, np.uint32), step).tolist()
+
+
+@pytest.mark.parametrize("address", [0, 4096, np.int64(1 << 40), np.uint64(2**64 - 4096)])
+def test_addresses_and_streams_of_any_integer_type(address):
+    want = ctypes.c_void_p(int(address)).value
+    for p in (SimpleNamespace(data_ptr=lambda: address), SimpleNamespace(ptr=address), address):
+        assert ctypes.c_void_p(mrg8_amd._ptr(p)).value == want
+    for s in (SimpleNamespace(cuda_stream=address), SimpleNamespace(handle=int(address)), address):
+        got = mrg8_amd._stream(s)
+        assert (got if isinstance(got, ctypes.c_void_p) else ctypes.c_void_p(got)).value == want
+    assert mrg8_amd._stream(None) is None
+
+
+@pytest.mark.parametrize("bad", [None, "0", SimpleNamespace(data_ptr=lambda: None), SimpleNamespace(cuda_stream=None)])
+def test_what_is_no_address_is_refused(bad):
+    with pytest.raises((TypeError, ValueError)):
+        ctypes.c_void_p(mrg8_amd._ptr(bad)).value + 0
