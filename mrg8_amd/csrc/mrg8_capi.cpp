@@ -257,7 +257,7 @@ int format_size(int format) {
 // 512 outputs are faster (2^20: 4.65 against 4.8 us).  Words below the
 // matrix-core fill's sizes: 256-thread blocks, down to 1024 outputs per wave
 // while that leaves fewer than four waves per SIMD (2^20: 4.4 us, 512 per
-// wave 4.6 us).
+// wave 4.6 us).  2048 doubles per wave where the grid would be too large.
 void default_shape(const DeviceContext& ctx, uint64_t n, int format, int per_lane, int* block, uint64_t* tile) {
   const uint64_t quantum = 64ull * per_lane;
   const uint64_t cu = (uint64_t)ctx.num_cu;
@@ -267,9 +267,35 @@ void default_shape(const DeviceContext& ctx, uint64_t n, int format, int per_lan
     while (t > 4 * quantum && (n + t - 1) / t < cu * 16) t /= 2;  // four waves per SIMD
   } else if ((n + t - 1) / t <= cu * 4) {
     t = 512;
+  } else if (n / t + 2 > kMaxGridWaves) {
+    t = 2048;
   }
   *tile = std::max<uint64_t>(quantum, t / quantum * quantum);
   *block = format == MRG8_U32 ? 256 : 64;
+}
+
+// Tiles per wave of a matrix-core fill by default.  Doubles: 32 KiB of output
+// per wave, fewer tiles when that would leave fewer than 8 waves per CU.
+// Words: 4 tiles (of 2048) per wave, fewer while at most 12 waves per CU hold
+// the fill (16 fit the LDS), and two, in XCD runs of 16 blocks (1 MiB), from 32
+// such waves per CU on, unless the grid would be too large (2^38 words).
+// us with 1 | 2 | 4 tiles in dispatch order | 2 in runs of 16:
+//   2^22.6 words (12 tiles per CU)  8.5 |   8.7 |   9.2 |   8.9
+//   2^23                           10.4 |   9.7 |   9.9 |  10.1
+//   2^24                           15.9 |  16.2 |  15.1 |  16.4
+//   2^24.6                         22.3 |  23.2 |  21.1 |  22.4
+//   2^25 (64 tiles per CU)         28.0 |  29.3 |  27.2 |  27.1
+//   2^26                           53.9 |  56.3 |  50.7 |  48.9
+//   2^28                           209  |   206 |   190 |   174
+// (512-thread blocks of 4 tiles: 2^26 48.9, 2^28 181.)
+uint64_t mfma_tiles_per_wave(const DeviceContext& ctx, int format, uint64_t tile, uint64_t tiles) {
+  const uint64_t cu = (uint64_t)ctx.num_cu, esz = (uint64_t)format_size(format);
+  const uint64_t most = std::max<uint64_t>(1, 32768 / esz / tile);
+  if (format != MRG8_U32) return std::min(most, tiles / (8 * cu));
+  if (tiles <= 12 * cu) return 1;
+  if (tiles <= 24 * cu) return 2;
+  const uint64_t half = std::max<uint64_t>(1, 16384 / esz / tile);
+  return tiles >= 64 * cu && tiles / half + 8 <= kMaxGridWaves ? half : most;
 }
 
 // Blocks per XCD run of a vector-kernel fill (1: blocks in dispatch order).
@@ -303,7 +329,7 @@ namespace {
 
 // Matrix-core fill of n outputs: whole tiles of 16 x `column` outputs from
 // the first 1 KiB boundary of dptr on, `outputs_per_wave` / tile consecutive
-// tiles per wave (0: 32 KiB of output) in blocks of `block_threads` (0:
+// tiles per wave (0: mfma_tiles_per_wave) in blocks of `block_threads` (0:
 // the format's default), the outputs before the first tile and after the last
 // by two extra waves.  Returns MRG8_ERR_STATE (and launches nothing) when the
 // fill has no whole tile or the state is all zero: the caller takes the
@@ -327,27 +353,7 @@ int fill_mfma(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, void
   a.tiles = tiles;
   a.column = (uint32_t)column;
   a.waves_per_block = (uint32_t)(block_threads ? block_threads / 64 : format == MRG8_U32 ? 4 : 16);
-  // Default, doubles: 32 KiB of output per wave, fewer tiles when that would
-  // leave fewer than 8 waves per CU.  Words: 4 tiles (of 2048) per wave, fewer
-  // while at most 12 waves per CU hold the fill (16 fit the LDS), and two, in
-  // XCD runs of 16 blocks (1 MiB), from 32 such waves per CU on.
-  // us with 1 | 2 | 4 tiles in dispatch order | 2 in runs of 16:
-  //   2^22.6 words (12 tiles per CU)  8.5 |   8.7 |   9.2 |   8.9
-  //   2^23                           10.4 |   9.7 |   9.9 |  10.1
-  //   2^24                           15.9 |  16.2 |  15.1 |  16.4
-  //   2^24.6                         22.3 |  23.2 |  21.1 |  22.4
-  //   2^25 (64 tiles per CU)         28.0 |  29.3 |  27.2 |  27.1
-  //   2^26                           53.9 |  56.3 |  50.7 |  48.9
-  //   2^28                           209  |   206 |   190 |   174
-  // (512-thread blocks of 4 tiles: 2^26 48.9, 2^28 181.)
-  const uint64_t cu = (uint64_t)ctx.num_cu;
-  const bool long_words = format == MRG8_U32 && tiles >= 64 * cu;
-  uint64_t per = format != MRG8_U32 ? std::min<uint64_t>(32768 / (uint64_t)esz / tile, tiles / (8 * cu))
-                 : long_words       ? 16384 / (uint64_t)esz / tile
-                 : tiles <= 12 * cu ? 1
-                 : tiles <= 24 * cu ? 2
-                                    : 32768 / (uint64_t)esz / tile;
-  if (outputs_per_wave) per = outputs_per_wave / tile;
+  const uint64_t per = outputs_per_wave ? outputs_per_wave / tile : mfma_tiles_per_wave(ctx, format, tile, tiles);
   a.tiles_per_wave = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(per, 1), 1u << 20);
   a.waves = (tiles + a.tiles_per_wave - 1) / a.tiles_per_wave;
   a.xcds = (uint32_t)ctx.num_xcc;

@@ -80,6 +80,13 @@ int fill_shaped(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, vo
 // What mrg8_tune_fill times: the automatic shape (not valid, all 0) first.
 std::vector<TunedShape> fill_candidates(int format);
 
+// A grid's work-items are a 32-bit quantity.
+constexpr uint64_t kMaxGridWaves = 0xffffffffull / 64;
+
+// Automatic shapes: threads per block and outputs per wave of the vector
+// kernel, and tiles (of `tile` outputs) per wave of the matrix-core fill.
+void default_shape(const DeviceContext& ctx, uint64_t n, int format, int per_lane, int* block, uint64_t* tile);
+uint64_t mfma_tiles_per_wave(const DeviceContext& ctx, int format, uint64_t tile, uint64_t tiles);
 // Blocks per XCD run of a vector-kernel fill (1: blocks in dispatch order).
 uint32_t fill_xcd_group(const DeviceContext& ctx, int format, uint64_t waves, int block_threads, uint64_t tile);
 // Whether the waves of a block of such a fill start their outputs together.

@@ -150,3 +150,28 @@ static void run(const DeviceContext&) {
   CHECK(tile_block_threads(kDefaultBatchConfig.block_threads) == kDefaultBatchConfig.block_threads);
 }
 """)
+
+
+def test_largest_fills_fit_the_grid(tmp_path):
+    """Fills of up to 2^37 doubles and 2^39 words (into mapped host memory, say) stay within a grid's 2^32 - 1
+    work-items; the shapes up to there are the measured ones."""
+    check(tmp_path, r"""
+static void run(const DeviceContext& ctx) {
+  for (uint64_t n : {1ull << 28, (1ull << 36) - 4096, 1ull << 36, (1ull << 37) - (1ull << 20)})
+    for (int format : {MRG8_F64, MRG8_F64_01}) {
+      int block = 0;
+      uint64_t tile = 0;
+      default_shape(ctx, n, format, 4, &block, &tile);
+      CHECK(block == 64 && fill_waves(n, 127, tile) * 64 <= 0xffffffffull);
+      CHECK(tile == (n < 1ull << 36 ? 1024u : 2048u));
+    }
+  for (uint64_t n : {1ull << 28, 1ull << 37, (1ull << 38) + 4096, (1ull << 39) - (1ull << 20)}) {
+    const uint64_t tiles = n / 2048, per = mfma_tiles_per_wave(ctx, MRG8_U32, 2048, tiles);
+    CHECK(((tiles + per - 1) / per + 2 + 3) / 4 * 256 <= 0xffffffffull);
+    CHECK(per == (n <= 1ull << 37 ? 2u : 4u));
+  }
+  CHECK(mfma_tiles_per_wave(ctx, MRG8_U32, 2048, 12 * 256) == 1 && mfma_tiles_per_wave(ctx, MRG8_U32, 2048, 12 * 256 + 1) == 2);
+  CHECK(mfma_tiles_per_wave(ctx, MRG8_U32, 2048, 24 * 256 + 1) == 4 && mfma_tiles_per_wave(ctx, MRG8_U32, 2048, 64 * 256) == 2);
+  CHECK(mfma_tiles_per_wave(ctx, MRG8_U32, 1024, 64 * 256) == 4 && mfma_tiles_per_wave(ctx, MRG8_F64, 1024, 1 << 18) == 4);
+}
+""")
