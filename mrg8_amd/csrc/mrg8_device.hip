@@ -1082,6 +1082,16 @@ __device__ __forceinline__ uint32_t mfma_stride_residue(const v4i_t (&acc)[kMfma
   return min(x, x - kP);
 }
 
+// Between a wave's writes to LDS and its lanes' reads of one another's words,
+// and between those reads and the next writes.  A wave's LDS operations take
+// effect in the order of the program; this keeps the compiler to that order
+// and is no instruction.
+__device__ __forceinline__ void wave_lds_handover() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // The tiles [t0, t0 + nt) of a matrix-core fill with columns of COL outputs,
 // made by one wave with the LDS area st (kMfmaColumns * (COL + 4) words: the
 // 4-word pad spreads the columns over the LDS banks).
@@ -1182,6 +1192,7 @@ __device__ __forceinline__ void mfma_tiles(const MfmaFillArgs& a, uint64_t t0, u
     }
     // this tile's slice of every store: tile outputs ch E + kPer lane .. + kPer - 1
     // (E = 1024 / sizeof(T) per store), within one column
+    wave_lds_handover();
 #pragma unroll
     for (int ch = 0; ch < kChunks; ++ch) {
       const uint32_t pos = ch * (1024 / (int)sizeof(T)) + kPer * lane;
@@ -1194,6 +1205,7 @@ __device__ __forceinline__ void mfma_tiles(const MfmaFillArgs& a, uint64_t t0, u
         pend[2 * ch] = v.x; pend[2 * ch + 1] = v.y;
       }
     }
+    wave_lds_handover();
     pend_base = static_cast<T*>(a.out) + a.head + (t0 + t) * kTile;
   }
 #pragma unroll
@@ -1380,6 +1392,7 @@ __global__ __launch_bounds__(64) void k_batch_short(BatchArgs a) {
       }
       // the next group's jumps before this run's stores: they would wait for them
       if (done == 0 && nnext) sn = jump_group(sn, grp < nnext ? tn.offset : 0, a.digits);
+      wave_lds_handover();
       if (plain) {
         switch (fmt) {
           case 0: store_runs<0>(ti, ngrp, done, stage); break;
@@ -1400,6 +1413,7 @@ __global__ __launch_bounds__(64) void k_batch_short(BatchArgs a) {
           }
         }
       }
+      wave_lds_handover();
       done += 2 * kShortRun;
       if (done >= most) break;
       // every column is at its other half's end of this run: A^128 once more
