@@ -280,7 +280,8 @@ inline bool jump_matrix_entries(const uint32_t* m, int32_t* out) {
 //   t0 = beta + (D & 0xffff), u0 = beta + (D >> 16),
 //   c_0 = t0 & 0xff, c_1 = t0 >> 8, c_2 = u0 & 0xff, c_3 = u0 >> 8.
 // The kernel then reduces x = t + ((u << 16) & p) + (u >> 15) (2^16 u mod p
-// is a 31-bit rotation of u), x < 2 p.
+// is a 31-bit rotation of u), x < 2 p, in the form of mfma_step_residue, for
+// which it doubles c_2 and takes class 2's product twice.
 //
 // Stride tables: A^steps in the same digit form, row 4 g + i (i < 2) giving
 // new word W(g) + i (oldest first), rows with i >= 2 zero, so that the new

@@ -5,9 +5,9 @@
 // v_mfma_i32_16x16x32_i8 as the kernel uses them (lane l = n + 16 g holds
 // K-group g of row/column n; result register i of lane l is row 4 g + i of
 // column n): the first tile's column states through the fan-out records,
-// each step from accumulators started at the step constants, the combine
-// exactly as the kernel writes it in 32/64-bit unsigned arithmetic, the
-// state hand-off between steps in registers 2 and 3, and the stride product
+// each step from accumulators started at the step constants, a combine of
+// them in 32/64-bit unsigned arithmetic (the kernel's own, in fewer
+// operations, is replayed in mfma_step_emul.cpp), the state hand-off between steps in registers 2 and 3, and the stride product
 // that gives the column states of the wave's next tile.  Tiles 0, W and 2 W
 // of a wave are compared with the oracle's serial generator
 // (oracle/mrg8_oracle.c, original/mrg8.cpp's randint) for several strides W
