@@ -187,12 +187,12 @@ __device__ __forceinline__ int32_t apply_rows4(const JumpRow m[4], uint32_t half
 
 // Jumps eight states at once: this lane's group of eight holds one state (word
 // s of it here) and its own 64-bit offset.  The rows of all of an offset's
-// digits are independent loads: AHEAD of them are in flight, so a jump does not
+// digits are independent loads: four of them are in flight, so a jump does not
 // wait for memory once per digit.  65536 random 63-bit jumps and 256 words
 // each: 25.5 us, 27.4 us with 48-byte records fetched one digit ahead and
 // words gathered through LDS swizzles; one tile per wave 73 against 104 us.
-template <int AHEAD = 4>
 __device__ __forceinline__ uint32_t jump_group(uint32_t s, uint64_t off, const int32_t* __restrict__ digits) {
+  constexpr int kAhead = 4;
   if (!__ballot(off != 0)) return s;
   const uint32_t lo = (uint32_t)off, hi = (uint32_t)(off >> 32);
   const bool more = __ballot(hi != 0u);
@@ -200,9 +200,9 @@ __device__ __forceinline__ uint32_t jump_group(uint32_t s, uint64_t off, const i
     return load_row(digits + k * kPositionInts + digit_of(k < 4 ? lo : hi, k) * kJumpMatrixInts + 4 * (threadIdx.x & 7));
   };
   // issued before the state is looked at, which may still be on its way
-  JumpRow m[AHEAD];
+  JumpRow m[kAhead];
 #pragma unroll
-  for (int k = 0; k < AHEAD; ++k) m[k] = row(k);
+  for (int k = 0; k < kAhead; ++k) m[k] = row(k);
   if (__ballot(s == 0u)) {
 #pragma unroll 1
     for (int k = 0; k < kJumpPositions; ++k) {
@@ -215,8 +215,8 @@ __device__ __forceinline__ uint32_t jump_group(uint32_t s, uint64_t off, const i
 #pragma unroll
   for (int k = 0; k < kJumpPositions; ++k) {
     if (k == 4 && !more) break;
-    if (__ballot(digit_of(k < 4 ? lo : hi, k) != 0u)) e = jump_row(m[k % AHEAD], e);
-    if (k + AHEAD < 4 || (k + AHEAD < kJumpPositions && more)) m[k % AHEAD] = row(k + AHEAD);
+    if (__ballot(digit_of(k < 4 ? lo : hi, k) != 0u)) e = jump_row(m[k % kAhead], e);
+    if (k + kAhead < 4 || (k + kAhead < kJumpPositions && more)) m[k % kAhead] = row(k + kAhead);
   }
   return word_of(e);
 }
@@ -857,7 +857,7 @@ __global__ __launch_bounds__(4 * kAdvanceGroups) void k_advance_lds(AdvanceArgs 
   uint32_t* const out = a.out + 8 * first;
   const uint32_t* const offs = reinterpret_cast<const uint32_t*>(a.offsets) + first * halves;
   auto state = [&](int g) { return min(grp + kAdvanceGroups * g, count - 1); };  // past the end: the last one again
-  // copies position k's matrices to LDS, 8 KiB per wave
+  // copies position k's matrices to LDS, 4 KiB per wave
   auto stage = [&](int k, int32_t* table) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int kInts = kPositionInts / (kThreads / 64);
@@ -1325,7 +1325,7 @@ __global__ __launch_bounds__(64) void k_batch_short(BatchArgs a) {
   // Full rounds of one group a wave, then one of as many waves as there are
   // full groups left, but enough of them to reach every SIMD (65536 x 16 words
   // 16.2 us; with equal rounds of fewer waves, uneven over the SIMDs, 17.7).
-  const uint32_t waves = gridDim.x, wave = (uint32_t)xcd_block(blockIdx.x, gridDim.x, a.xcds, a.xcd_group);
+  const uint32_t waves = gridDim.x, wave = blockIdx.x;
   const uint64_t round = (uint64_t)kShortGroup * waves, rounds = ntiles / round;
   const uint32_t last = (uint32_t)(ntiles - rounds * round);  // its tiles
   const uint32_t last_waves = max((last + kShortGroup - 1) / kShortGroup, min(a.min_waves, min(last, waves)));

@@ -37,7 +37,7 @@ constexpr int kTileBlockThreads = 256;
 
 // Per-device constant tables.
 struct DeviceTables {
-  CoefRecord* lane = nullptr;  // kLaneRows records: row 0 of A^(k+1), support 0xff
+  CoefRecord* lane = nullptr;  // kLaneRows records: row 0 of A^(k+1)
   // Jump matrices: A^(d 2^(kJumpBits k)) at k kPositionInts + d
   // kJumpMatrixInts, byte positions k = 0..kJumpPositions-1
   const int32_t* digits = nullptr;
@@ -248,7 +248,7 @@ hipError_t launch_batch(const BatchArgs& a, int grid, int block_threads, hipStre
 // Persistent grid of `waves` one-wave blocks for short tiles.
 hipError_t launch_batch_short(const BatchArgs& a, uint32_t waves, hipStream_t stream);
 // Persistent grid of `grid` blocks taking groups of (waves per block)
-// consecutive tiles, in address order, from the counters in the batch
+// consecutive tiles, in address order, from the counter in the batch
 // block's header.  Launches of one batch block must not overlap.
 hipError_t launch_batch_queue(const BatchArgs& a, int grid, int block_threads, hipStream_t stream);
 // One tile per wave: ceil(ntiles / waves per block) blocks.

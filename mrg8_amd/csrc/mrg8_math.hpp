@@ -179,16 +179,15 @@ inline std::vector<uint32_t> block_rows(int count) {
 //                                  + (2^30 sum_j c_j mod p) - 1
 // so V is in (0, 2^64) and V + 1 == dot(row, s) (mod p).  The canonical
 // residue r of V gives the reference's word directly as r + 1, in [1, p]
-// (a residue of 0 becomes p), except when the exact sum is 0: that happens
-// exactly when every word of s under a non-zero entry of the row is 0
-// (`support` marks the non-zero entries), and the word is then 0.
+// (a residue of 0 becomes p), except when the exact sum is 0: records are for
+// rows without a zero entry (all_nonzero), so that happens for the all-zero
+// state alone.
 constexpr uint32_t kCenter = 1u << 30;
 
 struct CoefRecord {   // 48 bytes, the layout the kernels read
   int32_t c[8];
   uint32_t b0_lo, b0_hi;
-  uint32_t support;  // bit j set when entry j is non-zero as an integer
-  uint32_t pad;
+  uint32_t pad[2];
 };
 static_assert(sizeof(CoefRecord) == 48, "record layout");
 
@@ -207,10 +206,6 @@ inline CoefRecord make_record(const uint32_t row[8]) {
   uint64_t b0 = base + k - 1;
   rec.b0_lo = (uint32_t)b0;
   rec.b0_hi = (uint32_t)(b0 >> 32);
-  rec.support = 0;
-  for (int j = 0; j < 8; ++j)
-    if (row[j] != 0) rec.support |= 1u << j;
-  rec.pad = 0;
   return rec;
 }
 

@@ -169,7 +169,7 @@ BatchKernel batch_kernel(const DeviceContext& ctx, const LaunchConfig& cfg, cons
   return ctx.tables.mfma_a && many && is_short && even ? BatchKernel::Short : BatchKernel::Striding;
 }
 
-hipError_t launch_batch_kernel(const DeviceContext& ctx, BatchArgs a, const LaunchConfig& cfg, BatchKernel kernel,
+hipError_t launch_batch_kernel(const DeviceContext& ctx, const BatchArgs& a, const LaunchConfig& cfg, BatchKernel kernel,
                                uint64_t ntiles, hipStream_t stream) {
   switch (kernel) {
     case BatchKernel::Tiles: return launch_batch_tiles(a, ntiles, tile_block_threads(cfg.block_threads), stream);
@@ -179,7 +179,6 @@ hipError_t launch_batch_kernel(const DeviceContext& ctx, BatchArgs a, const Laun
       // at most the three waves per SIMD that its registers allow: what a
       // larger grid costs to start is not hidden (65536 x 256 words, 12 waves
       // per CU 20.9 us, 8 22.5, 16 24.6)
-      a.xcd_group = xcd_run_blocks(ctx, 64);
       return launch_batch_short(a, (uint32_t)(ctx.num_cu * std::min(12, cfg.blocks_per_cu * (cfg.block_threads / 64))), stream);
   }
   return hipErrorInvalidValue;
@@ -246,7 +245,7 @@ int BatchSlot::run(const LaunchConfig& cfg, hipStream_t stream, bool graph, bool
     if ((work_.tiles + wpb - 1) / wpb * (uint64_t)cfg.block_threads > 0xffffffffull)
       return fail(MRG8_ERR_CAPACITY, "%llu tiles need more than 2^32 - 1 work-items at one tile per wave; use larger "
                   "tiles or a persistent grid", (unsigned long long)work_.tiles);
-  } else if (cfg.blocks_per_cu < 0) {  // the work counter is 32 bits: groups plus one last take per block
+  } else if (cfg.blocks_per_cu < 0) {  // a group's number, the grid's blocks plus the work counter, is 32 bits
     if ((work_.tiles + wpb - 1) / wpb + (uint64_t)ctx_->num_cu * (uint64_t)-cfg.blocks_per_cu > 0xffffffffull)
       return fail(MRG8_ERR_CAPACITY, "%llu tiles are more groups than the address-order grid counts; use larger tiles",
                   (unsigned long long)work_.tiles);

@@ -53,7 +53,7 @@ size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t 
 enum class BatchKernel { Tiles, Queue, Striding, Short };
 BatchKernel batch_kernel(const DeviceContext& ctx, const LaunchConfig& cfg, const BatchWork& work);
 BatchArgs batch_args(const DeviceContext& ctx, const uint8_t* block, const LaunchConfig& cfg, const uint32_t* states);
-hipError_t launch_batch_kernel(const DeviceContext& ctx, BatchArgs a, const LaunchConfig& cfg, BatchKernel kernel,
+hipError_t launch_batch_kernel(const DeviceContext& ctx, const BatchArgs& a, const LaunchConfig& cfg, BatchKernel kernel,
                                uint64_t ntiles, hipStream_t stream);
 
 class BatchSlot {

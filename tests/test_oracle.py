@@ -347,7 +347,7 @@ def test_wide_jump_matrices_have_no_zero_entries(oracle_mod):
     """A^(d 256^k) for byte positions k = 8..31 (the device's table for
     offsets past 64 bits) has no entry equal to 0 mod p, so the exact-zero
     case of bigDotProd (original/mrg8.cpp:72-82) depends only on the state's
-    zero words there, as the device's support masks assume."""
+    zero words there, as the device's jumps assume."""
     p = 2**31 - 1
     c = [int(x) for x in oracle_mod.coeffs()]
     a = [c] + [[1 if j == r - 1 else 0 for j in range(8)] for r in range(1, 8)]
