@@ -52,20 +52,20 @@ def _bits200(bits) -> "ctypes.Array":
 
 def _ptr(p) -> int:
     # int: an address of another integer type, which ctypes takes for no pointer
-    try:
-        data_ptr = p.data_ptr  # torch tensor
-    except AttributeError:
-        return int(p.ptr if hasattr(p, "ptr") else p)  # mrg8_amd.hip.DeviceBuffer
-    return int(data_ptr())
+    data_ptr = getattr(p, "data_ptr", None)  # no try: an AttributeError costs a microsecond
+    if data_ptr is not None:
+        return int(data_ptr())  # torch tensor
+    if hasattr(p, "ptr"):
+        return int(p.ptr)  # mrg8_amd.hip.DeviceBuffer
+    return int(p)
 
 
 def _stream(s):
     if s is None:
         return None
-    try:
-        return int(s.cuda_stream)  # torch.cuda.Stream
-    except AttributeError:
-        pass
+    stream = getattr(s, "cuda_stream", None)
+    if stream is not None:
+        return int(stream)  # torch.cuda.Stream
     if hasattr(s, "handle"):
         return ctypes.c_void_p(s.handle)
     return int(s)
