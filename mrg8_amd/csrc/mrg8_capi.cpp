@@ -258,20 +258,32 @@ int format_size(int format) {
 // matrix-core fill's sizes: 256-thread blocks, down to 1024 outputs per wave
 // while that leaves fewer than four waves per SIMD (2^20: 4.4 us, 512 per
 // wave 4.6 us).  2048 doubles per wave where the grid would be too large.
+// A caller's own half of the shape gets a fitting other half: blocks of more
+// than 512 threads 2048 doubles per wave where that leaves four waves per
+// SIMD (2^28: 1024 threads of 2048 343 us, of 1024 361; 512
+// threads of either 344), and waves of 4096 to 8192 doubles 512-thread blocks
+// that start in step, 256-thread ones at four or fewer waves per CU (2^28,
+// waves of 4096: 352 us, in one-wave blocks 378; 2^24: 24.8 and 26.6; waves of
+// 2048 345 and 350, 26.2 and 25.6; waves of 16384 413 and 404).
 void default_shape(const DeviceContext& ctx, uint64_t n, int format, int per_lane, int* block, uint64_t* tile) {
   const uint64_t quantum = 64ull * per_lane;
   const uint64_t cu = (uint64_t)ctx.num_cu;
-  uint64_t t = 1024;
-  if (format == MRG8_U32) {
-    t = 8192;
-    while (t > 4 * quantum && (n + t - 1) / t < cu * 16) t /= 2;  // four waves per SIMD
-  } else if ((n + t - 1) / t <= cu * 4) {
-    t = 512;
-  } else if (n / t + 2 > kMaxGridWaves) {
-    t = 2048;
+  auto waves = [&](uint64_t t) { return (n + t - 1) / t; };
+  if (*tile == 0) {
+    uint64_t t = 1024;
+    if (format == MRG8_U32) {
+      t = 8192;
+      while (t > 4 * quantum && waves(t) < cu * 16) t /= 2;  // four waves per SIMD
+    } else if (waves(t) <= cu * 4) {
+      t = 512;
+    } else if ((*block > 512 && waves(2 * t) >= cu * 16) || n / t + 2 > kMaxGridWaves) {
+      t = 2048;
+    }
+    *tile = std::max<uint64_t>(quantum, t / quantum * quantum);
+    if (*block == 0) *block = format == MRG8_U32 ? 256 : 64;
+  } else if (*block == 0) {
+    *block = format == MRG8_U32 ? 256 : *tile <= 2048 || *tile > 8192 ? 64 : waves(*tile) <= cu * 4 ? 256 : 512;
   }
-  *tile = std::max<uint64_t>(quantum, t / quantum * quantum);
-  *block = format == MRG8_U32 ? 256 : 64;
 }
 
 // Tiles per wave of a matrix-core fill by default.  Doubles: 32 KiB of output
@@ -292,10 +304,10 @@ uint64_t mfma_tiles_per_wave(const DeviceContext& ctx, int format, uint64_t tile
   const uint64_t cu = (uint64_t)ctx.num_cu, esz = (uint64_t)format_size(format);
   const uint64_t most = std::max<uint64_t>(1, 32768 / esz / tile);
   if (format != MRG8_U32) return std::min(most, tiles / (8 * cu));
-  if (tiles <= 12 * cu) return 1;
-  if (tiles <= 24 * cu) return 2;
-  const uint64_t half = std::max<uint64_t>(1, 16384 / esz / tile);
-  return tiles >= 64 * cu && tiles / half + 8 <= kMaxGridWaves ? half : most;
+  const uint64_t one = 2048 / tile;  // tiles in 2048 words
+  if (tiles <= 12 * one * cu) return one;
+  if (tiles <= 24 * one * cu) return 2 * one;
+  return tiles >= 64 * one * cu && tiles / (2 * one) + 8 <= kMaxGridWaves ? 2 * one : most;
 }
 
 // Blocks per XCD run of a vector-kernel fill (1: blocks in dispatch order).
@@ -422,14 +434,11 @@ int fill_shaped(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, vo
   // each wave writes the outputs before its first 1 KiB boundary one per lane.
   if (pl && pl != 1 && pl != 2 && pl != 4) return fail(MRG8_ERR_ARG, "outputs_per_lane must be 1, 2, 4, 16 or 32");
   if (!pl) pl = 4;
-  int def_block = 0;
-  uint64_t def_tile = 0;
-  default_shape(ctx, n, format, pl, &def_block, &def_tile);
-  if (block_threads <= 0) block_threads = def_block;
+  block_threads = std::max(block_threads, 0);
+  default_shape(ctx, n, format, pl, &block_threads, &tile);
   if (block_threads < 64 || block_threads > 1024 || block_threads % 64)
     return fail(MRG8_ERR_ARG, "block_threads %d must be a multiple of 64 in [64, 1024]", block_threads);
   const uint64_t quantum = 64ull * pl;
-  if (tile == 0) tile = def_tile;
   if (tile > n) tile = n;  // one wave takes everything (and the rounding below cannot wrap)
   if (tile % quantum) tile = (tile + quantum - 1) / quantum * quantum;
   // Wave 0 also takes the outputs before the first 1 KiB boundary, so every

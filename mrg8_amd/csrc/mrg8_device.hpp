@@ -171,10 +171,14 @@ __host__ __device__ inline uint64_t segment_head(const void* out, int32_t format
   return h < count ? h : count;
 }
 
-__host__ __device__ inline uint64_t segment_tiles(const void* out, int32_t format, uint64_t count, uint64_t tile) {
+// Tiles of a segment of `count` outputs with head h.
+__host__ __device__ inline uint64_t head_tiles(uint64_t h, uint64_t count, uint64_t tile) {
   if (count == 0) return 0;
-  const uint64_t h = segment_head(out, format, count, tile);
   return count == h ? 1 : (count - h + tile - 1) / tile;
+}
+
+__host__ __device__ inline uint64_t segment_tiles(const void* out, int32_t format, uint64_t count, uint64_t tile) {
+  return head_tiles(segment_head(out, format, count, tile), count, tile);
 }
 
 // Outputs [*first, *end) of tile k of a segment of `count` outputs with head h.

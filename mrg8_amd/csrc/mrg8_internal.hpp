@@ -84,7 +84,8 @@ std::vector<TunedShape> fill_candidates(int format);
 constexpr uint64_t kMaxGridWaves = 0xffffffffull / 64;
 
 // Automatic shapes: threads per block and outputs per wave of the vector
-// kernel, and tiles (of `tile` outputs) per wave of the matrix-core fill.
+// kernel (where they are 0), and tiles (of `tile` outputs) per wave of the
+// matrix-core fill.
 void default_shape(const DeviceContext& ctx, uint64_t n, int format, int per_lane, int* block, uint64_t* tile);
 uint64_t mfma_tiles_per_wave(const DeviceContext& ctx, int format, uint64_t tile, uint64_t tiles);
 // Blocks per XCD run of a vector-kernel fill (1: blocks in dispatch order).

@@ -86,15 +86,15 @@ size_t layout_batch_block(uint8_t* mem, uint32_t count, uint64_t tile, uint64_t 
   };
   for (uint32_t i = 0; i < count; ++i) {
     tiles[i] = t;
-    const uint64_t c = segs[i].count, n = segment_tiles(segs[i].out, segs[i].format, c, tile);
+    const uint64_t c = segs[i].count, head = segment_head(segs[i].out, segs[i].format, c, tile);
+    const uint64_t n = head_tiles(head, c, tile);
     w.weight += c * (segs[i].format == 2 ? 1 : kShortDouble);
     if (n == 1) {
       add(c, 1);
     } else if (n) {  // the first tile with the head, whole ones, the last
-      const uint64_t first = segment_head(segs[i].out, segs[i].format, c, tile) + tile;
-      add(first, 1);
+      add(head + tile, 1);
       if (n > 2) add(tile, n - 2);
-      add(c - first - (n - 2) * tile, 1);
+      add(c - head - (n - 1) * tile, 1);
     }
     const uint64_t end = std::min<uint64_t>(t + n, max_tiles);
     if (t < end) std::fill(tile_seg + t, tile_seg + end, i);

@@ -172,6 +172,30 @@ static void run(const DeviceContext& ctx) {
   }
   CHECK(mfma_tiles_per_wave(ctx, MRG8_U32, 2048, 12 * 256) == 1 && mfma_tiles_per_wave(ctx, MRG8_U32, 2048, 12 * 256 + 1) == 2);
   CHECK(mfma_tiles_per_wave(ctx, MRG8_U32, 2048, 24 * 256 + 1) == 4 && mfma_tiles_per_wave(ctx, MRG8_U32, 2048, 64 * 256) == 2);
-  CHECK(mfma_tiles_per_wave(ctx, MRG8_U32, 1024, 64 * 256) == 4 && mfma_tiles_per_wave(ctx, MRG8_F64, 1024, 1 << 18) == 4);
+  CHECK(mfma_tiles_per_wave(ctx, MRG8_U32, 1024, 64 * 256) == 8 && mfma_tiles_per_wave(ctx, MRG8_U32, 1024, 128 * 256) == 4);
+  CHECK(mfma_tiles_per_wave(ctx, MRG8_U32, 1024, 24 * 256) == 2 && mfma_tiles_per_wave(ctx, MRG8_F64, 1024, 1 << 18) == 4);
+}
+""")
+
+
+def test_half_given_fill_shapes(tmp_path):
+    """A caller's threads per block get fitting outputs per wave, and outputs per wave fitting blocks."""
+    check(tmp_path, r"""
+static bool is(const DeviceContext& ctx, uint64_t n, int format, int per_lane, int block, uint64_t tile, int want_block,
+               uint64_t want_tile) {
+  default_shape(ctx, n, format, per_lane, &block, &tile);
+  return block == want_block && tile == want_tile;
+}
+static void run(const DeviceContext& ctx) {
+  const uint64_t large = 1 << 28, small = 1 << 20;
+  CHECK(is(ctx, large, MRG8_F64, 4, 0, 0, 64, 1024) && is(ctx, small, MRG8_F64, 4, 0, 0, 64, 512));
+  CHECK(is(ctx, large, MRG8_F64, 4, 256, 0, 256, 1024) && is(ctx, large, MRG8_F64_01, 4, 512, 0, 512, 1024));
+  CHECK(is(ctx, large, MRG8_F64, 4, 1024, 0, 1024, 2048) && is(ctx, small, MRG8_F64, 4, 1024, 0, 1024, 512));
+  CHECK(is(ctx, 1 << 22, MRG8_F64, 1, 1024, 0, 1024, 1024) && is(ctx, 1 << 23, MRG8_F64, 1, 1024, 0, 1024, 2048));
+  CHECK(is(ctx, large, MRG8_F64, 4, 0, 2048, 64, 2048) && is(ctx, large, MRG8_F64, 4, 0, 16384, 64, 16384));
+  CHECK(is(ctx, large, MRG8_F64, 4, 0, 8192, 512, 8192) && is(ctx, large, MRG8_F64, 4, 0, 4096, 512, 4096));
+  CHECK(is(ctx, small, MRG8_F64, 4, 0, 4096, 256, 4096) && is(ctx, large, MRG8_F64, 4, 100, 7, 100, 7));
+  CHECK(is(ctx, large, MRG8_U32, 4, 0, 0, 256, 8192) && is(ctx, small, MRG8_U32, 4, 512, 0, 512, 1024));
+  CHECK(is(ctx, large, MRG8_U32, 4, 0, 2048, 256, 2048));
 }
 """)
