@@ -320,9 +320,9 @@ uint64_t mfma_tiles_per_wave(const DeviceContext& ctx, int format, uint64_t tile
 // Larger blocks and longer waves have longer runs, which pay from 64 waves per
 // CU on (at 16, in runs | in dispatch order: 64 threads of 65536 outputs per
 // wave, 2^28 473 | 413 us; 256 of 2048, 2^23 16.1 | 14.3; 256 of 1024, 2^22
-// 10.0 | 8.9).  Word fills were slower in runs and are left in dispatch order.
+// 10.0 | 8.9; but 64 of 2048, 2^24, 32 waves per CU, 25.0 | 26.2).  Word fills were slower in runs and are left in dispatch order.
 uint32_t fill_xcd_group(const DeviceContext& ctx, int format, uint64_t waves, int block_threads, uint64_t tile) {
-  const uint64_t per_cu = block_threads == 64 && tile <= 1024 ? 16 : 64;
+  const uint64_t per_cu = block_threads == 64 && tile <= 2048 ? 16 : 64;
   if (format == MRG8_U32 || ctx.num_xcc <= 1 || waves < (uint64_t)ctx.num_cu * per_cu) return 1;
   return std::min(64u, xcd_run_blocks(ctx, block_threads));
 }
@@ -465,11 +465,10 @@ int fill_shaped(DeviceContext& ctx, const uint32_t state[8], uint64_t offset, vo
   a.digits = ctx.tables.digits;
   a.xcds = (uint32_t)ctx.num_xcc;
   a.xcd_group = fill_xcd_group(ctx, format, fill_waves(n, head, tile), block_threads, tile);
-  a.in_step = fill_in_step(a.xcd_group, block_threads, tile);
   int prev = 0;
   (void)hipGetDevice(&prev);
   if (prev != ctx.device) (void)hipSetDevice(ctx.device);
-  hipError_t e = launch_fill(a, format, pl, block_threads, stream);
+  hipError_t e = launch_fill(a, format, pl, block_threads, fill_in_step(a.xcd_group, block_threads, tile), stream);
   if (prev != ctx.device) (void)hipSetDevice(prev);
   if (e != hipSuccess) return hip_fail(e, "fill launch");
   return MRG8_OK;

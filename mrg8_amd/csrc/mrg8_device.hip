@@ -508,16 +508,21 @@ __device__ __forceinline__ uint64_t xcd_block(uint32_t b, uint32_t nb, uint32_t 
 // between its loads and its products, 2^24 doubles took 25.1 and 24.9 us
 // against 24.1 us (2^28: 314 and 316 against 320 us).  Limited to 80
 // registers for a sixth wave per SIMD it spills (2^28: 401 us).
-template <int FMT, int PL>
+// IN_STEP: the waves of a block wait for one another before their outputs (see
+// fill_in_step).
+template <int FMT, int PL, bool IN_STEP>
 __global__ __launch_bounds__(1024) void k_fill(FillArgs a) {
   const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform wave index
   const uint32_t nw = blockDim.x >> 6;
   const uint64_t w = xcd_block(blockIdx.x, gridDim.x, a.xcds, a.xcd_group) * nw + wib;
   const uint64_t first = fill_first(a, w);
-  const uint32_t word = jump_uniform(own_word(a.start.state), a.start.offset + first, a.digits);
-  if (a.in_step) __syncthreads();  // every wave of the block, with outputs or not
-  if (first >= a.n) return;
+  if (!IN_STEP && first >= a.n) return;
   const uint64_t cnt = min(a.head + (w + 1) * a.tile, a.n) - first;
+  const uint32_t word = jump_uniform(own_word(a.start.state), a.start.offset + first, a.digits);
+  if constexpr (IN_STEP) {
+    __syncthreads();  // every wave of the block, with outputs or not
+    if (first >= a.n) return;
+  }
   uint32_t s[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) s[j] = __builtin_amdgcn_readlane(word, j);
@@ -1432,29 +1437,35 @@ __global__ __launch_bounds__(64) void k_batch_short(BatchArgs a) {
 }
 
 template <int FMT, int PL>
-hipError_t fill_one(const FillArgs& a, int block_threads, hipStream_t stream) {
+hipError_t fill_one(const FillArgs& a, int block_threads, bool in_step, hipStream_t stream) {
   if (a.n == 0) return hipSuccess;
   const uint64_t waves = fill_waves(a.n, a.head, a.tile);
   const uint64_t wpb = (uint64_t)block_threads / 64;
   const uint64_t blocks = (waves + wpb - 1) / wpb;
   if (blocks * (uint64_t)block_threads > 0xffffffffull) return hipErrorInvalidConfiguration;  // 32-bit grid
-  hipLaunchKernelGGL((k_fill<FMT, PL>), dim3((uint32_t)blocks), dim3(block_threads), 0, stream, a);
+  if constexpr (FMT != 2) {
+    if (in_step) {
+      hipLaunchKernelGGL((k_fill<FMT, PL, true>), dim3((uint32_t)blocks), dim3(block_threads), 0, stream, a);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((k_fill<FMT, PL, false>), dim3((uint32_t)blocks), dim3(block_threads), 0, stream, a);
   return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_fill(const FillArgs& a, int format, int per_lane, int block_threads, hipStream_t stream) {
+hipError_t launch_fill(const FillArgs& a, int format, int per_lane, int block_threads, bool in_step, hipStream_t stream) {
   switch (format * 8 + per_lane) {
-    case 0 * 8 + 1: return fill_one<0, 1>(a, block_threads, stream);
-    case 0 * 8 + 2: return fill_one<0, 2>(a, block_threads, stream);
-    case 0 * 8 + 4: return fill_one<0, 4>(a, block_threads, stream);
-    case 1 * 8 + 1: return fill_one<1, 1>(a, block_threads, stream);
-    case 1 * 8 + 2: return fill_one<1, 2>(a, block_threads, stream);
-    case 1 * 8 + 4: return fill_one<1, 4>(a, block_threads, stream);
-    case 2 * 8 + 1: return fill_one<2, 1>(a, block_threads, stream);
-    case 2 * 8 + 2: return fill_one<2, 2>(a, block_threads, stream);
-    case 2 * 8 + 4: return fill_one<2, 4>(a, block_threads, stream);
+    case 0 * 8 + 1: return fill_one<0, 1>(a, block_threads, in_step, stream);
+    case 0 * 8 + 2: return fill_one<0, 2>(a, block_threads, in_step, stream);
+    case 0 * 8 + 4: return fill_one<0, 4>(a, block_threads, in_step, stream);
+    case 1 * 8 + 1: return fill_one<1, 1>(a, block_threads, in_step, stream);
+    case 1 * 8 + 2: return fill_one<1, 2>(a, block_threads, in_step, stream);
+    case 1 * 8 + 4: return fill_one<1, 4>(a, block_threads, in_step, stream);
+    case 2 * 8 + 1: return fill_one<2, 1>(a, block_threads, in_step, stream);
+    case 2 * 8 + 2: return fill_one<2, 2>(a, block_threads, in_step, stream);
+    case 2 * 8 + 4: return fill_one<2, 4>(a, block_threads, in_step, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -95,7 +95,6 @@ struct FillArgs {
   const int32_t* digits;    // jump matrices (DeviceTables::digits)
   uint32_t xcds;            // XCDs that blocks are dealt to in turn (block b runs on XCD b mod xcds)
   uint32_t xcd_group;       // consecutive blocks of output per XCD run (1: blocks in dispatch order)
-  uint32_t in_step;         // a block's waves start their outputs together
 };
 
 // A matrix-core fill: `tiles` whole tiles of 16 x `column` outputs at
@@ -245,7 +244,8 @@ struct AdvanceArgs {
 };
 
 // Launchers (mrg8_device.hip).  All are asynchronous on `stream`.
-hipError_t launch_fill(const FillArgs& a, int format, int per_lane, int block_threads, hipStream_t stream);
+// in_step: the waves of a block start their outputs together (doubles).
+hipError_t launch_fill(const FillArgs& a, int format, int per_lane, int block_threads, bool in_step, hipStream_t stream);
 // Blocks of a.waves_per_block waves.
 hipError_t launch_fill_mfma(const MfmaFillArgs& a, int format, hipStream_t stream);
 hipError_t launch_batch(const BatchArgs& a, int grid, int block_threads, hipStream_t stream);

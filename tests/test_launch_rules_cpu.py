@@ -93,12 +93,13 @@ static void run(const DeviceContext& ctx) {
 
 
 def test_xcd_runs_of_fills(tmp_path):
-    """Only one-wave blocks of up to 1024 doubles run on the XCDs in runs below
+    """Only one-wave blocks of up to 2048 doubles run on the XCDs in runs below
     64 waves per CU; blocks of several waves in such runs start in step."""
     check(tmp_path, r"""
 static void run(const DeviceContext& ctx) {
   CHECK(fill_xcd_group(ctx, MRG8_F64, 4096, 64, 1024) == 64);
   CHECK(fill_xcd_group(ctx, MRG8_F64, 4095, 64, 1024) == 1);
+  CHECK(fill_xcd_group(ctx, MRG8_F64, 4096, 64, 2048) == 64 && fill_xcd_group(ctx, MRG8_F64, 16383, 64, 4096) == 1);
   CHECK(fill_xcd_group(ctx, MRG8_F64_01, 4096, 64, 65536) == 1);
   CHECK(fill_xcd_group(ctx, MRG8_F64, 4096, 256, 1024) == 1);
   CHECK(fill_xcd_group(ctx, MRG8_F64, 16383, 512, 2048) == 1);
