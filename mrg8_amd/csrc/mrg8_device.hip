@@ -779,9 +779,9 @@ __device__ __forceinline__ uint32_t advance_zero_words(uint32_t s, const uint32_
 
 // Eight lanes per state, lane r holding word r and computing row r of each
 // product; the byte positions of the offset in order, the rows of four
-// positions fetched while the four before them are computed (20011 states,
-// 64-bit offsets: 3.8 us a launch, one position ahead 4.3 us; 1000 states,
-// 256 bits: 5.5 and 8.1 us).  Positions where
+// positions fetched while the four before them are computed (launched back to
+// back, 20011 states, 64-bit offsets: 3.8 us, one position ahead 4.3 us; 1000
+// states, 256 bits: 5.5 and 8.1 us; alone in a trace 4.4 and 5.8 us).  Positions where
 // no state of the wave has a digit are skipped.  A state is read before it is
 // written, so `in` and `out` may be the same buffer.
 __global__ __launch_bounds__(256) void k_advance(AdvanceArgs a) {
